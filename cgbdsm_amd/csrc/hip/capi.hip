@@ -271,6 +271,30 @@ void ValidatePlanTables(const cgbdsm_plan* p, bool order) {
     }
 }
 
+PlanLds MakePlanLds(const DevPlan& h) {
+    const cgbdsm_plan& p = h.p;
+    PlanLds L{};
+    for (uint32_t d = 0; d < p.qv; d++) {
+        const uint32_t nbn = p.go_bni_offs[d + 1] - p.go_bni_offs[d];
+        for (uint32_t k = 0; k < nbn && k < (uint32_t)kMaxQV; k++) {
+            const uint32_t bq = p.go_bni[p.go_bni_offs[d] + k];
+            L.pair[d][k] = (uint16_t)(p.eidx[p.go_vs[bq] * kMaxQV + p.go_vs[d]] | (bq << 8));
+        }
+        L.dep_mask[d] = h.dep_mask[d];
+        L.vs |= (uint64_t)p.go_vs[d] << (4 * d);
+        L.cls |= (uint64_t)p.go_lcls[d] << (4 * d);
+        L.nbn |= (uint64_t)nbn << (4 * d);
+    }
+    for (uint32_t e = 0; e < p.qe; e++) {
+        for (uint32_t dir = 0; dir < p.ndir; dir++)
+            if (p.dir_to_edge[dir] < e) L.app[e][dir >> 6] |= 1ull << (dir & 63);
+        for (uint32_t v = 0; v < p.qv; v++)
+            if (h.all_ones[e][v]) L.ones[e] |= 1u << v;
+        L.own[e] = (uint32_t)h.sa[e] | ((uint32_t)h.sb[e] << 8);
+    }
+    return L;
+}
+
 void UploadPlan(cgbdsm_query* q) {
     CGD_HIP(hipMemcpyAsync(q->d_plan, &q->hplan, sizeof(DevPlan), hipMemcpyHostToDevice, q->s));
     CGD_HIP(hipStreamSynchronize(q->s));
@@ -335,7 +359,10 @@ StealQueue MakeSteal(cgbdsm_query* q, bool donate) {
     Q.donate_min = donate ? q->donate_min : 0;
     Q.range_min = q->dfs_range_min;
     Q.abort = q->d_abort;
-    Q.poll_ticks = std::max<long long>(1, q->ctx->wall_khz / 20);  // 50 us
+    // 200 us: a working wave's look at the queue words costs it a few
+    // microseconds and the words' lines a place in the queue of atomics
+    // (dense 6-vertex query on scale 20: 61 ms at 50 us, 49 ms at 200 us).
+    Q.poll_ticks = std::max<long long>(1, q->ctx->wall_khz / 5);
     Q.host_ticks = (long long)q->ctx->wall_khz * 2;              // 2 ms
     return Q;
 }
@@ -371,12 +398,16 @@ void RunDfsJobs(cgbdsm_query* q, uint32_t* tuples, uint64_t tup_cap) {
     const int k = tuples ? -1 : KBegin(q, CGBDSM_K_DFS);
     uint32_t levels = 1;  // survivor stacks: qv - 1 levels cover every job
     for (const DfsJob& j : q->h_jobs) levels = std::max<uint32_t>(levels, j.T.qv - 1);
-    {
-        const uint32_t full = DfsLdsShape(levels, tuples != nullptr).stab_cap;
-        q->st.last_dfs_lds_cache = q->dfs_cache_cap && q->dfs_cache_cap < full ? q->dfs_cache_cap & ~63u : full;
-    }
-    LaunchDfs(q->d_jobs.p, (uint32_t)q->h_jobs.size(), q->d_rowbase.p, n, q->d_cnt, MakeSteal(q, tuples == nullptr),
-              tuples, tup_cap, q->ctx->num_cus, q->dfs_bpc, q->dfs_grab, levels, q->dfs_cache_cap, q->s);
+    bool batched = !tuples;
+    for (const DfsJob& j : q->h_jobs) batched &= (j.opts & kJobBatched) != 0;
+    const DfsShape sh = DfsLdsShape(levels, tuples != nullptr, batched);
+    q->st.last_dfs_lds_cache =
+        q->dfs_cache_cap && q->dfs_cache_cap < sh.stab_cap ? q->dfs_cache_cap & ~63u : sh.stab_cap;
+    const uint32_t grid = DfsGrid(sh, n, q->ctx->num_cus, q->dfs_bpc);
+    Ensure(q, q->dfs_out, grid);
+    LaunchDfs(q->d_jobs.p, (uint32_t)q->h_jobs.size(), q->d_rowbase.p, n, q->d_cnt, q->dfs_out.p,
+              MakeSteal(q, tuples == nullptr), tuples, tup_cap, sh, grid, q->dfs_grab, levels,
+              q->st.last_dfs_lds_cache, batched, q->s);
     KEnd(q, k);
     CGD_HIP(hipGetLastError());
     if (q->deadline_ms > 0) {
@@ -412,9 +443,13 @@ void RunDfsJobs(cgbdsm_query* q, uint32_t* tuples, uint64_t tup_cap) {
     }
 }
 
+// q's share of a final-DFS launch; its frontier has been built, so h_cnt
+// holds the duplicates of the batch's update lists.
 DfsJob MakeJob(cgbdsm_query* q, const uint32_t* rows, uint32_t depth) {
+    const bool batched = q->hplan.sfx_batch && q->hplan.cp_start < q->qv && depth < q->hplan.cp_start &&
+                         q->dfs_shortest && q->dfs_suffix && q->dfs_wsearch && q->h_cnt->u_dups == 0;
     return DfsJob{MakeTables(q), rows, q->d_cnt, depth,
-                  (q->dfs_shortest ? kJobShortest : 0u) | (q->dfs_suffix ? kJobSuffix : 0u) |
+                  (batched ? kJobBatched : 0u) | (q->dfs_shortest ? kJobShortest : 0u) | (q->dfs_suffix ? kJobSuffix : 0u) |
                       (q->dfs_wsearch ? kJobWaveSearch | (q->dfs_wsearch << kJobWaveShift) : 0u)};
 }
 
@@ -773,6 +808,7 @@ cgbdsm_status cgbdsm_query_destroy(cgbdsm_query* q) {
             Release(q, *b);
         Release(q, q->pma.meta);
         Release(q, q->d_jobs);
+        Release(q, q->dfs_out);
         Release(q, q->d_rowbase);
         Release(q, q->tag_hist);
         for (auto& r : q->fifo) {
@@ -885,6 +921,7 @@ cgbdsm_status cgbdsm_query_set_plan(cgbdsm_query* q, const cgbdsm_plan* plan) {
                     if (plan->go_bni[k] == x) m |= 1u << j;
             q->hplan.dep_mask[x] = m;
         }
+        q->hplan.lds = MakePlanLds(q->hplan);
         UploadPlan(q);
         q->have_order = true;
     });

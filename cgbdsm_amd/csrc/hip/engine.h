@@ -94,9 +94,23 @@ struct StealQueue {
     uint32_t donate_min;      // remaining survivors needed before donating (0: never)
     uint32_t range_min;       // candidates a donated range must at least hold
     const uint32_t* abort;    // host-mapped coherent flag, non-zero asks kernels to stop
-    long long poll_ticks;     // wall-clock ticks between a wave's reads of shared queue words
-    long long host_ticks;     // wall-clock ticks between a wave's reads of the host flag
+    long long poll_ticks;     // wall-clock ticks between a block's reads of shared queue words
+    long long host_ticks;     // wall-clock ticks between a block's reads of the host flag
 };
+
+// Plan facts the matching kernels read in their inner loops, kept in LDS and
+// uniform registers there: the plan's byte tables cannot be read with scalar
+// loads, and a vector load of a plan byte ahead of every list access would put
+// one more dependent trip to L2 on every step.
+struct PlanLds {
+    uint16_t pair[kMaxQV][kMaxQV];  // backward neighbour k of position d: dir | position << 8
+    uint64_t app[kMaxQE][2];        // edge tag ei: dirs (bits 0..127) whose undirected edge index < ei
+    uint32_t ones[kMaxQE];          // edge tag ei: query vertices whose support tile is all ones
+    uint32_t own[kMaxQE];           // edge tag ei: its two dirs, sa | sb << 8
+    uint32_t dep_mask[kMaxQV];      // positions whose candidate set has position x as backward neighbour
+    uint64_t vs, cls, nbn;          // per position, 4 bits each: query vertex, label class, backward neighbours
+};
+static_assert(sizeof(PlanLds) % 8 == 0, "copied as 64-bit words");
 
 // Per-query parameter block in device memory (read through scalar loads).
 // Replaces the __constant__ tables of graph/graph_gpu.cu:35-46 and
@@ -116,6 +130,7 @@ struct DevPlan {
                                        // siblings at the position before it at once
     uint8_t maxbn[kMaxQV];             // largest backward-neighbour position of each position
     uint32_t dep_mask[kMaxQV];         // positions whose candidate set depends on position x
+    PlanLds lds;                       // what the matching kernels copy to LDS
 };
 
 // Device pointers of one query's index, passed by value to kernels.

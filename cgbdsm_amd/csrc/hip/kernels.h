@@ -67,6 +67,7 @@ void LaunchExtend(const Tables& T, const uint32_t* in, uint64_t n_in, uint32_t d
 enum : uint32_t {
     kJobShortest = 1u,  // scan the shortest backward-neighbour list when lists are sets
     kJobSuffix = 2u,    // count the product suffix of the order in closed form
+    kJobBatched = 16u,    // batched product suffix, default options, update lists without duplicates
     kJobWaveSearch = 4u,  // search long backward-neighbour lists with the whole wavefront
     kJobWaveShift = 8u,   // bits 8..12: log2 of the shortest list searched so (0: 256)
 };
@@ -77,22 +78,31 @@ struct DfsJob {
     uint32_t D;
     uint32_t opts;  // kJob* bits
 };
-// Final DFS over the rows of njobs queries (row_base[j] = first global row of
-// job j, row_base[njobs] = all rows); `cnt` holds the shared work queue.
-// surv_levels >= qv - 1 of every job (survivor stacks in LDS); blocks_per_cu
-// 0 = as many as fit.
-// cache_cap: u32 per wave of the stable-intersection cache (0: all the LDS
-// left; smaller values leave part of it unused).
-void LaunchDfs(const DfsJob* jobs, uint32_t njobs, const unsigned long long* row_base, uint64_t n_rows, Counters* cnt,
-               const StealQueue& Q, uint32_t* tuples, uint64_t tup_cap, uint32_t num_cus, uint32_t blocks_per_cu,
-               uint32_t grab, uint32_t surv_levels, uint32_t cache_cap, hipStream_t s);
-// LDS plan of a final-DFS launch (see DfsLdsShapeT in match.hip).
+// What one block of a final-DFS launch counted: its statistics (scanned,
+// probes, steps, step lanes, batched steps, donated, wave and idle ticks) and,
+// per query its waves ended with (job[w], ~0: none), the counts per edge.
+constexpr int kDfsWaves = 4, kDfsStats = 8;
+struct DfsOut {
+    unsigned long long stat[kDfsStats];
+    uint32_t job[kDfsWaves];
+    unsigned long long pe[kDfsWaves][kMaxQE];
+};
+// LDS plan of a final-DFS launch (see DfsLdsShapeT in match.hip): survivor
+// stacks of surv_levels levels, a stable-intersection cache of stab_cap u32 per
+// wave.  batched: every job has kJobBatched.
 struct DfsShape {
     uint32_t blocks_per_cu, dyn_bytes, stab_cap;
 };
-DfsShape DfsLdsShape(uint32_t surv_levels, bool tuples);
-// Resident KDfs blocks per CU at full occupancy.
-uint32_t DfsBlocksPerCU();
+DfsShape DfsLdsShape(uint32_t surv_levels, bool tuples, bool batched);
+// Blocks of a launch over n_rows rows (blocks_per_cu 0: as many as fit).
+uint32_t DfsGrid(const DfsShape& sh, uint64_t n_rows, uint32_t num_cus, uint32_t blocks_per_cu);
+// Final DFS over the rows of njobs queries (row_base[j] = first global row of
+// job j, row_base[njobs] = all rows); `cnt` holds the shared work queue, outs
+// one record per block.  surv_levels >= qv - 1 of every job (survivor stacks in
+// LDS); stab_cap <= sh.stab_cap.
+void LaunchDfs(const DfsJob* jobs, uint32_t njobs, const unsigned long long* row_base, uint64_t n_rows, Counters* cnt,
+               DfsOut* outs, const StealQueue& Q, uint32_t* tuples, uint64_t tup_cap, const DfsShape& sh, uint32_t grid,
+               uint32_t grab, uint32_t surv_levels, uint32_t stab_cap, bool batched, hipStream_t s);
 
 void LaunchCountDups(const uint64_t* k, uint64_t n, Counters* cnt, hipStream_t s);
 

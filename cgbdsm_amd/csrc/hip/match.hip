@@ -31,16 +31,14 @@
 #include "kernels.h"
 #include "wave.h"
 
-// Register budget of the final DFS (occupancy against spills), a build-time
-// tuning knob: -DCGD_DFS_WAVES_PER_EU=N asks for N resident waves per SIMD
-// (3: 168 VGPRs with some spills, measured best; 2 and 4 are slower; 0: no cap).
-#ifndef CGD_DFS_WAVES_PER_EU
-#define CGD_DFS_WAVES_PER_EU 3
-#endif
-#if CGD_DFS_WAVES_PER_EU > 0
-#define CGD_DFS_ATTR __attribute__((amdgpu_waves_per_eu(CGD_DFS_WAVES_PER_EU)))
-#else
-#define CGD_DFS_ATTR
+// Resident blocks per CU (= waves per SIMD) of the final DFS, a build-time
+// tuning knob.  Its loops' carried values are scalar (75 to 92 VGPRs, nothing
+// spilled to memory), so registers would allow 6; what decides is the LDS left
+// for the stable-intersection cache and the waves that share the work queue's
+// lines.  Scale-21 four-query batch: 154 ms of DFS at 3, 135 at 4, 131 at 5;
+// scale-20 dense 6-vertex query: 48, 49, 74.
+#ifndef CGD_DFS_BLOCKS
+#define CGD_DFS_BLOCKS 4
 #endif
 
 namespace cgd {
@@ -49,6 +47,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWpb = kThreads / kWave;
+static_assert(kWpb == kDfsWaves, "DfsOut holds one slot per wave of a block");
 
 struct List {
     const uint32_t* base;
@@ -56,109 +55,18 @@ struct List {
     uint32_t bl, al;
 };
 
-// Plan facts the matching kernels read in their inner loops, kept where a
-// read costs no vector-memory round trip: per-block LDS tables (filled once
-// at kernel start) and uniform registers.  The plan's byte tables cannot be
-// read with scalar loads, and a vector load of a plan byte ahead of every
-// list access would put one more dependent trip to L2 on every step.
-struct PlanLds {
-    uint16_t pair[kMaxQV][kMaxQV];  // backward neighbour k of position d: dir | position << 8
-    uint64_t app[kMaxQE][2];        // edge tag ei: dirs (bits 0..127) whose undirected edge index < ei
-    uint32_t ones[kMaxQE];          // edge tag ei: query vertices whose support tile is all ones
-    uint32_t own[kMaxQE];           // edge tag ei: its two dirs, sa | sb << 8
-    uint32_t dep_mask[kMaxQV];      // positions whose candidate set has position x as backward neighbour
-    uint64_t vs, cls, nbn;          // per position, 4 bits each: query vertex, label class, backward neighbours
-};
-
+// The plan's tables (PlanLds) into LDS, by a block or by one wavefront into
+// its own copy (the final DFS switches between queries per wavefront).  The
+// host lays them out when the plan is set: a wave that derived them here from
+// the plan's byte tables spent tens of dependent loads before its first row.
 __device__ void FillPlanLds(const Tables& T, PlanLds* L) {
-    const cgbdsm_plan& p = T.P->p;
-    const uint32_t t = threadIdx.x;
-    for (uint32_t i = t; i < (uint32_t)(kMaxQV * kMaxQV); i += blockDim.x) {
-        const uint32_t d = i / kMaxQV, k = i % kMaxQV;
-        uint16_t v = 0;
-        if (d < p.qv && k < (uint32_t)(p.go_bni_offs[d + 1] - p.go_bni_offs[d])) {
-            const uint32_t bq = p.go_bni[p.go_bni_offs[d] + k];
-            v = (uint16_t)(p.eidx[p.go_vs[bq] * kMaxQV + p.go_vs[d]] | (bq << 8));
-        }
-        L->pair[d][k] = v;
-    }
-    for (uint32_t e = t; e < (uint32_t)kMaxQE; e += blockDim.x) {
-        uint64_t a0 = 0, a1 = 0;
-        uint32_t ones = 0, own = 0;
-        if (e < p.qe) {
-            for (uint32_t dir = 0; dir < p.ndir; dir++)
-                if (p.dir_to_edge[dir] < e) {
-                    if (dir < 64) a0 |= 1ull << dir;
-                    else a1 |= 1ull << (dir - 64);
-                }
-            for (uint32_t q = 0; q < p.qv; q++)
-                if (T.P->all_ones[e][q]) ones |= 1u << q;
-            own = (uint32_t)T.P->sa[e] | ((uint32_t)T.P->sb[e] << 8);
-        }
-        L->app[e][0] = a0;
-        L->app[e][1] = a1;
-        L->ones[e] = ones;
-        L->own[e] = own;
-    }
-    for (uint32_t x = t; x < (uint32_t)kMaxQV; x += blockDim.x) L->dep_mask[x] = T.P->dep_mask[x];
-    if (t == 0) {
-        uint64_t vs = 0, cls = 0, nbn = 0;
-        for (uint32_t d = 0; d < p.qv; d++) {
-            vs |= (uint64_t)p.go_vs[d] << (4 * d);
-            cls |= (uint64_t)p.go_lcls[d] << (4 * d);
-            nbn |= (uint64_t)(p.go_bni_offs[d + 1] - p.go_bni_offs[d]) << (4 * d);
-        }
-        L->vs = vs;
-        L->cls = cls;
-        L->nbn = nbn;
-    }
+    const uint64_t* src = (const uint64_t*)&T.P->lds;
+    for (uint32_t i = threadIdx.x; i < sizeof(PlanLds) / 8; i += blockDim.x) ((uint64_t*)L)[i] = LdG(src + i);
     __syncthreads();
 }
-
-// The same tables filled by one wavefront into its own copy (the final DFS
-// switches between queries per wavefront).
-__device__ void FillPlanLdsWave(const Tables& T, PlanLds* L) {
-    const cgbdsm_plan& p = T.P->p;
-    const uint32_t t = LaneId();
-    for (uint32_t i = t; i < (uint32_t)(kMaxQV * kMaxQV); i += kWave) {
-        const uint32_t d = i / kMaxQV, k = i % kMaxQV;
-        uint16_t v = 0;
-        if (d < p.qv && k < (uint32_t)(p.go_bni_offs[d + 1] - p.go_bni_offs[d])) {
-            const uint32_t bq = p.go_bni[p.go_bni_offs[d] + k];
-            v = (uint16_t)(p.eidx[p.go_vs[bq] * kMaxQV + p.go_vs[d]] | (bq << 8));
-        }
-        L->pair[d][k] = v;
-    }
-    for (uint32_t e = t; e < (uint32_t)kMaxQE; e += kWave) {
-        uint64_t a0 = 0, a1 = 0;
-        uint32_t ones = 0, own = 0;
-        if (e < p.qe) {
-            for (uint32_t dir = 0; dir < p.ndir; dir++)
-                if (p.dir_to_edge[dir] < e) {
-                    if (dir < 64) a0 |= 1ull << dir;
-                    else a1 |= 1ull << (dir - 64);
-                }
-            for (uint32_t q = 0; q < p.qv; q++)
-                if (T.P->all_ones[e][q]) ones |= 1u << q;
-            own = (uint32_t)T.P->sa[e] | ((uint32_t)T.P->sb[e] << 8);
-        }
-        L->app[e][0] = a0;
-        L->app[e][1] = a1;
-        L->ones[e] = ones;
-        L->own[e] = own;
-    }
-    if (t < (uint32_t)kMaxQV) L->dep_mask[t] = T.P->dep_mask[t];
-    if (t == 0) {
-        uint64_t vs = 0, cls = 0, nbn = 0;
-        for (uint32_t d = 0; d < p.qv; d++) {
-            vs |= (uint64_t)p.go_vs[d] << (4 * d);
-            cls |= (uint64_t)p.go_lcls[d] << (4 * d);
-            nbn |= (uint64_t)(p.go_bni_offs[d + 1] - p.go_bni_offs[d]) << (4 * d);
-        }
-        L->vs = vs;
-        L->cls = cls;
-        L->nbn = nbn;
-    }
+__device__ __forceinline__ void FillPlanLdsWave(const Tables& T, PlanLds* L) {
+    const uint64_t* src = (const uint64_t*)&T.P->lds;
+    for (uint32_t i = LaneId(); i < sizeof(PlanLds) / 8; i += kWave) ((uint64_t*)L)[i] = LdG(src + i);
     WaveSync();
 }
 
@@ -538,6 +446,14 @@ __global__ void __launch_bounds__(kThreads) KExtend(Tables T, const uint32_t* __
     }
 }
 
+// What a final-DFS launch can meet, fixed at compile time so that the common
+// launch does not carry the registers of the paths it cannot take:
+//   kDfsGeneral  every job;
+//   kDfsTuples   emits the embeddings;
+//   kDfsBatched  every job counts a batched product suffix with the default
+//                options (kJobBatched).
+enum { kDfsGeneral, kDfsTuples, kDfsBatched };
+
 struct DfsLevel {
     uint32_t off, cnt, pos, end;  // scan offset, survivors, next survivor, range end (exclusive)
     uint32_t sel;                 // backward neighbour whose list is scanned (kNoSel: not chosen yet)
@@ -585,13 +501,26 @@ __device__ __forceinline__ uint32_t GetAgent(const uint32_t* p) {
 // (lane 0) and read once at the end.  Held in scalar registers they were
 // spilled to memory by the pressure of the candidate loops, a round trip on
 // every step.
-struct WaveStats {
-    unsigned long long steps, step_lanes, batched, donated, scanned, probes;
+struct WaveStats {  // in the order of DfsOut::stat
+    unsigned long long scanned, probes, steps, step_lanes, batched, donated, wave_ticks, idle_ticks;
 };
+static_assert(sizeof(WaveStats) == kDfsStats * sizeof(unsigned long long), "one word per statistic");
 typedef __attribute__((address_space(3))) WaveStats LdsStats;
 __device__ __forceinline__ void StatAdd(__attribute__((address_space(3))) unsigned long long& f, unsigned long long v) {
     if (LaneId() == 0) __hip_atomic_fetch_add(&f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
+
+// A block's latest reading of the shared queue words.
+struct Hint {
+    long long t_poll, t_host;
+    uint32_t idle, stop;  // waves waiting for work; the launch was asked to stop
+};
+
+// Marks a ticket's slot (seq = ticket + 1 with this bit) when no work is left.
+constexpr unsigned long long kSeqDone = 1ull << 63;
+// An idle wave's sleep between looks at its slot: kIdleSleep * 64 cycles,
+// doubled up to kIdleMax times that.
+constexpr uint32_t kIdleSleep = 16, kIdleMax = 8;
 
 __device__ __forceinline__ void PublishItem(StealQueue& Q, uint64_t slot, unsigned long long ticket) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -603,7 +532,9 @@ __device__ __forceinline__ void PublishItem(StealQueue& Q, uint64_t slot, unsign
 // k must be the same in every lane.
 __device__ __forceinline__ List BnList(const Ctx& X, const Tables& T, uint32_t d, uint32_t k, const uint32_t* matched) {
     const uint32_t pr = Pair(X, d, k);
-    return Resolve(X, T, pr & 0xFFu, Uniform(matched[pr >> 8]));
+    const List L = Resolve(X, T, pr & 0xFFu, Uniform(matched[pr >> 8]));
+    return List{(const uint32_t*)Uniform64((uint64_t)L.base), (const uint32_t*)Uniform64((uint64_t)L.app),
+                Uniform(L.bl), Uniform(L.al)};
 }
 
 // Occurrences test by binary search in both parts of a list (probes counted).
@@ -854,7 +785,9 @@ __device__ __forceinline__ void StabBuild(const Ctx& X, const Tables& T, uint32_
 // B (bit mask, all at or after j0): every backward-neighbour list of every
 // position of B, and the support-mask bit of each.  `raw` leaves the
 // positions 0..j0-1 in; `hits` counts those of them that lie in C_B (only
-// positions of the same label class can).  All lists must be sets.
+// positions of the same label class can).  All lists must be sets.  kOne: B
+// holds one position.
+template <bool kOne>
 __device__ __forceinline__ void SetSize(const Ctx& X, const Tables& T, uint32_t B, uint32_t j0, const uint32_t* matched, bool need_raw,
                         uint32_t& raw, uint32_t& hits, StabCache& sc, uint32_t& scanned,
                         uint32_t& probes) {
@@ -912,7 +845,7 @@ __device__ __forceinline__ void SetSize(const Ctx& X, const Tables& T, uint32_t 
     }
     // Source: the shortest list over all (position, backward neighbour) pairs.
     uint32_t best = 0xFFFFFFFFu, src_j = jf, src_k = 0, npairs = 0;
-    for (uint32_t bb = B; bb; bb &= bb - 1) {
+    for (uint32_t bb = B; bb; bb = kOne ? 0u : bb & (bb - 1)) {
         const uint32_t j = (uint32_t)__builtin_ctz(bb);
         const uint32_t nbn = Nbn(X, j);
         for (uint32_t k = 0; k < nbn; k++, npairs++) {
@@ -925,9 +858,9 @@ __device__ __forceinline__ void SetSize(const Ctx& X, const Tables& T, uint32_t 
             }
         }
     }
-    const bool single = (B & (B - 1)) == 0 && npairs == 1 && ((X.ones >> Vs(X, jf)) & 1u);
+    const bool single = (kOne || (B & (B - 1)) == 0) && npairs == 1 && ((X.ones >> Vs(X, jf)) & 1u);
     auto member = [&](uint32_t c, bool skip_src) -> bool {
-        for (uint32_t bb = B; bb; bb &= bb - 1) {
+        for (uint32_t bb = B; bb; bb = kOne ? 0u : bb & (bb - 1)) {
             const uint32_t j = (uint32_t)__builtin_ctz(bb);
             if (!TileBit(X, T, Vs(X, j), c)) return false;
             const uint32_t nbn = Nbn(X, j);
@@ -972,7 +905,7 @@ __device__ __forceinline__ void SetSize(const Ctx& X, const Tables& T, uint32_t 
 // 0..j0-1; the planner keeps classes of the suffix to 3 members).  Raw
 // sizes of single positions are cached per wave (valid bits in `cvalid`)
 // until a position they depend on changes.
-__device__ unsigned long long SuffixCount(const Ctx& X, const Tables& T, uint32_t j0, const uint32_t* matched,
+__device__ __forceinline__ unsigned long long SuffixCount(const Ctx& X, const Tables& T, uint32_t j0, const uint32_t* matched,
                                           uint32_t* csize, uint32_t& cvalid, StabCache& sc,
                                           uint32_t& scanned, uint32_t& probes) {
     const uint32_t qv = X.qv;
@@ -1008,7 +941,7 @@ __device__ unsigned long long SuffixCount(const Ctx& X, const Tables& T, uint32_
             const uint32_t pi = t == 0 ? p0 : t == 1 ? p1 : p2;
             const bool cached = single && ((cvalid >> pi) & 1u);
             uint32_t raw = cached ? Uniform(csize[pi]) : 0, hits = 0;
-            SetSize(X, T, B, j0, matched, !cached, raw, hits, sc, scanned, probes);
+            SetSize<false>(X, T, B, j0, matched, !cached, raw, hits, sc, scanned, probes);
             if (single && !cached) {
                 if (LaneId() == 0) csize[pi] = raw;
                 cvalid |= 1u << pi;
@@ -1049,7 +982,8 @@ struct BxLds {
 // to end over the 64 lanes, each entry tested against j's other lists (or
 // the cached stable intersection) and its support mask, and counted per
 // sibling in LDS.  Equal to SuffixCount per sibling (identical counts).
-__device__ unsigned long long BatchSuffix(const Ctx& X, const Tables& T, uint32_t p, const uint32_t* matched,
+template <bool kLean>
+__device__ __forceinline__ unsigned long long BatchSuffix(const Ctx& X, const Tables& T, uint32_t p, const uint32_t* matched,
                                           uint64_t m, uint32_t x, uint32_t* csize, uint32_t& cvalid, StabCache& sc,
                                           BxLds& B, uint32_t& scanned, uint32_t& probes, uint32_t wmin) {
     const uint32_t lane = LaneId();
@@ -1090,7 +1024,7 @@ __device__ unsigned long long BatchSuffix(const Ctx& X, const Tables& T, uint32_
             if (hcached) {
                 hits = Uniform(csize[kMaxQV + j]);
             } else {
-                SetSize(X, T, 1u << j, p, matched, !cached, raw, hits, sc, scanned, probes);
+                SetSize<true>(X, T, 1u << j, p, matched, !cached, raw, hits, sc, scanned, probes);
                 if (lane == 0) {
                     csize[j] = raw;
                     csize[kMaxQV + j] = hits;
@@ -1102,14 +1036,14 @@ __device__ unsigned long long BatchSuffix(const Ctx& X, const Tables& T, uint32_
             // the sibling, so with the wave search on, the siblings (sorted,
             // one per lane) are searched in each list by the whole wavefront.
             const bool act = same && prod && val > 0;
-            if (wmin && __ballot(act)) {
+            if ((kLean || wmin) && __ballot(act)) {
                 bool in = act && TileBit(X, T, qj, x);
                 for (uint32_t k = 0; k < nbn; k++) {
                     if (!__ballot(in)) break;
                     in = InListLanes(BnList(X, T, j, k, matched), x, in, probes, wmin);
                 }
                 val -= in ? 1 : 0;
-            } else if (!wmin && act) {
+            } else if (!kLean && !wmin && act) {
                 bool in = TileBit(X, T, qj, x);
                 for (uint32_t k = 0; k < nbn && in; k++) in = InList(BnList(X, T, j, k, matched), x, probes);
                 val -= in ? 1 : 0;
@@ -1266,15 +1200,19 @@ __device__ unsigned long long BatchSuffix(const Ctx& X, const Tables& T, uint32_
 //  * the product suffix of the order (positions cp_start..qv-1, mutually
 //    non-adjacent) is never enumerated: a partial match of the positions
 //    before it adds SuffixCount.
-template <bool kTuples>
-__global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __restrict__ jobs, uint32_t njobs,
+template <int kMode>
+__global__ void __launch_bounds__(kThreads)
+    __attribute__((amdgpu_waves_per_eu(CGD_DFS_BLOCKS))) KDfs(const DfsJob* __restrict__ jobs, uint32_t njobs,
                                                               const unsigned long long* __restrict__ row_base,
-                                                              uint32_t grab, Counters* __restrict__ cnt, StealQueue Q,
+                                                              uint32_t grab, Counters* __restrict__ cnt,
+                                                              DfsOut* __restrict__ outs, StealQueue Q,
                                                               uint32_t* __restrict__ tuples, uint64_t tup_cap,
                                                               uint32_t surv_levels, uint32_t stab_cap) {
+    constexpr bool kTuples = kMode == kDfsTuples, kLean = kMode == kDfsBatched;
     // Per-edge counts gather in LDS per wave and reach the query's counters
-    // when the wave changes query or ends: a device-scope atomic per item on
-    // one address would serialize.
+    // when the wave changes query, or through this block's record of `outs`
+    // at the end (KDfsFold).  Device-scope atomics of all waves on one line
+    // serialize at about 10 ns each.
     __shared__ unsigned long long s_pe[kWpb][kMaxQE];
     __shared__ uint32_t s_matched[kWpb][kMaxQV];
     __shared__ DfsLevel s_lvl[kWpb][kMaxQV];
@@ -1282,6 +1220,8 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
     __shared__ uint32_t s_csize[kWpb][2 * kMaxQV];  // cached raw sizes, then cached hits
     __shared__ BxLds s_bx[kWpb];
     __shared__ WaveStats s_stats[kWpb];
+    __shared__ uint32_t s_job[kWpb];
+    __shared__ Hint s_hint;
     // Dynamic LDS, per wave: survivor stacks of surv_levels levels (64 u32
     // each; every job of the launch has qv - 1 <= surv_levels) and the
     // stable-intersection cache of stab_cap u32.
@@ -1303,7 +1243,7 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
     Counters* jc = nullptr;
     Ctx X = MakeCtx(T, &s_plan[wv]);
     StabCache sc{stab, stab_cap, 0, 0, 0, 0xFFu, 0, 0};
-    bool sets = false, cart = false, bsfx = false, wsearch = false;
+    bool sets = kLean, cart = kLean, bsfx = kLean, wsearch = kLean;
     uint32_t wmin = kWaveSearchMin;
     auto flush_pe = [&]() {
         if (!jc) return;
@@ -1327,17 +1267,25 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
         X = MakeCtx(T, &s_plan[wv]);
         qv = X.qv;
         last = qv - 1;
-        tag_shift = T.P->tag_shift;
-        v_mask = T.P->v_mask;
-        sc = StabCache{stab, stab_cap, 0, 0, 0, T.P->stab_pos, T.P->stab_var_k, T.P->stab_deps};
+        // Loads through a pointer read from memory count as per-lane values
+        // to the compiler, and one branch on such a value makes every value
+        // the main loop carries per-lane too: each is read first lane.
+        tag_shift = Uniform(LdG(&T.P->tag_shift));
+        v_mask = Uniform(LdG(&T.P->v_mask));
+        sc = StabCache{stab, stab_cap, 0, 0, 0, Uniform(LdG(&T.P->stab_pos)), Uniform(LdG(&T.P->stab_var_k)),
+                       Uniform(LdG(&T.P->stab_deps))};
         // Every list is a set when the update lists hold no duplicate value.
-        const bool lists_are_sets = Uniform64(jc->u_dups) == 0;
         const uint32_t opts = jobs[j].opts;
-        sets = (opts & kJobShortest) && lists_are_sets;
-        cps = T.P->cp_start;
-        cart = !kTuples && lists_are_sets && (opts & kJobSuffix) && cps < qv;
-        bsfx = cart && T.P->sfx_batch;
-        wsearch = (opts & kJobWaveSearch) != 0;
+        cps = Uniform(LdG(&T.P->cp_start));
+        if constexpr (kLean) {
+            sets = cart = bsfx = wsearch = true;
+        } else {
+            const bool lists_are_sets = Uniform64(LdG(&jc->u_dups)) == 0;
+            sets = (opts & kJobShortest) && lists_are_sets;
+            cart = !kTuples && lists_are_sets && (opts & kJobSuffix) && cps < qv;
+            bsfx = cart && Uniform(LdG(&T.P->sfx_batch));
+            wsearch = (opts & kJobWaveSearch) != 0;
+        }
         // At least 64 entries: every lane's bucket pivot index is >= 0.
         wmin = (opts >> kJobWaveShift) & 31u ? 1u << ((opts >> kJobWaveShift) & 31u) : kWaveSearchMin;
         wmin = wmin < (uint32_t)kWave ? (uint32_t)kWave : wmin;
@@ -1361,42 +1309,74 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
         my_scanned = 0;
         my_probes = 0;
     };
-    uint64_t r_next = 0, r_end = 0, r_first = 0, ticket = 0;
+    // Every row is handed out by the cursor: a share fixed by the block index
+    // would wait for a block that another launch keeps from running, whose own
+    // blocks may be waiting the same way.  Rows retire from `pending`
+    // together, when the wave finds no more of them.
+    uint64_t r_next = 0, r_end = 0, held = 0, ticket = 0;
     bool primary = true, idle = false, stop = false, have_ticket = false, from_row = false;
-    uint32_t iter = 0, backoff = 1;
+    uint32_t iter = 0, backoff = 1, waits = 0;
     // Shared words (idle count, flags) and the host flag are read at most
-    // once per poll_ticks / host_ticks of wall clock per wave: thousands of
-    // waves polling one address would otherwise saturate the memory-side
-    // path that agent-scope loads take and stall the waves that work.
-    long long t_poll = Uniform64(wall_clock64()), t_host = t_poll;
-    const long long t_born = t_poll;
+    // once per poll_ticks / host_ticks of wall clock per block, by whichever
+    // wave finds the block's last reading (s_hint) too old: thousands of waves
+    // polling one address would otherwise saturate the memory-side path that
+    // agent-scope loads take and stall the waves that work.
+    const long long t_born = (long long)Uniform64((unsigned long long)wall_clock64());
+    if (threadIdx.x == 0) s_hint = Hint{t_born, t_born, 0, 0};
+    __syncthreads();
+    volatile Hint* hint = &s_hint;
     long long t_idle0 = 0, idle_sum = 0;
-    unsigned long long idl_hint = 0;
+    uint32_t idl_hint = 0;
     // Returns true when the kernel is asked to stop.
     auto poll = [&]() -> bool {
         const long long now = (long long)Uniform64((unsigned long long)wall_clock64());
-        if (now - t_poll < Q.poll_ticks) return false;
-        t_poll = now;
         if (__ballot(my_scanned >= (1u << 30) || my_probes >= (1u << 30))) fold();
-        const bool host = now - t_host >= Q.host_ticks;
-        if (host) t_host = now;
-        unsigned long long idl = 0, fl = 0;
-        int ab = 0;
-        if (lane == 0) {
-            // Waves waiting for work hold tickets at or above the tail.
-            const unsigned long long h = LoadAgent(&cnt->q_head.v), t = LoadAgent(&cnt->q_tail.v);
-            idl = h > t ? h - t : 0;
-            fl = LoadAgent(&cnt->flags);
-            if (host && AbortRequested(Q)) {
-                atomicOr(&cnt->flags, kFlagAborted);
-                ab = 1;
+        if (now - (long long)Uniform64((unsigned long long)hint->t_poll) >= Q.poll_ticks) {
+            if (lane == 0) {
+                hint->t_poll = now;
+                // Waves waiting for work hold tickets at or above the tail.
+                const unsigned long long h = LoadAgent(&cnt->q_head.v), t = LoadAgent(&cnt->q_tail.v);
+                hint->idle = h > t ? (uint32_t)(h - t) : 0u;
+                unsigned long long fl = LoadAgent(&cnt->flags);
+                if (now - hint->t_host >= Q.host_ticks) {
+                    hint->t_host = now;
+                    if (AbortRequested(Q)) {
+                        atomicOr(&cnt->flags, kFlagAborted);
+                        fl |= kFlagAborted;
+                    }
+                }
+                if (fl & kFlagAborted) hint->stop = 1;
             }
+            WaveSync();
         }
         // Uniform values (read first lane): branches on them stay scalar, so
         // the loops' carried state can stay in scalar registers.
-        idl_hint = ReadLane64(idl, 0);
-        fl = ReadLane64(fl, 0);
-        return ReadLane((uint32_t)ab, 0) || (fl & kFlagAborted);
+        idl_hint = Uniform(hint->idle);
+        return Uniform(hint->stop) != 0;
+    };
+    // The waves this one handed k pieces to no longer wait.
+    auto took = [&](uint32_t k) {
+        idl_hint = idl_hint > k ? idl_hint - k : 0;
+        if (lane == 0) hint->idle = idl_hint;
+    };
+    // k rows or items are finished.  The wave that brings `pending` to zero
+    // ends the launch: it marks the slots of all tickets still waiting, so
+    // that idle waves watch their own slot alone.  (A ticket is taken before
+    // its wave reads `pending`: one taken after this head was read finds zero.)
+    auto retire = [&](uint64_t k) {
+        unsigned long long last = 0, h = 0, t = 0;
+        if (lane == 0) {
+            last = atomicSub(&cnt->q_pending.v, (unsigned long long)k) == k;
+            if (last) {
+                h = LoadAgent(&cnt->q_head.v);
+                t = LoadAgent(&cnt->q_tail.v);
+            }
+        }
+        h = ReadLane64(h, 0);
+        t = ReadLane64(t, 0);
+        for (uint64_t i = t + lane; i < h; i += kWave)
+            __hip_atomic_store(&Q.seq[i & (Q.cap - 1)], (i + 1) | kSeqDone, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
     };
     while (!stop) {
         // ---------------- obtain a work item
@@ -1409,8 +1389,12 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
                 r0 = ReadLane64(r0, 0);
                 r_next = r0;
                 r_end = r0 + grab < n_rows ? r0 + grab : n_rows;
-                r_first = r0;
-                if (r0 >= n_rows) primary = false;
+                if (r0 >= n_rows) {
+                    primary = false;
+                    if (held) retire(held);
+                } else {
+                    held += r_end - r0;
+                }
             }
             if (primary) {
                 const uint64_t r = r_next++;
@@ -1431,10 +1415,7 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
                 // written out of order with this launch) is not followed into
                 // the index: it is dropped and flagged, and the call fails.
                 if (ei >= T.qe || __ballot(lane < D && mv >= T.dv)) {
-                    if (lane == 0) {
-                        atomicOr(&cnt->flags, kFlagBadRow);
-                        if (r_next >= r_end) atomicSub(&cnt->q_pending.v, (unsigned long long)(r_end - r_first));
-                    }
+                    if (lane == 0) atomicOr(&cnt->flags, kFlagBadRow);
                     continue;
                 }
                 if (lane < D) matched[lane] = mv;
@@ -1444,18 +1425,19 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
         }
         if (!got) {
             // One ticket per idle wave (fetch-and-add, no retries): the wave
-            // then waits on its own slot until a donor fills it or no work
-            // is left anywhere (`pending` = rows and items not yet finished;
-            // donations only come from waves holding one, so none can
-            // arrive once it is zero).
+            // then waits on its own slot until a donor fills it or the last
+            // piece of work is retired (`pending` = rows and items not yet
+            // finished; donations only come from waves holding one, so none
+            // can arrive once it is zero).
+            bool check = false;
             if (!have_ticket) {
                 unsigned long long tk = 0;
-                if (lane == 0) {
-                    tk = atomicAdd(&cnt->q_head.v, 1ull);
-                }
+                if (lane == 0) tk = atomicAdd(&cnt->q_head.v, 1ull);
                 ticket = ReadLane64(tk, 0);
                 have_ticket = true;
                 idle = true;
+                check = true;
+                waits = 0;
                 t_idle0 = (long long)Uniform64((unsigned long long)wall_clock64());
             }
             const uint64_t slot = ticket & (Q.cap - 1);
@@ -1480,13 +1462,16 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
                 idle = false;
                 idle_sum += (long long)Uniform64((unsigned long long)wall_clock64()) - t_idle0;
             } else {
-                unsigned long long pend = 0;
-                if (lane == 0) pend = LoadAgent(&cnt->q_pending.v);
-                pend = ReadLane64(pend, 0);
-                if (pend == 0) break;
+                if (sq == ((ticket + 1) | kSeqDone)) break;
+                if (check || (++waits & 255u) == 0) {
+                    unsigned long long pend = 0;
+                    if (lane == 0) pend = LoadAgent(&cnt->q_pending.v);
+                    pend = ReadLane64(pend, 0);
+                    if (pend == 0) break;
+                }
                 if (poll()) break;
-                for (uint32_t b = 0; b < backoff; b++) __builtin_amdgcn_s_sleep(63);
-                backoff = backoff < 16 ? backoff * 2 : 16;
+                for (uint32_t b = 0; b < backoff; b++) __builtin_amdgcn_s_sleep(kIdleSleep);
+                backoff = backoff < kIdleMax ? backoff * 2 : kIdleMax;
                 continue;
             }
         }
@@ -1506,7 +1491,7 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
                 break;
             }
             // The product suffix is counted, not enumerated.
-            if (cart && d >= cps) {
+            if (!kLean && cart && d >= cps) {
                 count = SatAdd(count, SuffixCount(X, T, d, matched, s_csize[wv], cvalid, sc, my_scanned, my_probes));
                 if (d == D0) break;
                 d--;
@@ -1553,7 +1538,7 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
                             }
                             StatAdd(ws->donated, k);
                             ccount -= k;
-                            idl_hint = idl_hint > k ? idl_hint - k : 0;
+                            took(k);
                             if (lane == 0) lvl[d].cnt = ccount;
                             WaveSync();
                         }
@@ -1592,7 +1577,7 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
             // carries a whole suffix count and its survivors are not descended
             // into, so its ranges are split down to one step each (smaller
             // pieces would repeat the per-item set-up of the suffix sizes).
-            const bool blev = bsfx && d + 1 == cps;
+            const bool blev = (kLean || bsfx) && d + 1 == cps;
             const uint32_t rmin = blev ? kWave : Q.range_min;
             if (Q.donate_min && idl_hint > 0 && limit - off >= 2 * rmin) {
                 unsigned long long h = 0, t = 0;
@@ -1626,7 +1611,7 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
                         PublishItem(Q, slot, t0 + lane);
                     }
                     StatAdd(ws->donated, k);
-                    idl_hint = idl_hint > k ? idl_hint - k : 0;
+                    took(k);
                     limit = off + piece;
                     if (lane == 0) lvl[d].end = limit;
                     WaveSync();
@@ -1637,7 +1622,7 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
             bool ok = false;
             StatAdd(ws->steps, 1);
             StatAdd(ws->step_lanes, limit - off < kWave ? limit - off : kWave);
-            if (wsearch) {
+            if (kLean || wsearch) {
                 if (i < limit) {
                     c = At(L, i);
                     my_scanned++;
@@ -1653,7 +1638,7 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
             // every survivor of this step at once instead of descending.
             if (blev) {
                 if (m) {
-                    count = SatAdd(count, BatchSuffix(X, T, d, matched, m, c, s_csize[wv], cvalid, sc, s_bx[wv],
+                    count = SatAdd(count, BatchSuffix<kLean>(X, T, d, matched, m, c, s_csize[wv], cvalid, sc, s_bx[wv],
                                                       my_scanned, my_probes, wsearch ? wmin : 0u));
                     StatAdd(ws->batched, 1);
                 }
@@ -1661,7 +1646,7 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
                 WaveSync();
                 continue;
             }
-            if (d == last) {
+            if (!kLean && d == last) {
                 count = SatAdd(count, (unsigned long long)__popcll(m));
                 if (kTuples && ok) {
                     unsigned long long slot = atomicAdd(&cnt->tuples, 1ull);
@@ -1687,32 +1672,87 @@ __global__ void __launch_bounds__(kThreads) CGD_DFS_ATTR KDfs(const DfsJob* __re
             }
             WaveSync();
         }
-        if (lane == 0) {
-            if (count) pe[ei] = SatAdd(pe[ei], count);
-            // Rows retire from `pending` a whole grab at a time, stolen items one by one.
-            if (!from_row) atomicSub(&cnt->q_pending.v, 1ull);
-            else if (r_next >= r_end) atomicSub(&cnt->q_pending.v, (unsigned long long)(r_end - r_first));
-        }
+        if (lane == 0 && count) pe[ei] = SatAdd(pe[ei], count);
+        if (!from_row) retire(1);  // stolen items retire one by one
     }
-    {
-        const long long now = (long long)Uniform64((unsigned long long)wall_clock64());
-        if (idle) idle_sum += now - t_idle0;
-        if (lane == 0) {
-            atomicAdd(&cnt->wave_ticks, (unsigned long long)(now - t_born));
-            atomicAdd(&cnt->idle_ticks, (unsigned long long)idle_sum);
-        }
-    }
+    const long long now = (long long)Uniform64((unsigned long long)wall_clock64());
+    if (idle) idle_sum += now - t_idle0;
     fold();
-    WaveSync();
     if (lane == 0) {
-        atomicAdd(&cnt->scanned, (unsigned long long)ws->scanned);
-        atomicAdd(&cnt->probes, (unsigned long long)ws->probes);
-        atomicAdd(&cnt->steps, (unsigned long long)ws->steps);
-        atomicAdd(&cnt->step_lanes, (unsigned long long)ws->step_lanes);
-        if (ws->batched) atomicAdd(&cnt->batched, (unsigned long long)ws->batched);
-        if (ws->donated) atomicAdd(&cnt->donated, (unsigned long long)ws->donated);
+        ws->wave_ticks = (unsigned long long)(now - t_born);
+        ws->idle_ticks = (unsigned long long)idle_sum;
+        s_job[wv] = job;
     }
-    flush_pe();
+    __syncthreads();
+    // The block's record: statistics summed over its waves; per-edge counts
+    // under the first wave of each query, the other waves' slots marked empty.
+    DfsOut* o = outs + blockIdx.x;
+    const uint32_t t = threadIdx.x;
+    if (t < (uint32_t)kDfsStats) {
+        unsigned long long v = 0;
+        for (uint32_t w = 0; w < (uint32_t)kWpb; w++) v += ((const unsigned long long*)&s_stats[w])[t];
+        o->stat[t] = v;
+    }
+    for (uint32_t w = 0; w < (uint32_t)kWpb; w++) {
+        bool first = s_job[w] != 0xFFFFFFFFu;
+        for (uint32_t v = 0; v < w; v++) first = first && s_job[v] != s_job[w];
+        if (t == 0) o->job[w] = first ? s_job[w] : 0xFFFFFFFFu;
+        if (first && t < (uint32_t)kMaxQE) {
+            unsigned long long v = s_pe[w][t];
+            for (uint32_t u = w + 1; u < (uint32_t)kWpb; u++)
+                if (s_job[u] == s_job[w]) v = SatAdd(v, s_pe[u][t]);
+            o->pe[w][t] = v;
+        }
+    }
+}
+
+// Adds the block records of a final-DFS launch to the counters: block j sums
+// the per-edge counts of query j, block 0 also the launch's statistics.
+__global__ void __launch_bounds__(kThreads) KDfsFold(const DfsJob* __restrict__ jobs, const DfsOut* __restrict__ outs,
+                                                     uint32_t n, Counters* __restrict__ cnt) {
+    __shared__ unsigned long long s_sum[kMaxQE], s_stat[kDfsStats];
+    __shared__ uint32_t s_wide;
+    const uint32_t t = threadIdx.x, j = blockIdx.x;
+    if (t < (uint32_t)kMaxQE) s_sum[t] = 0;
+    if (t < (uint32_t)kDfsStats) s_stat[t] = 0;
+    if (t == 0) s_wide = 0;
+    __syncthreads();
+    Counters* jc = jobs[j].cnt;
+    const uint32_t qe = jobs[j].T.qe;
+    for (uint32_t i = t; i < n * kWpb; i += kThreads) {
+        const DfsOut* o = outs + i / kWpb;
+        const uint32_t w = i % kWpb;
+        if (o->job[w] != j) continue;
+        for (uint32_t e = 0; e < qe; e++) {
+            const unsigned long long v = o->pe[w][e];
+            if (!v) continue;
+            const unsigned long long old = atomicAdd(&s_sum[e], v);
+            if (v == kCountSat || old + v < old) s_wide = 1;
+        }
+    }
+    if (j == 0)
+        for (uint32_t i = t; i < n * kDfsStats; i += kThreads)
+            atomicAdd(&s_stat[i % kDfsStats], outs[i / kDfsStats].stat[i % kDfsStats]);
+    __syncthreads();
+    if (t < qe) {
+        const unsigned long long a = jc->per_edge[t], v = s_sum[t];
+        jc->per_edge[t] = a + v;
+        if (a + v < a) s_wide = 1;
+    }
+    __syncthreads();
+    if (t == 0) {
+        if (s_wide) atomicOr(&jc->count_ovf, 1ull);
+        if (j == 0) {
+            cnt->scanned = s_stat[0];
+            cnt->probes = s_stat[1];
+            cnt->steps = s_stat[2];
+            cnt->step_lanes = s_stat[3];
+            cnt->batched = s_stat[4];
+            cnt->donated = s_stat[5];
+            cnt->wave_ticks = s_stat[6];
+            cnt->idle_ticks = s_stat[7];
+        }
+    }
 }
 
 // Before a DFS launch: tickets taken but never filled in the previous launch
@@ -1774,7 +1814,7 @@ constexpr size_t DfsBlockLds(int nb) { return ((size_t)(160 * 1024 - 4096) / (si
 // LDS plan of a final-DFS launch: the register budget fixes the resident
 // blocks per CU; the LDS those blocks leave after the static tables is split
 // among their waves into survivor stacks and the stable-intersection cache.
-template <bool kTuples>
+template <int kMode>
 DfsShape DfsLdsShapeT(uint32_t surv_levels) {
     static DfsShape cache[kMaxQV + 1] = {};
     static std::mutex mu;  // queries launch from several host threads
@@ -1784,15 +1824,16 @@ DfsShape DfsLdsShapeT(uint32_t surv_levels) {
     if (c.blocks_per_cu) return c;
     int nb = 0;
     const size_t surv_bytes = (size_t)kWpb * surv_levels * kWave * sizeof(uint32_t);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, KDfs<kTuples>, kThreads, surv_bytes) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, KDfs<kMode>, kThreads, surv_bytes) != hipSuccess ||
         nb <= 0)
         throw HipError(hipErrorInvalidValue, "final-DFS occupancy query", __FILE__, __LINE__);
+    nb = std::min(nb, CGD_DFS_BLOCKS);
     // The cache takes what is left of DfsBlockLds per block.  The occupancy
     // query accepted 54.2 KB blocks at 3 per CU, but those ran 25 % slower
     // than 53.2 KB ones (measured), as if only 2 blocks fit: the budget is
     // the largest block measured to run at full occupancy.
     hipFuncAttributes attr{};
-    if (hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(KDfs<kTuples>)) != hipSuccess)
+    if (hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(KDfs<kMode>)) != hipSuccess)
         throw HipError(hipErrorInvalidValue, "final-DFS attributes", __FILE__, __LINE__);
     const size_t fixed = attr.sharedSizeBytes + surv_bytes;
     const size_t budget = DfsBlockLds(nb);
@@ -1801,7 +1842,7 @@ DfsShape DfsLdsShapeT(uint32_t surv_levels) {
     for (;; cap = cap >= 64 ? cap - 64 : 0) {
         const size_t dyn = surv_bytes + (size_t)kWpb * cap * sizeof(uint32_t);
         int got = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&got, KDfs<kTuples>, kThreads, dyn) == hipSuccess &&
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&got, KDfs<kMode>, kThreads, dyn) == hipSuccess &&
             got >= nb) {
             c.dyn_bytes = (uint32_t)dyn;
             c.stab_cap = cap;
@@ -1812,29 +1853,34 @@ DfsShape DfsLdsShapeT(uint32_t surv_levels) {
     }
 }
 
-DfsShape DfsLdsShape(uint32_t surv_levels, bool tuples) {
-    return tuples ? DfsLdsShapeT<true>(surv_levels) : DfsLdsShapeT<false>(surv_levels);
+DfsShape DfsLdsShape(uint32_t surv_levels, bool tuples, bool batched) {
+    return tuples    ? DfsLdsShapeT<kDfsTuples>(surv_levels)
+           : batched ? DfsLdsShapeT<kDfsBatched>(surv_levels)
+                     : DfsLdsShapeT<kDfsGeneral>(surv_levels);
 }
-
-uint32_t DfsBlocksPerCU() { return DfsLdsShape(kMaxQV, false).blocks_per_cu; }
 
 void LaunchQueueSync(Counters* cnt, hipStream_t s) { KQueueSync<<<1, 64, 0, s>>>(cnt); }
 
-void LaunchDfs(const DfsJob* jobs, uint32_t njobs, const unsigned long long* row_base, uint64_t n_rows, Counters* cnt,
-               const StealQueue& Q, uint32_t* tuples, uint64_t tup_cap, uint32_t num_cus, uint32_t blocks_per_cu,
-               uint32_t grab, uint32_t surv_levels, uint32_t cache_cap, hipStream_t s) {
-    if (!n_rows || !njobs) return;
-    DfsShape sh = DfsLdsShape(surv_levels, tuples != nullptr);
-    if (cache_cap && cache_cap < sh.stab_cap) sh.stab_cap = cache_cap & ~63u;
+uint32_t DfsGrid(const DfsShape& sh, uint64_t n_rows, uint32_t num_cus, uint32_t blocks_per_cu) {
     const uint32_t bpc = blocks_per_cu && blocks_per_cu < sh.blocks_per_cu ? blocks_per_cu : sh.blocks_per_cu;
-    const unsigned g = Grid1(n_rows, kWpb, num_cus * bpc);
+    return Grid1(n_rows, kWpb, num_cus * bpc);
+}
+
+void LaunchDfs(const DfsJob* jobs, uint32_t njobs, const unsigned long long* row_base, uint64_t n_rows, Counters* cnt,
+               DfsOut* outs, const StealQueue& Q, uint32_t* tuples, uint64_t tup_cap, const DfsShape& sh, uint32_t grid,
+               uint32_t grab, uint32_t surv_levels, uint32_t stab_cap, bool batched, hipStream_t s) {
+    if (!n_rows || !njobs) return;
     grab = grab < 1 ? 1 : grab;
     if (tuples)
-        KDfs<true><<<g, kThreads, sh.dyn_bytes, s>>>(jobs, njobs, row_base, grab, cnt, Q, tuples, tup_cap,
-                                                      surv_levels, sh.stab_cap);
+        KDfs<kDfsTuples><<<grid, kThreads, sh.dyn_bytes, s>>>(jobs, njobs, row_base, grab, cnt, outs, Q, tuples,
+                                                              tup_cap, surv_levels, stab_cap);
+    else if (batched)
+        KDfs<kDfsBatched><<<grid, kThreads, sh.dyn_bytes, s>>>(jobs, njobs, row_base, grab, cnt, outs, Q, nullptr, 0,
+                                                               surv_levels, stab_cap);
     else
-        KDfs<false><<<g, kThreads, sh.dyn_bytes, s>>>(jobs, njobs, row_base, grab, cnt, Q, nullptr, 0, surv_levels,
-                                                       sh.stab_cap);
+        KDfs<kDfsGeneral><<<grid, kThreads, sh.dyn_bytes, s>>>(jobs, njobs, row_base, grab, cnt, outs, Q, nullptr, 0,
+                                                               surv_levels, stab_cap);
+    KDfsFold<<<njobs, kThreads, 0, s>>>(jobs, outs, grid, cnt);
 }
 
 }  // namespace cgd

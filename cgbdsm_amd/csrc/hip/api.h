@@ -31,6 +31,8 @@ struct cgbdsm_ctx {
     int wall_khz = 100000;  // device wall clock (wall_clock64) rate
 };
 
+constexpr uint64_t kBfsRowLimit = 65536;  // default of cgbdsm_set_match_params
+
 // Rows left for the final DFS after seeds and BFS levels: count, depth and
 // which of the two frontier buffers holds them.
 struct Frontier {
@@ -57,10 +59,12 @@ struct cgbdsm_query {
     DBuf<uint8_t> scan_scratch;
     DBuf<uint64_t> masks;
     DBuf<uint32_t> front[2];
+    DBuf<uint64_t> ext_offs;  // BFS level: first candidate of each row
+    DBuf<uint8_t> ext_sel;    // and its scanned backward neighbour
     DBuf<unsigned long long> tag_hist;  // 2 * kMaxQE counters of the seed grouping
     uint64_t n_ins = 0, n_del = 0, n_upd = 0, u_rows_upper = 0;
     uint8_t edge_ok[kMaxQE] = {};
-    uint64_t bfs_row_limit = 65536, frontier_cap_rows = 0;
+    uint64_t bfs_row_limit = kBfsRowLimit, frontier_cap_rows = 0;
     uint32_t donate_min = 4;
     bool dfs_shortest = true, dfs_suffix = true;
     // Final-DFS launch shape: frontier rows taken per cursor atomic, and

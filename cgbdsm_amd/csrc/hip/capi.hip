@@ -809,6 +809,8 @@ cgbdsm_status cgbdsm_query_destroy(cgbdsm_query* q) {
         Release(q, q->pma.meta);
         Release(q, q->d_jobs);
         Release(q, q->dfs_out);
+        Release(q, q->ext_offs);
+        Release(q, q->ext_sel);
         Release(q, q->d_rowbase);
         Release(q, q->tag_hist);
         for (auto& r : q->fifo) {
@@ -1235,6 +1237,9 @@ cgbdsm_status cgbdsm_set_deadline_ms(cgbdsm_query* q, double ms) {
     });
 }
 
+// Words (64 MiB) a BFS level past the row limit may take.
+static constexpr uint64_t kExtendWords = 16ull << 20;
+
 // Seeds and BFS levels of one query's matching (phase 4): the rows left for
 // the final DFS, their depth and the buffer holding them, kept in q->fr.
 // The last kernel (the tag grouping) may still run on q's stream on return;
@@ -1288,21 +1293,46 @@ static const Frontier& BuildFrontier(cgbdsm_query* q) {
     // before the suffix (cp_start - 1) itself: BFS levels stop short of it.
     const bool batched_suffix =
         q->hplan.sfx_batch && q->dfs_suffix && q->h_cnt->u_dups == 0 && q->hplan.cp_start < q->qv;
-    while (n > 0 && n < q->bfs_row_limit && depth + 1 < q->qv &&
-           !(batched_suffix && depth + 2 > q->hplan.cp_start)) {
-        const uint64_t want_rows =
-            fixed_cap ? q->frontier_cap_rows : std::min<uint64_t>(std::max<uint64_t>(n * 64, 1u << 20), 1ull << 28);
-        const uint64_t want_words = want_rows * (depth + 1);
-        Ensure(q, q->front[cur ^ 1], want_words);
-        SetCounter(q, &Counters::rows_out, 0);
-        SetCounter(q, &Counters::flags, 0);
-        const int ke = KBegin(q, CGBDSM_K_EXTEND);
-        LaunchExtend(T, q->front[cur].p, n, depth, q->front[cur ^ 1].p, q->front[cur ^ 1].cap / (depth + 1),
-                     q->d_cnt, q->s);
-        KEnd(q, ke);
-        ReadCounters(q);
-        KAdd(q, CGBDSM_K_EXTEND, 0, n);
-        if (q->h_cnt->flags & kFlagFrontier) break;  // keep this level, count it by DFS
+    // Rows at the position the batched suffix starts from balance by the row
+    // cursor, where shallower ones are split up by donations that cost more
+    // than the level written out (dense 6-vertex query on scale 20: 49 ms of
+    // DFS from depth 2; dense 5-vertex 25 ms; a 6-vertex cycle on scale 17 24
+    // ms).  So with the default limit or a larger one the levels go on to it
+    // while a level fits kExtendWords.
+    const bool to_suffix = batched_suffix && !fixed_cap && q->bfs_row_limit >= kBfsRowLimit;
+    while (n > 0 && depth + 1 < q->qv && !(batched_suffix && depth + 2 > q->hplan.cp_start)) {
+        const bool wide = n >= q->bfs_row_limit;
+        if (wide && !(to_suffix && n * (depth + 1) <= kExtendWords)) break;
+        uint64_t want_rows = fixed_cap ? q->frontier_cap_rows
+                             : wide    ? std::min<uint64_t>(n * 4, kExtendWords / (depth + 1))
+                                       : std::min<uint64_t>(std::max<uint64_t>(n * 64, 1u << 20), 1ull << 28);
+        bool done = false;
+        try {
+            Ensure(q, q->ext_offs, n + 1);
+            Ensure(q, q->ext_sel, n);
+            Ensure(q, q->scan_scratch, ScanScratchBytes(n + 1) + 64);
+            for (int attempt = 0;; attempt++) {
+                Ensure(q, q->front[cur ^ 1], want_rows * (depth + 1));
+                SetCounters(q, {{&Counters::rows_out, 0}, {&Counters::flags, 0}}, q->s);
+                const int ke = KBegin(q, CGBDSM_K_EXTEND);
+                LaunchExtend(T, q->front[cur].p, n, depth, q->h_cnt->u_dups == 0, q->ext_offs.p, q->ext_sel.p,
+                             q->scan_scratch.p, q->front[cur ^ 1].p, q->front[cur ^ 1].cap / (depth + 1), q->d_cnt,
+                             q->s);
+                KEnd(q, ke);
+                ReadCounters(q);
+                KAdd(q, CGBDSM_K_EXTEND, 0, n);
+                if (!(q->h_cnt->flags & kFlagFrontier)) {
+                    done = true;
+                    break;
+                }
+                // A wide level that fits after all is written again at its size.
+                want_rows = q->h_cnt->rows_out;
+                if (!wide || attempt || want_rows * (depth + 1) > kExtendWords) break;
+            }
+        } catch (const ApiError& e) {
+            if (e.code != CGBDSM_ERR_OOM || !wide) throw;
+        }
+        if (!done) break;  // keep this level, count it by DFS
         n = q->h_cnt->rows_out;
         cur ^= 1;
         depth++;

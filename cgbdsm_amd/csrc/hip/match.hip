@@ -5,13 +5,14 @@
 //            whose batch lists exist (writeInitialResultsAllBit,
 //            kernels/enumeration.cu:727-809), all tags in one pass: one
 //            wavefront per 64 owners reads the shared first-pair lists once,
-//            spreads their entries over lanes; scan + one atomic per 64
-//            entries reserves rows.
+//            spreads their entries over lanes; rows leave through a buffer in
+//            LDS, one atomic per flush.
 //   KSeed1   depth-1 rows [(ei << tag_shift) | v0] instead, when the product
 //            suffix starts at position 2.
 //   KTag*    counting sort of the seed rows by edge tag.
-//   KExtend  one BFS level, one wavefront per row, 64 candidates per step
-//            (extendBFSAllBit with write_res, kernels/enumeration.cu:811-1155).
+//   KExtend  one BFS level, the rows' candidate lists laid end to end over the
+//            lanes (extendBFSAllBit with write_res,
+//            kernels/enumeration.cu:811-1155).
 //   KDfs     the final count: persistent wavefronts pull rows (of one or
 //            several queries) from a global atomic queue; each runs an
 //            iterative DFS whose per-level survivor stacks live in LDS (64 u32
@@ -32,13 +33,14 @@
 #include "wave.h"
 
 // Resident blocks per CU (= waves per SIMD) of the final DFS, a build-time
-// tuning knob.  Its loops' carried values are scalar (75 to 92 VGPRs, nothing
-// spilled to memory), so registers would allow 6; what decides is the LDS left
-// for the stable-intersection cache and the waves that share the work queue's
-// lines.  Scale-21 four-query batch: 154 ms of DFS at 3, 135 at 4, 131 at 5;
-// scale-20 dense 6-vertex query: 48, 49, 74.
+// tuning knob.  Its loops' carried values are scalar (87 to 92 VGPRs, nothing
+// spilled to memory); what decides is latency hiding against the LDS left for
+// the stable-intersection cache and the waves that share the work queue's
+// lines.  DFS ms per launch at 3 / 4 / 5 blocks: scale-21 four-query batch 152
+// / 133 / 126; scale-20 dense 6-vertex query 29.2 / 23.9 / 21.3; 8-query mix
+// 25.9 / 21.3 / 18.7; a 50 000-edge 5-vertex walk batch 4.26 / 4.07 / 4.35.
 #ifndef CGD_DFS_BLOCKS
-#define CGD_DFS_BLOCKS 4
+#define CGD_DFS_BLOCKS 5
 #endif
 
 namespace cgd {
@@ -155,21 +157,31 @@ __device__ __forceinline__ List Resolve(const Ctx& X, const Tables& T, uint32_t 
 
 __device__ __forceinline__ uint32_t At(const List& L, uint32_t i) { return i < L.bl ? LdG(L.base + i) : LdG(L.app + (i - L.bl)); }
 
-// Candidate c for position d given positions 0..d-1 in `matched` (LDS,
-// uniform): support-mask bit, injective, present in the list of every
-// backward neighbour after the first (whose list supplied c).
-__device__ __forceinline__ bool Accept(const Ctx& X, const Tables& T, uint32_t d, const uint32_t* matched, uint32_t c) {
-    if (!TileBit(X, T, Vs(X, d), c)) return false;
-    for (uint32_t i = 0; i < d; i++)
-        if (matched[i] == c) return false;
-    const uint32_t nbn = Nbn(X, d);
-    for (uint32_t k = 1; k < nbn; k++) {
-        const uint32_t pr = Pair(X, d, k);
-        const List L = Resolve(X, T, pr & 0xFFu, Uniform(matched[pr >> 8]));
-        if (!SortedContains(L.base, L.bl, c) && !(L.al && SortedContains(L.app, L.al, c))) return false;
+// Frontier rows a wavefront has found, kept in its LDS until kRowBuf words are
+// full: one atomic on the row counter and one contiguous store per flush.  (An
+// atomic for every 64 candidates, on one line, took most of the kernels' time.)
+constexpr uint32_t kRowBuf = 1024;
+struct RowBuf {
+    uint32_t* buf;
+    uint32_t words, n;  // words per row, rows held
+    __device__ __forceinline__ uint32_t Room() const { return kRowBuf / words - n; }
+    __device__ __forceinline__ void Flush(uint32_t* __restrict__ rows, uint64_t cap_rows,
+                                          Counters* __restrict__ cnt) {
+        if (!n) return;
+        const uint32_t lane = LaneId();
+        WaveSync();
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(&cnt->rows_out, (unsigned long long)n);
+        base = ReadLane64(base, 0);
+        if (base + n > cap_rows) {
+            if (lane == 0) atomicOr(&cnt->flags, kFlagFrontier);
+        } else {
+            for (uint32_t i = lane; i < n * words; i += kWave) rows[base * words + i] = buf[i];
+        }
+        WaveSync();
+        n = 0;
     }
-    return true;
-}
+};
 
 // Depth-2 seeds of every active edge tag in one pass.  Position 0 -> 1 of
 // the global order is one query direction `idx` for every tag, so the list
@@ -185,6 +197,7 @@ __global__ void __launch_bounds__(kThreads) KSeed(Tables T, EiList EL, uint32_t*
     __shared__ uint32_t s_tag[kMaxQE];
     __shared__ uint32_t s_incl[kWpb][kWave], s_lenm[kWpb][kWave], s_offu[kWpb][kWave];
     __shared__ uint64_t s_m0[kWpb][kWave], s_offm[kWpb][kWave];
+    __shared__ uint32_t s_buf[kWpb][kRowBuf];
     const cgbdsm_plan& p = T.P->p;
     const uint32_t q0 = p.go_vs[0], q1 = p.go_vs[1];
     const uint32_t idx = p.eidx[q0 * kMaxQV + q1];
@@ -207,6 +220,7 @@ __global__ void __launch_bounds__(kThreads) KSeed(Tables T, EiList EL, uint32_t*
     }
     __syncthreads();
     uint32_t* incl_l = s_incl[wv];
+    RowBuf out{s_buf[wv], 2, 0};
     const uint64_t nw = (uint64_t)gridDim.x * kWpb;
     for (uint64_t w = (uint64_t)blockIdx.x * kWpb + wv; w < T.W; w += nw) {
         const uint32_t v = (uint32_t)(w * kWave + lane);
@@ -269,26 +283,22 @@ __global__ void __launch_bounds__(kThreads) KSeed(Tables T, EiList EL, uint32_t*
                     if (((ones1 >> k) & 1ull) || (s_tile1[k][nb >> 6] & bit1)) ok |= 1ull << k;
                 }
             }
-            const uint32_t nr = (uint32_t)__popcll(ok);
-            const uint32_t incl2 = WaveInclusiveScan(nr);
-            const uint32_t tot2 = ReadLane(incl2, kWave - 1);
-            if (!tot2) continue;
-            unsigned long long base = 0;
-            if (lane == 0) base = atomicAdd(&cnt->rows_out, (unsigned long long)tot2);
-            base = ReadLane64(base, 0);
-            if (base + tot2 > cap_rows) {
-                if (lane == 0) atomicOr(&cnt->flags, kFlagFrontier);
-                continue;
-            }
-            uint64_t pos = base + incl2 - nr;
-            for (; ok; ok &= ok - 1, pos++) {
-                const uint32_t k = (uint32_t)__builtin_ctzll(ok);
-                rows[2 * pos] = s_tag[k] | v0;
-                rows[2 * pos + 1] = nb;
+            // One row per lane and round: a candidate's tags in ascending order.
+            for (uint64_t any = __ballot(ok != 0); any; any = __ballot(ok != 0)) {
+                const uint32_t k = (uint32_t)__popcll(any);
+                if (out.Room() < k) out.Flush(rows, cap_rows, cnt);
+                if (ok) {
+                    const uint32_t at = 2 * (out.n + RankBelow(any));
+                    out.buf[at] = s_tag[__builtin_ctzll(ok)] | v0;
+                    out.buf[at + 1] = nb;
+                    ok &= ok - 1;
+                }
+                out.n += k;
             }
         }
         WaveSync();
     }
+    out.Flush(rows, cap_rows, cnt);
 }
 
 // Depth-1 rows [(ei << tag_shift) | v0] for every active edge tag whose
@@ -300,6 +310,8 @@ __global__ void __launch_bounds__(kThreads) KSeed(Tables T, EiList EL, uint32_t*
 __global__ void __launch_bounds__(kThreads) KSeed1(Tables T, EiList EL, uint32_t* __restrict__ rows,
                                                    uint64_t cap_rows, Counters* __restrict__ cnt) {
     __shared__ uint32_t s_tag[kMaxQE];
+    __shared__ uint32_t s_buf[kWpb][kRowBuf];
+    RowBuf out{s_buf[threadIdx.x / kWave], 1, 0};
     const cgbdsm_plan& p = T.P->p;
     const uint32_t q0 = p.go_vs[0], q1 = p.go_vs[1];
     const uint32_t idx = p.eidx[q0 * kMaxQV + q1];
@@ -331,20 +343,17 @@ __global__ void __launch_bounds__(kThreads) KSeed1(Tables T, EiList EL, uint32_t
         uint64_t emit = 0;
         if ((m0 & use_m) && LdMRec(T.m_rec + r).len) emit |= m0 & use_m;
         if ((m0 & use_u) && LdURec(T.u_rec + r).len) emit |= m0 & use_u;
-        const uint32_t nr = (uint32_t)__popcll(emit);
-        const uint32_t incl = WaveInclusiveScan(nr);
-        const uint32_t tot = ReadLane(incl, kWave - 1);
-        if (!tot) continue;
-        unsigned long long base = 0;
-        if (lane == 0) base = atomicAdd(&cnt->rows_out, (unsigned long long)tot);
-        base = ReadLane64(base, 0);
-        if (base + tot > cap_rows) {
-            if (lane == 0) atomicOr(&cnt->flags, kFlagFrontier);
-            continue;
+        for (uint64_t any = __ballot(emit != 0); any; any = __ballot(emit != 0)) {
+            const uint32_t k = (uint32_t)__popcll(any);
+            if (out.Room() < k) out.Flush(rows, cap_rows, cnt);
+            if (emit) {
+                out.buf[out.n + RankBelow(any)] = s_tag[__builtin_ctzll(emit)] | v;
+                emit &= emit - 1;
+            }
+            out.n += k;
         }
-        uint64_t pos = base + incl - nr;
-        for (; emit; emit &= emit - 1, pos++) rows[pos] = s_tag[__builtin_ctzll(emit)] | v;
     }
+    out.Flush(rows, cap_rows, cnt);
 }
 
 // Counting sort of depth-2 rows by edge tag (KSeed emits the tags of one
@@ -393,56 +402,6 @@ __global__ void __launch_bounds__(kThreads) KTagScatter(const uint32_t* __restri
         const uint64_t pos = base[k] + atomicAdd(&h[k], 1u);
         out[W * pos] = w0;
         if (W > 1) out[W * pos + 1] = in[W * r + 1];
-    }
-}
-
-__global__ void __launch_bounds__(kThreads) KExtend(Tables T, const uint32_t* __restrict__ in, uint64_t n_in,
-                                                    uint32_t D, uint32_t* __restrict__ out, uint64_t cap_rows,
-                                                    Counters* __restrict__ cnt) {
-    __shared__ uint32_t s_matched[kWpb][kMaxQV];
-    __shared__ PlanLds s_plan;
-    FillPlanLds(T, &s_plan);
-    Ctx X = MakeCtx(T, &s_plan);
-    const uint32_t wv = threadIdx.x / kWave, lane = LaneId();
-    uint32_t* matched = s_matched[wv];
-    const uint32_t p0 = Pair(X, D, 0);
-    const uint32_t pe = p0 & 0xFFu, pq = p0 >> 8;
-    const uint32_t tag_shift = T.P->tag_shift, v_mask = T.P->v_mask;
-    const uint64_t nw = (uint64_t)gridDim.x * kWpb;
-    for (uint64_t r = (uint64_t)blockIdx.x * kWpb + wv; r < n_in; r += nw) {
-        const uint32_t w0 = Uniform(in[r * D]);
-        const uint32_t ei = w0 >> tag_shift;
-        if (ei != X.ei || r == (uint64_t)blockIdx.x * kWpb + wv) SetTag(X, ei);
-        if (lane < D) matched[lane] = lane == 0 ? (w0 & v_mask) : in[r * D + lane];
-        WaveSync();
-        const List L = Resolve(X, T, pe, Uniform(matched[pq]));
-        const uint32_t total = L.bl + L.al;
-        for (uint32_t off = 0; off < total; off += kWave) {
-            const uint32_t i = off + lane;
-            uint32_t c = 0;
-            bool ok = false;
-            if (i < total) {
-                c = At(L, i);
-                ok = Accept(X, T, D, matched, c);
-            }
-            const uint64_t m = __ballot(ok);
-            const uint32_t k = (uint32_t)__popcll(m);
-            if (!k) continue;
-            unsigned long long base = 0;
-            if (lane == 0) base = atomicAdd(&cnt->rows_out, (unsigned long long)k);
-            base = __shfl(base, 0, kWave);
-            if (base + k > cap_rows) {
-                if (lane == 0) atomicOr(&cnt->flags, kFlagFrontier);
-                continue;
-            }
-            if (ok) {
-                uint32_t* o = out + (base + RankBelow(m)) * (uint64_t)(D + 1);
-                o[0] = w0;
-                for (uint32_t j = 1; j < D; j++) o[j] = matched[j];
-                o[D] = c;
-            }
-        }
-        WaveSync();
     }
 }
 
@@ -516,6 +475,13 @@ struct Hint {
     uint32_t idle, stop;  // waves waiting for work; the launch was asked to stop
 };
 
+// Frontier rows a block has taken and not yet given to its waves, the rows its
+// waves are done with, and the waves still taking rows.
+struct RowRange {
+    unsigned long long next, end, held;
+    uint32_t lock, done, waves;
+};
+
 // Marks a ticket's slot (seq = ticket + 1 with this bit) when no work is left.
 constexpr unsigned long long kSeqDone = 1ull << 63;
 // An idle wave's sleep between looks at its slot: kIdleSleep * 64 cycles,
@@ -564,6 +530,124 @@ __device__ __forceinline__ bool InList(const List& L, uint32_t c, uint32_t& prob
         return LdG(L.app + lo) == c;
     }
     return false;
+}
+
+// List of directed query edge `dir` at data vertex `owner` under edge tag ei
+// (Resolve with a tag of each lane's own).
+__device__ __forceinline__ List ResolveTag(LdsPlan* L, const Tables& T, uint32_t ei, uint32_t dir, uint32_t owner) {
+    List l{nullptr, nullptr, 0, 0};
+    const uint64_t r = (uint64_t)owner * T.ndir + dir;
+    const uint32_t own = L->own[ei];
+    const bool mine = dir == (own & 0xFFu) || dir == own >> 8;
+    const bool app = (L->app[ei][dir >> 6] >> (dir & 63u)) & 1ull;
+    if (!mine) {
+        const MRec m = LdMRec(T.m_rec + r);
+        l.base = T.pool + m.off;
+        l.bl = m.len;
+    }
+    if (mine || app) {
+        const URec u = LdURec(T.u_rec + r);
+        if (mine) {
+            l.base = T.u_vals + u.off;
+            l.bl = u.len;
+        }
+        if (app) {
+            l.app = T.u_vals + u.off;
+            l.al = u.len;
+        }
+    }
+    return l;
+}
+
+__device__ __forceinline__ uint32_t RowVertex(const uint32_t* __restrict__ row, uint32_t i, uint32_t v_mask) {
+    return i ? row[i] : row[0] & v_mask;
+}
+
+// First half of a BFS level: per frontier row, the backward neighbour of
+// position D whose list is scanned (the shortest when every list is a set,
+// else the first, as the reference does) and that list's length.
+__global__ void __launch_bounds__(kThreads) KExtendLens(Tables T, const uint32_t* __restrict__ in, uint64_t n,
+                                                        uint32_t D, uint32_t sets, uint64_t* __restrict__ offs,
+                                                        uint8_t* __restrict__ sel) {
+    __shared__ PlanLds s_plan;
+    FillPlanLds(T, &s_plan);
+    LdsPlan* L = (LdsPlan*)&s_plan;
+    const uint32_t tag_shift = T.P->tag_shift, v_mask = T.P->v_mask;
+    const uint32_t nbn = sets ? (uint32_t)(L->nbn >> (4 * D)) & 15u : 1u;
+    for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += (uint64_t)gridDim.x * blockDim.x) {
+        const uint32_t* row = in + r * D;
+        const uint32_t ei = row[0] >> tag_shift;
+        uint32_t best = 0xFFFFFFFFu, bk = 0;
+        for (uint32_t k = 0; k < nbn; k++) {
+            const uint32_t pr = L->pair[D][k];
+            const List l = ResolveTag(L, T, ei, pr & 0xFFu, RowVertex(row, pr >> 8, v_mask));
+            if (l.bl + l.al < best) {
+                best = l.bl + l.al;
+                bk = k;
+            }
+        }
+        offs[r] = best;
+        sel[r] = (uint8_t)bk;
+    }
+}
+
+// Second half: the rows' scanned lists laid end to end over the lanes (offs
+// scanned), one candidate per lane, whatever row it belongs to; survivors
+// leave through the wave's row buffer.  A wavefront per row left most lanes
+// idle (lists of a few entries), the hubs' rows to one wave each, and took an
+// atomic per 64 candidates: dense 6-vertex query on scale 20, 376k rows to
+// 2.2M: 7.2 -> 0.43 ms.
+__global__ void __launch_bounds__(kThreads) KExtend(Tables T, const uint32_t* __restrict__ in, uint64_t n, uint32_t D,
+                                                    const uint64_t* __restrict__ offs, const uint8_t* __restrict__ sel,
+                                                    uint32_t* __restrict__ out, uint64_t cap_rows,
+                                                    Counters* __restrict__ cnt) {
+    __shared__ PlanLds s_plan;
+    __shared__ uint32_t s_buf[kWpb][kRowBuf];
+    FillPlanLds(T, &s_plan);
+    LdsPlan* L = (LdsPlan*)&s_plan;
+    const uint32_t wv = threadIdx.x / kWave;
+    const uint32_t tag_shift = T.P->tag_shift, v_mask = T.P->v_mask;
+    const uint32_t nbn = (uint32_t)(L->nbn >> (4 * D)) & 15u, qv = (uint32_t)(L->vs >> (4 * D)) & 15u;
+    RowBuf buf{s_buf[wv], D + 1, 0};
+    const uint64_t total = offs[n], nw = (uint64_t)gridDim.x * kWpb;
+    const uint64_t per = ((total + nw - 1) / nw + kWave - 1) & ~(uint64_t)(kWave - 1);
+    const uint64_t lo = ((uint64_t)blockIdx.x * kWpb + wv) * per, hi = lo + per < total ? lo + per : total;
+    uint64_t p0 = lo < hi ? LbFirst(offs, n, lo) : 0;
+    uint32_t probes = 0;
+    for (uint64_t it0 = lo; it0 < hi; it0 += kWave) {
+        const LbItem it = LbLocateFrom(offs, n, p0, it0, hi);
+        if (it0 + kWave <= hi) p0 = ReadLane64(it.p, kWave - 1);
+        const uint32_t* row = in + it.p * D;
+        uint32_t c = 0;
+        bool ok = false;
+        if (it.valid) {
+            const uint32_t ei = row[0] >> tag_shift;
+            const uint32_t k0 = sel[it.p];
+            {
+                const uint32_t pr = L->pair[D][k0];
+                c = At(ResolveTag(L, T, ei, pr & 0xFFu, RowVertex(row, pr >> 8, v_mask)), it.j);
+            }
+            ok = ((L->ones[ei] >> qv) & 1u) ||
+                 ((LdG(T.masks + ((uint64_t)ei * kMaxQV + qv) * T.W + (c >> 6)) >> (c & 63u)) & 1ull);
+            for (uint32_t i = 0; i < D; i++) ok = ok && RowVertex(row, i, v_mask) != c;
+            for (uint32_t k = 0; k < nbn && ok; k++) {
+                if (k == k0) continue;
+                const uint32_t pr = L->pair[D][k];
+                ok = InList(ResolveTag(L, T, ei, pr & 0xFFu, RowVertex(row, pr >> 8, v_mask)), c, probes);
+            }
+        }
+        const uint64_t m = __ballot(ok);
+        const uint32_t k = (uint32_t)__popcll(m);
+        if (!k) continue;
+        if (buf.Room() < k) buf.Flush(out, cap_rows, cnt);
+        if (ok) {
+            uint32_t* o = buf.buf + (buf.n + RankBelow(m)) * (D + 1);
+            for (uint32_t i = 0; i < D; i++) o[i] = row[i];
+            o[D] = c;
+        }
+        buf.n += k;
+    }
+    buf.Flush(out, cap_rows, cnt);
 }
 
 // Candidate c for position d: support-mask bit, distinct from positions
@@ -1222,6 +1306,7 @@ __global__ void __launch_bounds__(kThreads)
     __shared__ WaveStats s_stats[kWpb];
     __shared__ uint32_t s_job[kWpb];
     __shared__ Hint s_hint;
+    __shared__ RowRange s_rows;
     // Dynamic LDS, per wave: survivor stacks of surv_levels levels (64 u32
     // each; every job of the launch has qv - 1 <= surv_levels) and the
     // stable-intersection cache of stab_cap u32.
@@ -1311,9 +1396,36 @@ __global__ void __launch_bounds__(kThreads)
     };
     // Every row is handed out by the cursor: a share fixed by the block index
     // would wait for a block that another launch keeps from running, whose own
-    // blocks may be waiting the same way.  Rows retire from `pending`
-    // together, when the wave finds no more of them.
+    // blocks may be waiting the same way.  A block takes a grab for each of
+    // its waves with one atomic, and its rows retire from `pending` together,
+    // when its last wave finds no more of them.
     uint64_t r_next = 0, r_end = 0, held = 0, ticket = 0;
+    // (fewer rows at a time when there are not two grabs for every wave)
+    grab = (uint32_t)min((uint64_t)grab, max((uint64_t)1, n_rows / (2ull * gridDim.x * kWpb)));
+    auto take_rows = [&]() {
+        unsigned long long a = 0, b = 0;
+        if (lane == 0) {
+            while (atomicCAS(&s_rows.lock, 0u, 1u) != 0u) __builtin_amdgcn_s_sleep(1);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            volatile RowRange* R = &s_rows;
+            if (R->next >= R->end && !R->done) {
+                const unsigned long long r0 = atomicAdd(&cnt->q_rows.v, (unsigned long long)grab * kWpb);
+                R->next = r0;
+                R->end = r0 + grab * kWpb < n_rows ? r0 + grab * kWpb : n_rows;
+                if (r0 >= n_rows) R->done = 1;
+            }
+            if (!R->done) {
+                a = R->next;
+                b = a + grab < R->end ? a + grab : R->end;
+                R->next = b;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            atomicExch(&s_rows.lock, 0u);
+        }
+        r_next = ReadLane64(a, 0);
+        r_end = ReadLane64(b, 0);
+        held += r_end - r_next;
+    };
     bool primary = true, idle = false, stop = false, have_ticket = false, from_row = false;
     uint32_t iter = 0, backoff = 1, waits = 0;
     // Shared words (idle count, flags) and the host flag are read at most
@@ -1322,7 +1434,10 @@ __global__ void __launch_bounds__(kThreads)
     // polling one address would otherwise saturate the memory-side path that
     // agent-scope loads take and stall the waves that work.
     const long long t_born = (long long)Uniform64((unsigned long long)wall_clock64());
-    if (threadIdx.x == 0) s_hint = Hint{t_born, t_born, 0, 0};
+    if (threadIdx.x == 0) {
+        s_hint = Hint{t_born, t_born, 0, 0};
+        s_rows = RowRange{0, 0, 0, 0, 0, (uint32_t)kWpb};
+    }
     __syncthreads();
     volatile Hint* hint = &s_hint;
     long long t_idle0 = 0, idle_sum = 0;
@@ -1381,19 +1496,20 @@ __global__ void __launch_bounds__(kThreads)
     while (!stop) {
         // ---------------- obtain a work item
         uint32_t D0 = 0, ei = 0, lo0 = 0, hi0 = kFull, sel0 = kNoSel;
+        uint64_t changed = 0;  // positions whose vertex differs from the last item's
         bool got = false;
         if (primary) {
             if (r_next >= r_end) {
-                unsigned long long r0 = 0;
-                if (lane == 0) r0 = atomicAdd(&cnt->q_rows.v, (unsigned long long)grab);
-                r0 = ReadLane64(r0, 0);
-                r_next = r0;
-                r_end = r0 + grab < n_rows ? r0 + grab : n_rows;
-                if (r0 >= n_rows) {
+                take_rows();
+                if (r_next >= r_end) {
                     primary = false;
-                    if (held) retire(held);
-                } else {
-                    held += r_end - r0;
+                    unsigned long long all = 0;
+                    if (lane == 0) {
+                        atomicAdd(&s_rows.held, (unsigned long long)held);
+                        if (atomicSub(&s_rows.waves, 1u) == 1u) all = atomicAdd(&s_rows.held, 0ull);
+                    }
+                    all = ReadLane64(all, 0);
+                    if (all) retire(all);
                 }
             }
             if (primary) {
@@ -1418,6 +1534,7 @@ __global__ void __launch_bounds__(kThreads)
                     if (lane == 0) atomicOr(&cnt->flags, kFlagBadRow);
                     continue;
                 }
+                changed = __ballot(lane < D && matched[lane] != mv);
                 if (lane < D) matched[lane] = mv;
                 D0 = D;
                 got = true;
@@ -1454,7 +1571,9 @@ __global__ void __launch_bounds__(kThreads)
                 use_job(tag >> 16);
                 lo0 = Uniform(GetAgent(&it->lo));
                 hi0 = Uniform(GetAgent(&it->hi));
-                if (lane < D0) matched[lane] = GetAgent(&it->v[lane]);
+                const uint32_t mv = lane < D0 ? GetAgent(&it->v[lane]) : 0u;
+                changed = __ballot(lane < D0 && matched[lane] != mv);
+                if (lane < D0) matched[lane] = mv;
                 got = true;
                 from_row = false;
                 have_ticket = false;
@@ -1476,10 +1595,22 @@ __global__ void __launch_bounds__(kThreads)
             }
         }
         // ---------------- DFS from position D0
-        if (ei != X.ei || X.sa == 0xFFu) SetTag(X, ei);
+        // What the last item cached (suffix sizes, the stable intersection)
+        // holds as far as its positions are the same: consecutive rows often
+        // share all but the last.
+        if (ei != X.ei || X.sa == 0xFFu) {
+            SetTag(X, ei);
+            cvalid = 0;
+            sc.state = 0;
+        } else if (changed) {
+            cvalid &= 0xFFFFu;
+            for (uint32_t m = (uint32_t)changed; m; m &= m - 1) {
+                const uint32_t x = (uint32_t)__builtin_ctz(m);
+                cvalid &= ~Uniform(s_plan[wv].dep_mask[x]);
+                if ((sc.deps >> x) & 1u) sc.state = 0;
+            }
+        }
         if (lane == 0) lvl[D0] = DfsLevel{lo0, 0, 0, hi0, sel0};
-        cvalid = 0;
-        sc.state = 0;
         WaveSync();
         unsigned long long count = 0;
         uint32_t d = Uniform(D0);
@@ -1799,10 +1930,12 @@ void LaunchSeed1(const Tables& T, const EiList& L, uint32_t* rows, uint64_t cap_
     KSeed1<<<Grid1(T.W, kWpb, 8192), kThreads, 0, s>>>(T, L, rows, cap_rows, cnt);
 }
 
-void LaunchExtend(const Tables& T, const uint32_t* in, uint64_t n_in, uint32_t depth, uint32_t* out, uint64_t cap_rows,
-                  Counters* cnt, hipStream_t s) {
+void LaunchExtend(const Tables& T, const uint32_t* in, uint64_t n_in, uint32_t depth, bool sets, uint64_t* offs,
+                  uint8_t* sel, void* scan_scratch, uint32_t* out, uint64_t cap_rows, Counters* cnt, hipStream_t s) {
     if (!n_in) return;
-    KExtend<<<Grid1(n_in, kWpb, 65535), kThreads, 0, s>>>(T, in, n_in, depth, out, cap_rows, cnt);
+    KExtendLens<<<Grid1(n_in, kThreads, 2048), kThreads, 0, s>>>(T, in, n_in, depth, sets, offs, sel);
+    ScanU64(offs, offs, n_in, offs + n_in, scan_scratch, s);
+    KExtend<<<Grid1(n_in, kWpb, 2048), kThreads, 0, s>>>(T, in, n_in, depth, offs, sel, out, cap_rows, cnt);
 }
 
 // LDS per final-DFS block (static tables + survivor stacks + cache) at nb

@@ -131,60 +131,6 @@ __device__ __forceinline__ bool Enqueue(uint32_t* queued, uint32_t v, uint32_t u
     return !((atomicOr(&queued[v], 1u << u) >> u) & 1u);
 }
 
-// ---------------------------------------------------------------- load-balanced list walks
-// The items of a pair list are the entries of its pairs' adjacency lists,
-// offs[p] = first item of pair p (exclusive scan of list lengths, offs[np] =
-// total).  Locates item it0 + lane: its pair and position in that list.
-struct LbItem {
-    uint64_t p;
-    uint32_t j;
-    bool valid;
-};
-
-__device__ __forceinline__ LbItem LbLocate(const uint64_t* __restrict__ offs, uint64_t np, uint64_t it0,
-                                           uint64_t total) {
-    const uint32_t lane = LaneId();
-    const uint64_t it = it0 + lane;
-    // p0: the last pair starting at or before it0 (uniform).
-    uint64_t lo = 0, hi = np;
-    while (hi - lo > 1) {
-        const uint64_t mid = (lo + hi) >> 1;
-        if (offs[mid] <= it0) lo = mid;
-        else hi = mid;
-    }
-    const uint64_t p0 = lo;
-    const uint64_t e = p0 + 1 + lane <= np ? offs[p0 + 1 + lane] : ~0ull;
-    uint32_t pos = 0;
-#pragma unroll
-    for (uint32_t step = 32; step >= 1; step >>= 1) {
-        const uint64_t ee = __shfl(e, (int)(pos + step - 1), kWave);
-        if (ee <= it) pos += step;
-    }
-    const uint64_t last = ReadLane64(e, 63);
-    const uint64_t prev = __shfl(e, (int)(pos ? pos - 1 : 0), kWave);
-    LbItem r;
-    r.valid = it < total;
-    if (last <= it) {
-        // Beyond the 64 pairs after p0 (runs of empty lists): search the rest.
-        uint64_t a = p0 + 64, b = np;
-        while (b - a > 1) {
-            const uint64_t mid = (a + b) >> 1;
-            if (offs[mid] <= it) a = mid;
-            else b = mid;
-        }
-        r.p = a;
-        r.j = (uint32_t)(it - offs[a]);
-    } else {
-        r.p = p0 + pos;
-        r.j = (uint32_t)(it - (pos ? prev : offs[p0]));
-    }
-    if (!r.valid) {
-        r.p = 0;
-        r.j = 0;
-    }
-    return r;
-}
-
 // ---------------------------------------------------------------- graph kernels
 // Both orientations of every valid pair of stream ints [start, start + 2 * np)
 // as keys (src << vbits) | dst (invalid pairs: ~0, sorted to the end).

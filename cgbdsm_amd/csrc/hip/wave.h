@@ -121,6 +121,69 @@ __device__ __forceinline__ uint64_t Uniform64(uint64_t v) {
     return ((uint64_t)hi << 32) | lo;
 }
 
+// Load-balanced list walks.  The items of np lists laid end to end, offs[p] =
+// first item of list p (exclusive scan of the lengths, offs[np] = total):
+// which list an item lies in and at which place.
+struct LbItem {
+    uint64_t p;
+    uint32_t j;
+    bool valid;
+};
+
+// The last list starting at or before item it (uniform).
+__device__ __forceinline__ uint64_t LbFirst(const uint64_t* __restrict__ offs, uint64_t np, uint64_t it) {
+    uint64_t lo = 0, hi = np;
+    while (hi - lo > 1) {
+        const uint64_t mid = (lo + hi) >> 1;
+        if (offs[mid] <= it) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Item it0 + lane, given a list p0 that starts at or before it0 (uniform;
+// nearer is faster).  Every lane calls.
+__device__ __forceinline__ LbItem LbLocateFrom(const uint64_t* __restrict__ offs, uint64_t np, uint64_t p0,
+                                               uint64_t it0, uint64_t total) {
+    const uint32_t lane = LaneId();
+    const uint64_t it = it0 + lane;
+    const uint64_t e = p0 + 1 + lane <= np ? offs[p0 + 1 + lane] : ~0ull;
+    uint32_t pos = 0;
+#pragma unroll
+    for (uint32_t step = 32; step >= 1; step >>= 1) {
+        const uint64_t ee = __shfl(e, (int)(pos + step - 1), 64);
+        if (ee <= it) pos += step;
+    }
+    const uint64_t last = ReadLane64(e, 63);
+    const uint64_t prev = __shfl(e, (int)(pos ? pos - 1 : 0), 64);
+    LbItem r;
+    r.valid = it < total;
+    if (last <= it) {
+        // Beyond the 64 lists after p0 (runs of empty lists): search the rest.
+        uint64_t a = p0 + 64, b = np;
+        while (b - a > 1) {
+            const uint64_t mid = (a + b) >> 1;
+            if (offs[mid] <= it) a = mid;
+            else b = mid;
+        }
+        r.p = a;
+        r.j = (uint32_t)(it - offs[a]);
+    } else {
+        r.p = p0 + pos;
+        r.j = (uint32_t)(it - (pos ? prev : offs[p0]));
+    }
+    if (!r.valid) {
+        r.p = 0;
+        r.j = 0;
+    }
+    return r;
+}
+
+__device__ __forceinline__ LbItem LbLocate(const uint64_t* __restrict__ offs, uint64_t np, uint64_t it0,
+                                           uint64_t total) {
+    return LbLocateFrom(offs, np, LbFirst(offs, np, it0), it0, total);
+}
+
 // First index i in [0, n) with a[i] >= v (n if none).
 __device__ __forceinline__ uint32_t LowerBound(const uint32_t* __restrict__ a, uint32_t n, uint32_t v) {
     uint32_t lo = 0, hi = n;

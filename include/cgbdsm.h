@@ -237,7 +237,9 @@ cgbdsm_status cgbdsm_batch_update_global_index(cgbdsm_query* q);
 
 /* Matching knobs (no reference counterpart beyond utils/config.h:22):
  * bfs_row_limit = MIN_NRESULTS_TO_GPU analogue (rows below which a BFS
- * level is expanded before the final DFS); frontier_cap = capacity of the
+ * level is expanded before the final DFS; with the default of 65536 or more,
+ * a query whose product suffix is counted in batches expands its wider levels
+ * too, as far as they fit 64 MiB); frontier_cap = capacity of the
  * frontier buffer in rows (small values force the overflow fallback of
  * graph/graph_gpu.cu:1323-1327); donate_min = pending candidates at which a
  * DFS wavefront donates work to the global stealing queue (0 disables). */

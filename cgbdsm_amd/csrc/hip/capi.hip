@@ -204,9 +204,8 @@ void GrowPool(cgbdsm_query* q, uint64_t min_cap) {
 // M <- M u keys (sorted internal keys, unique), retrying after pool growth.
 void InsertSorted(cgbdsm_query* q, const uint64_t* keys, const unsigned long long* n_segs, uint64_t n_upper) {
     for (int attempt = 0;; attempt++) {
-        SetCounter(q, &Counters::flags, 0);
-        SetCounter(q, &Counters::bytes, 0);
-        SetCounter(q, &Counters::n_long, 0);
+        SetCounters(q, {{&Counters::flags, 0}, {&Counters::bytes, 0}, {&Counters::n_long, 0}, {&Counters::n_huge, 0}},
+                    q->s);
         const int k = KBegin(q, CGBDSM_K_MERGE_INSERT);
         // q->flags (segment discovery's scan) is free again: long-list queue.
         LaunchMergeInsert(MakeTables(q), keys, q->vbits, q->seg_row.p, q->seg_start.p, n_segs, n_upper, q->sc_val.p,
@@ -1100,8 +1099,7 @@ cgbdsm_status cgbdsm_transfer_update_all(cgbdsm_query* q) {
             SetCounter(q, &Counters::n_unique, q->n_del);
             LaunchSegments(q->k_alt.p, Cnt(q, &Counters::n_unique), q->n_del, q->vbits, q->flags.p, q->seg_row.p,
                            q->seg_start.p, Cnt(q, &Counters::n_segs), q->scan_scratch.p, q->s);
-            SetCounter(q, &Counters::bytes, 0);
-            SetCounter(q, &Counters::n_long, 0);
+            SetCounters(q, {{&Counters::bytes, 0}, {&Counters::n_long, 0}, {&Counters::n_huge, 0}}, q->s);
             const int k = KBegin(q, CGBDSM_K_MERGE_REMOVE);
             LaunchMergeRemove(MakeTables(q), q->k_alt.p, q->vbits, q->seg_row.p, q->seg_start.p,
                               Cnt(q, &Counters::n_segs), q->n_del, q->flags.p, q->d_cnt, q->s);

@@ -62,6 +62,7 @@ struct alignas(128) Counters {
     unsigned long long wave_ticks;    // final DFS: summed wave lifetimes (wall-clock ticks)
     unsigned long long idle_ticks;    // final DFS: summed time waves waited for work
     unsigned long long n_long;        // index merges: touched lists left to one wavefront each
+    unsigned long long n_huge;        // and to a whole block each (follows n_long)
     // Words polled by many wavefronts at once, one 128-byte L2 line each.
     struct alignas(128) Line {
         unsigned long long v;

@@ -15,7 +15,8 @@
 //   it fits its capacity: every store lands at or above the reads still to
 //   come; else into a fresh pool block, the untouched head copied after);
 //   remove: one forward compaction pass (stores land at or below the reads).
-// Longer lists are queued (a ballot append) for one wavefront each:
+// Longer lists are queued (a ballot append) for one wavefront each, those of
+// kHugeLen entries or more for a whole block:
 //   1. dedup: each lane binary-searches its delta value in the old list; the
 //      survivors B' are compacted with a ballot and their final positions
 //      (rank in old list + rank in B') are recorded.
@@ -34,7 +35,6 @@ namespace cgd {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kWavesPerBlock = kThreads / kWave;
 
 __global__ void KDecode(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n, uint32_t ushift,
                         uint32_t umask, uint32_t ndir, uint32_t vbits) {
@@ -146,24 +146,57 @@ constexpr uint32_t kShortWork = 48;
 // flight per lane; a hub's list is thousands of chunks long).
 constexpr uint32_t kMergeUnroll = 4;
 
-// Appends segment s (lanes with push set) to the queue of long lists.
-__device__ __forceinline__ void PushLong(bool push, uint64_t s, uint32_t* __restrict__ long_segs,
-                                         unsigned long long* __restrict__ n_long) {
+// Touched lists of at least this many entries are merged by a whole block: one
+// wavefront moves 256 entries per dependent round trip, so a hub's list alone
+// set the length of the launch.  Scale-22 graph, 1 M-edge batches: adjacency
+// and index removals 3.2 -> 0.6 ms a batch, insertions 3.0 -> 0.6 ms.
+constexpr uint32_t kHugeLen = 4096;
+constexpr int kTeam = 512, kTeamWaves = kTeam / kWave;
+constexpr uint32_t kHugeUnroll = 8;  // entries a lane loads per step of a huge list
+
+// Appends segment s (lanes with push set) to a queue of n counted entries:
+// from the front of `segs` upwards (dir 1) or from its end downwards (dir -1).
+__device__ __forceinline__ void PushSeg(bool push, uint64_t s, uint32_t* __restrict__ segs, int dir,
+                                        unsigned long long* __restrict__ n) {
     const uint64_t m = __ballot(push);
+    if (!m) return;
     unsigned long long base = 0;
-    if (m && LaneId() == 0) base = atomicAdd(n_long, (unsigned long long)__popcll(m));
+    if (LaneId() == 0) base = atomicAdd(n, (unsigned long long)__popcll(m));
     base = ReadLane64(base, 0);
-    if (push) long_segs[base + RankBelow(m)] = (uint32_t)s;
+    if (push) segs[dir * (int64_t)(base + RankBelow(m))] = (uint32_t)s;
 }
 
+// A block's byte and list counts into the counters: one atomic each, and none
+// where nothing was counted (an atomic per wave of a full grid on one line
+// took 0.2 ms whether or not there was a list to merge).
 __device__ __forceinline__ void FoldCounters(unsigned long long bytes, unsigned long long touched,
                                              Counters* __restrict__ cnt) {
+    __shared__ unsigned long long s_bytes, s_touched;
+    if (threadIdx.x == 0) s_bytes = s_touched = 0;
+    __syncthreads();
     bytes = ReadLane64(WaveInclusiveScan(bytes), 63);
     touched = ReadLane64(WaveInclusiveScan(touched), 63);
-    if (LaneId() == 0) {
-        if (bytes) atomicAdd(&cnt->bytes, bytes);
-        if (touched) atomicAdd(&cnt->rows_touched, touched);
+    if (LaneId() == 0 && bytes) atomicAdd(&s_bytes, bytes);
+    if (LaneId() == 0 && touched) atomicAdd(&s_touched, touched);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (s_bytes) atomicAdd(&cnt->bytes, s_bytes);
+        if (s_touched) atomicAdd(&cnt->rows_touched, s_touched);
     }
+}
+
+// Exclusive prefix of the counts c[0..n) (n <= 64, in LDS) in place, for the
+// whole block; returns their sum.
+__device__ __forceinline__ uint32_t BlockPrefix64(uint32_t* c, uint32_t n, uint32_t* total) {
+    __syncthreads();
+    if (threadIdx.x < (uint32_t)kWave) {
+        const uint32_t v = threadIdx.x < n ? c[threadIdx.x] : 0u;
+        const uint32_t incl = WaveInclusiveScan(v);
+        if (threadIdx.x < n) c[threadIdx.x] = incl - v;
+        if (threadIdx.x == (uint32_t)kWave - 1) *total = incl;
+    }
+    __syncthreads();
+    return *total;
 }
 
 // One lane per short touched list: M[row] <- M[row] u B (B sorted, unique).
@@ -172,7 +205,7 @@ __global__ void __launch_bounds__(kThreads) KMergeInsertShort(Tables T, const ui
                                                               const uint64_t* __restrict__ seg_start,
                                                               const unsigned long long* __restrict__ n_segs_dev,
                                                               uint64_t pool_cap, uint32_t* __restrict__ long_segs,
-                                                              Counters* __restrict__ cnt) {
+                                                              uint64_t n_upper, Counters* __restrict__ cnt) {
     const uint64_t n_segs = *n_segs_dev;
     const uint64_t vmask = (1ull << vbits) - 1ull;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -190,8 +223,9 @@ __global__ void __launch_bounds__(kThreads) KMergeInsertShort(Tables T, const ui
             nb = (uint32_t)(seg_start[s + 1] - bs);
             rec = T.m_rec[row];
         }
-        const bool is_long = valid && rec.len + nb > kShortWork;
-        PushLong(is_long, s, long_segs, &cnt->n_long);
+        const bool is_long = valid && rec.len + nb > kShortWork, is_huge = is_long && rec.len >= kHugeLen;
+        PushSeg(is_long && !is_huge, s, long_segs, 1, &cnt->n_long);
+        PushSeg(is_huge, s, long_segs + n_upper - 1, -1, &cnt->n_huge);
         if (!valid || is_long) continue;
         const uint64_t* B = keys + bs;
         uint32_t* A = T.pool + rec.off;
@@ -247,7 +281,7 @@ __global__ void __launch_bounds__(kThreads) KMergeRemoveShort(Tables T, const ui
                                                               uint32_t vbits, const uint32_t* __restrict__ seg_row,
                                                               const uint64_t* __restrict__ seg_start,
                                                               const unsigned long long* __restrict__ n_segs_dev,
-                                                              uint32_t* __restrict__ long_segs,
+                                                              uint32_t* __restrict__ long_segs, uint64_t n_upper,
                                                               Counters* __restrict__ cnt) {
     const uint64_t n_segs = *n_segs_dev;
     const uint64_t vmask = (1ull << vbits) - 1ull;
@@ -266,8 +300,9 @@ __global__ void __launch_bounds__(kThreads) KMergeRemoveShort(Tables T, const ui
             na = rec.len;
             off = rec.off;
         }
-        const bool is_long = valid && na + nd > kShortWork;
-        PushLong(is_long, s, long_segs, &cnt->n_long);
+        const bool is_long = valid && na + nd > kShortWork, is_huge = is_long && na >= kHugeLen;
+        PushSeg(is_long && !is_huge, s, long_segs, 1, &cnt->n_long);
+        PushSeg(is_huge, s, long_segs + n_upper - 1, -1, &cnt->n_huge);
         if (!valid || is_long) continue;
         bytes += 8ull * nd;
         if (na == 0) continue;
@@ -290,20 +325,116 @@ __global__ void __launch_bounds__(kThreads) KMergeRemoveShort(Tables T, const ui
     FoldCounters(bytes, touched, cnt);
 }
 
-// One wavefront per long touched list: M[row] <- M[row] u B (B sorted, unique).
-__global__ void __launch_bounds__(kThreads) KMergeInsert(Tables T, const uint64_t* __restrict__ keys, uint32_t vbits,
-                                                         const uint32_t* __restrict__ seg_row,
-                                                         const uint64_t* __restrict__ seg_start,
-                                                         const uint32_t* __restrict__ long_segs,
-                                                         const unsigned long long* __restrict__ n_long_dev,
-                                                         uint32_t* __restrict__ sc_val, uint32_t* __restrict__ sc_pos,
-                                                         uint64_t pool_cap, Counters* __restrict__ cnt) {
+// The whole block on one huge list: M[row] <- M[row] u B.  Same steps as the
+// wavefront's below, kHugeUnroll entries per lane and step.
+__device__ __forceinline__ void InsertHuge(const Tables& T, const uint64_t* __restrict__ keys, uint64_t vmask,
+                                           uint32_t row, uint64_t bs, uint32_t nb, uint32_t* __restrict__ sc_val,
+                                           uint32_t* __restrict__ sc_pos, uint64_t pool_cap,
+                                           Counters* __restrict__ cnt, unsigned long long& bytes,
+                                           unsigned long long& touched) {
+    __shared__ uint32_t s_c[kTeamWaves], s_total;
+    __shared__ unsigned long long s_off;
+    const uint32_t t = threadIdx.x, w = t / kWave;
+    MRec rec = T.m_rec[row];
+    uint32_t* A = T.pool + rec.off;
+    const uint32_t na = rec.len;
+    const uint32_t astep = (na + kWave - 1) / kWave;
+    const uint32_t apiv = Pivots(A, na, astep);
+    uint32_t nbp = 0;
+    for (uint32_t k = 0; k < nb; k += kTeam) {
+        const uint32_t j = k + t;
+        const bool valid = j < nb;
+        const uint32_t b = valid ? (uint32_t)(keys[bs + j] & vmask) : 0u;
+        const uint32_t p = LowerBoundPiv(A, na, astep, apiv, b);
+        const bool keep = valid && !(p < na && A[p] == b);
+        const uint64_t m = __ballot(keep);
+        if (LaneId() == 0) s_c[w] = (uint32_t)__popcll(m);
+        const uint32_t all = BlockPrefix64(s_c, kTeamWaves, &s_total);
+        const uint32_t r = nbp + s_c[w] + RankBelow(m);
+        if (keep) {
+            sc_val[bs + r] = b;
+            sc_pos[bs + r] = p + r;
+        }
+        nbp += all;
+        __syncthreads();
+    }
+    if (t == 0) bytes += 8ull * nb;
+    if (nbp == 0) return;
+    const uint32_t newlen = na + nbp;
+    const uint32_t* Bv = sc_val + bs;
+    const uint32_t* Bp = sc_pos + bs;
+    const bool in_lanes = nbp < (uint32_t)kWave;
+    const uint32_t bstep = (nbp + kWave - 1) / kWave;
+    const uint32_t held = Pivots(Bv, nbp, bstep);
+    uint32_t* C = A;
+    const bool grow = newlen > rec.cap;
+    if (grow) {
+        const uint32_t ncap = CapFor(newlen);
+        if (t == 0) s_off = atomicAdd(&cnt->pool_top, (unsigned long long)ncap);
+        __syncthreads();
+        const uint64_t off = s_off;
+        if (off + ncap > pool_cap) {
+            if (t == 0) atomicOr(&cnt->flags, kFlagPool);
+            __syncthreads();  // s_off is read before the next list's write
+            return;
+        }
+        C = T.pool + off;
+        rec.off = off;
+        rec.cap = ncap;
+    }
+    // Back to front over [i0, na); into a fresh extent, over all of it.  All
+    // entries of a step are loaded before any is stored (see KMergeInsert).
+    const uint32_t i0 = grow ? 0u : Bp[0];
+    for (uint32_t hi = na; hi > i0;) {
+        const uint32_t lo = hi > i0 + kTeam * kHugeUnroll ? hi - kTeam * kHugeUnroll : i0;
+        uint32_t a[kHugeUnroll], r[kHugeUnroll];
+#pragma unroll
+        for (uint32_t u = 0; u < kHugeUnroll; u++) {
+            const uint32_t d = u * kTeam + t;  // distance below hi - 1
+            a[u] = d < hi - lo ? A[hi - 1 - d] : 0u;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kHugeUnroll; u++)
+            r[u] = in_lanes ? RankInLanes(held, a[u]) : LowerBoundPiv(Bv, nbp, bstep, held, a[u]);
+        __syncthreads();
+#pragma unroll
+        for (uint32_t u = 0; u < kHugeUnroll; u++) {
+            const uint32_t d = u * kTeam + t;
+            if (d < hi - lo) C[hi - 1 - d + r[u]] = a[u];
+        }
+        __syncthreads();
+        hi = lo;
+    }
+    for (uint32_t j = t; j < nbp; j += kTeam) C[Bp[j]] = Bv[j];
+    if (t == 0) {
+        bytes += 8ull * (na - i0) + 4ull * nbp;
+        touched++;
+        rec.len = newlen;
+        T.m_rec[row] = rec;
+    }
+    __syncthreads();
+}
+
+// Long touched lists: M[row] <- M[row] u B (B sorted, unique).  The block's
+// huge lists first, then one wavefront per other long list.
+__global__ void __launch_bounds__(kTeam) KMergeInsert(Tables T, const uint64_t* __restrict__ keys, uint32_t vbits,
+                                                      const uint32_t* __restrict__ seg_row,
+                                                      const uint64_t* __restrict__ seg_start,
+                                                      const uint32_t* __restrict__ long_segs, uint64_t n_upper,
+                                                      uint32_t* __restrict__ sc_val, uint32_t* __restrict__ sc_pos,
+                                                      uint64_t pool_cap, Counters* __restrict__ cnt) {
     const uint32_t lane = LaneId();
-    const uint64_t nw = (uint64_t)gridDim.x * kWavesPerBlock;
-    const uint64_t n_long = *n_long_dev;
+    const uint64_t nw = (uint64_t)gridDim.x * kTeamWaves;
+    const uint64_t n_long = cnt->n_long, n_huge = cnt->n_huge;
     const uint64_t vmask = (1ull << vbits) - 1ull;
     unsigned long long bytes = 0, touched = 0;
-    for (uint64_t t = (uint64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave; t < n_long; t += nw) {
+    for (uint64_t t = blockIdx.x; t < n_huge; t += gridDim.x) {
+        const uint64_t s = long_segs[n_upper - 1 - t];
+        InsertHuge(T, keys, vmask, seg_row[s], seg_start[s], (uint32_t)(seg_start[s + 1] - seg_start[s]), sc_val,
+                   sc_pos, pool_cap, cnt, bytes, touched);
+    }
+    unsigned long long wbytes = 0, wtouched = 0;
+    for (uint64_t t = (uint64_t)blockIdx.x * kTeamWaves + threadIdx.x / kWave; t < n_long; t += nw) {
         const uint64_t s = long_segs[t];
         const uint32_t row = seg_row[s];
         const uint64_t bs = seg_start[s];
@@ -331,7 +462,7 @@ __global__ void __launch_bounds__(kThreads) KMergeInsert(Tables T, const uint64_
             }
             nbp += (uint32_t)__popcll(m);
         }
-        bytes += 8ull * nb;
+        wbytes += 8ull * nb;
         if (nbp == 0) continue;
         WaveSync();
         const uint32_t newlen = na + nbp;
@@ -368,7 +499,7 @@ __global__ void __launch_bounds__(kThreads) KMergeInsert(Tables T, const uint64_
                     if (i < na) C[i + r] = a[u];
                 }
             }
-            bytes += 4ull * na + 4ull * na;
+            wbytes += 4ull * na + 4ull * na;
             if (lane == 0) {
                 rec.off = off;
                 rec.cap = ncap;
@@ -402,38 +533,97 @@ __global__ void __launch_bounds__(kThreads) KMergeInsert(Tables T, const uint64_
                 WaveSync();
                 hi = lo;
             }
-            bytes += 8ull * (na - i0);
+            wbytes += 8ull * (na - i0);
         }
         for (uint32_t k = 0; k < nbp; k += kWave) {
             const uint32_t j = k + lane;
             if (j < nbp) C[Bp[j]] = Bv[j];
         }
-        bytes += 4ull * nbp;
-        touched++;
+        wbytes += 4ull * nbp;
+        wtouched++;
         if (lane == 0) {
             rec.len = newlen;
             T.m_rec[row] = rec;
         }
     }
     if (lane == 0) {
-        atomicAdd(&cnt->bytes, bytes);
-        atomicAdd(&cnt->rows_touched, touched);
+        bytes += wbytes;
+        touched += wtouched;
     }
+    FoldCounters(bytes, touched, cnt);
 }
 
-// One wavefront per long touched list: M[row] <- M[row] \ D (D sorted).
-__global__ void __launch_bounds__(kThreads) KMergeRemove(Tables T, const uint64_t* __restrict__ keys, uint32_t vbits,
-                                                         const uint32_t* __restrict__ seg_row,
-                                                         const uint64_t* __restrict__ seg_start,
-                                                         const uint32_t* __restrict__ long_segs,
-                                                         const unsigned long long* __restrict__ n_long_dev,
-                                                         Counters* __restrict__ cnt) {
+// The whole block on one huge list: M[row] <- M[row] \ D, compacted forwards
+// (see KMergeRemove), kHugeUnroll entries per lane and step.
+__device__ __forceinline__ void RemoveHuge(const Tables& T, const uint64_t* __restrict__ D, uint64_t vmask,
+                                           uint32_t row, uint32_t nd, unsigned long long& bytes,
+                                           unsigned long long& touched) {
+    static_assert(kTeamWaves * kHugeUnroll <= 64, "one wavefront scans a step's counts");
+    __shared__ uint32_t s_c[kTeamWaves * kHugeUnroll], s_total;
+    const uint32_t t = threadIdx.x, wv = t / kWave, lane = LaneId();
+    const uint32_t na = T.m_rec[row].len;
+    uint32_t* A = T.pool + T.m_rec[row].off;
+    const uint32_t i0 = WaveLowerBound(A, na, (uint32_t)(D[0] & vmask));
+    uint32_t w = i0;
+    const bool in_lanes = nd < (uint32_t)kWave;
+    const uint32_t dstep = (nd + kWave - 1) / kWave;
+    const uint32_t held = lane * dstep < nd ? (uint32_t)(D[lane * dstep] & vmask) : ~0u;
+    for (uint32_t k = i0; k < na; k += kTeam * kHugeUnroll) {
+        uint32_t a[kHugeUnroll];
+        uint64_t m[kHugeUnroll];
+#pragma unroll
+        for (uint32_t u = 0; u < kHugeUnroll; u++) {
+            const uint32_t i = k + u * kTeam + t;
+            a[u] = i < na ? A[i] : 0u;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kHugeUnroll; u++) {
+            bool del;
+            if (in_lanes) {
+                const uint32_t p = RankInLanes(held, a[u]);
+                const uint32_t at = __shfl(held, (int)(p < (uint32_t)kWave ? p : kWave - 1), kWave);
+                del = p < nd && at == a[u];
+            } else {
+                const uint32_t p = LowerBoundKeysPiv(D, nd, dstep, held, a[u], vmask);
+                del = p < nd && (uint32_t)(D[p] & vmask) == a[u];
+            }
+            m[u] = __ballot(k + u * kTeam + t < na && !del);
+            if (lane == 0) s_c[u * kTeamWaves + wv] = (uint32_t)__popcll(m[u]);
+        }
+        const uint32_t all = BlockPrefix64(s_c, kTeamWaves * kHugeUnroll, &s_total);
+#pragma unroll
+        for (uint32_t u = 0; u < kHugeUnroll; u++)
+            if ((m[u] >> lane) & 1ull) A[w + s_c[u * kTeamWaves + wv] + RankBelow(m[u])] = a[u];
+        w += all;
+        __syncthreads();
+    }
+    if (t == 0) {
+        bytes += 8ull * nd + 4ull * (na - i0) + 4ull * (w - i0);
+        if (w != na) touched++;
+        T.m_rec[row].len = w;
+    }
+    __syncthreads();
+}
+
+// Long touched lists: M[row] <- M[row] \ D (D sorted).  The block's huge lists
+// first, then one wavefront per other long list.
+__global__ void __launch_bounds__(kTeam) KMergeRemove(Tables T, const uint64_t* __restrict__ keys, uint32_t vbits,
+                                                      const uint32_t* __restrict__ seg_row,
+                                                      const uint64_t* __restrict__ seg_start,
+                                                      const uint32_t* __restrict__ long_segs, uint64_t n_upper,
+                                                      Counters* __restrict__ cnt) {
     const uint32_t lane = LaneId();
-    const uint64_t nw = (uint64_t)gridDim.x * kWavesPerBlock;
-    const uint64_t n_long = *n_long_dev;
+    const uint64_t nw = (uint64_t)gridDim.x * kTeamWaves;
+    const uint64_t n_long = cnt->n_long, n_huge = cnt->n_huge;
     const uint64_t vmask = (1ull << vbits) - 1ull;
     unsigned long long bytes = 0, touched = 0;
-    for (uint64_t t = (uint64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave; t < n_long; t += nw) {
+    for (uint64_t t = blockIdx.x; t < n_huge; t += gridDim.x) {
+        const uint64_t s = long_segs[n_upper - 1 - t];
+        RemoveHuge(T, keys + seg_start[s], vmask, seg_row[s], (uint32_t)(seg_start[s + 1] - seg_start[s]), bytes,
+                   touched);
+    }
+    unsigned long long wbytes = 0, wtouched = 0;
+    for (uint64_t t = (uint64_t)blockIdx.x * kTeamWaves + threadIdx.x / kWave; t < n_long; t += nw) {
         const uint64_t s = long_segs[t];
         const uint32_t row = seg_row[s];
         const uint64_t bs = seg_start[s];
@@ -441,7 +631,7 @@ __global__ void __launch_bounds__(kThreads) KMergeRemove(Tables T, const uint64_
         const uint64_t* D = keys + bs;
         const uint32_t na = T.m_rec[row].len;
         uint32_t* A = T.pool + T.m_rec[row].off;
-        bytes += 8ull * nd;
+        wbytes += 8ull * nd;
         if (na == 0) continue;
         const uint32_t i0 = WaveLowerBound(A, na, (uint32_t)(D[0] & vmask));
         uint32_t w = i0;
@@ -485,14 +675,15 @@ __global__ void __launch_bounds__(kThreads) KMergeRemove(Tables T, const uint64_
             }
             WaveSync();
         }
-        bytes += 4ull * (na - i0) + 4ull * (w - i0);
-        if (w != na) touched++;
+        wbytes += 4ull * (na - i0) + 4ull * (w - i0);
+        if (w != na) wtouched++;
         if (lane == 0) T.m_rec[row].len = w;
     }
     if (lane == 0) {
-        atomicAdd(&cnt->bytes, bytes);
-        atomicAdd(&cnt->rows_touched, touched);
+        bytes += wbytes;
+        touched += wtouched;
     }
+    FoldCounters(bytes, touched, cnt);
 }
 
 __global__ void KClearU(URec* __restrict__ u_rec, const uint32_t* __restrict__ u_rows,
@@ -619,15 +810,16 @@ void LaunchSegments(const uint64_t* keys, const unsigned long long* n_dev, uint6
     KWriteSegs<<<GridFor(n_upper), 256, 0, s>>>(keys, n_dev, vbits, flags, n_segs_dev, seg_row, seg_start);
 }
 
-// Both merges expect cnt->n_long zeroed; long_segs holds n_upper entries.
+// Both merges expect cnt->n_long and n_huge zeroed; long_segs holds n_upper
+// entries (long lists from its front, huge ones from its end).
 void LaunchMergeInsert(const Tables& T, const uint64_t* keys, uint32_t vbits, const uint32_t* seg_row,
                        const uint64_t* seg_start, const unsigned long long* n_segs, uint64_t n_upper, uint32_t* sc_val,
                        uint32_t* sc_pos, uint32_t* long_segs, uint64_t pool_cap, Counters* cnt, hipStream_t s) {
     if (!n_upper) return;
     KMergeInsertShort<<<GridFor(n_upper, kThreads, 8192), kThreads, 0, s>>>(T, keys, vbits, seg_row, seg_start,
-                                                                           n_segs, pool_cap, long_segs, cnt);
-    KMergeInsert<<<GridFor(n_upper, kWavesPerBlock, 2048), kThreads, 0, s>>>(
-        T, keys, vbits, seg_row, seg_start, long_segs, &cnt->n_long, sc_val, sc_pos, pool_cap, cnt);
+                                                                           n_segs, pool_cap, long_segs, n_upper, cnt);
+    KMergeInsert<<<GridFor(n_upper, kTeamWaves, 1024), kTeam, 0, s>>>(T, keys, vbits, seg_row, seg_start, long_segs,
+                                                                     n_upper, sc_val, sc_pos, pool_cap, cnt);
 }
 
 void LaunchMergeRemove(const Tables& T, const uint64_t* keys, uint32_t vbits, const uint32_t* seg_row,
@@ -635,9 +827,9 @@ void LaunchMergeRemove(const Tables& T, const uint64_t* keys, uint32_t vbits, co
                        uint32_t* long_segs, Counters* cnt, hipStream_t s) {
     if (!n_upper) return;
     KMergeRemoveShort<<<GridFor(n_upper, kThreads, 8192), kThreads, 0, s>>>(T, keys, vbits, seg_row, seg_start,
-                                                                           n_segs, long_segs, cnt);
-    KMergeRemove<<<GridFor(n_upper, kWavesPerBlock, 2048), kThreads, 0, s>>>(T, keys, vbits, seg_row, seg_start,
-                                                                            long_segs, &cnt->n_long, cnt);
+                                                                           n_segs, long_segs, n_upper, cnt);
+    KMergeRemove<<<GridFor(n_upper, kTeamWaves, 1024), kTeam, 0, s>>>(T, keys, vbits, seg_row, seg_start, long_segs,
+                                                                     n_upper, cnt);
 }
 
 void LaunchClearU(URec* u_rec, const uint32_t* u_rows, const unsigned long long* n_dev, uint64_t n_upper,

@@ -23,8 +23,9 @@ void LaunchSegments(const uint64_t* keys, const unsigned long long* n_dev, uint6
                     uint32_t* flags, uint32_t* seg_row, uint64_t* seg_start, unsigned long long* n_segs_dev,
                     void* scan_scratch, hipStream_t s);
 // Merges of sorted keys into (insert) or out of (remove) the lists they
-// touch: one lane per short list, one wavefront per long one (queued in
-// long_segs, n_upper entries; cnt->n_long must be zero at the launch).
+// touch: one lane per short list, one wavefront per long one, a block per huge
+// one (queued in long_segs, n_upper entries; cnt->n_long and n_huge must be
+// zero at the launch).
 void LaunchMergeInsert(const Tables& T, const uint64_t* keys, uint32_t vbits, const uint32_t* seg_row,
                        const uint64_t* seg_start, const unsigned long long* n_segs, uint64_t n_upper, uint32_t* sc_val,
                        uint32_t* sc_pos, uint32_t* long_segs, uint64_t pool_cap, Counters* cnt, hipStream_t s);

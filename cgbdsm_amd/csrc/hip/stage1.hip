@@ -1053,7 +1053,7 @@ void GraphRemove(cgbdsm_graph* g, const uint64_t* keys, uint64_t nk) {
     FillU64((uint64_t*)&g->d_cnt->n_unique, nk, 1, g->s);
     LaunchSegments(keys, &g->d_cnt->n_unique, nk, g->vbits, g->flags.p, g->seg_row.p, g->seg_start.p, n_s, g->scan.p,
                    g->s);
-    FillU64((uint64_t*)&g->d_cnt->n_long, 0, 1, g->s);
+    FillU64((uint64_t*)&g->d_cnt->n_long, 0, 2, g->s);  // and n_huge
     LaunchMergeRemove(GraphTables(g), keys, g->vbits, g->seg_row.p, g->seg_start.p, n_s, nk, g->flags.p, g->d_cnt,
                       g->s);
 }
@@ -1068,7 +1068,7 @@ void GraphMerge(cgbdsm_graph* g, const uint64_t* keys, uint64_t nk) {
                    g->s);
     for (int attempt = 0;; attempt++) {
         FillU64((uint64_t*)&g->d_cnt->flags, 0, 1, g->s);
-        FillU64((uint64_t*)&g->d_cnt->n_long, 0, 1, g->s);
+        FillU64((uint64_t*)&g->d_cnt->n_long, 0, 2, g->s);  // and n_huge
         LaunchMergeInsert(GraphTables(g), keys, g->vbits, g->seg_row.p, g->seg_start.p, n_s, nk, g->sc_val.p,
                           g->sc_pos.p, g->flags.p, g->pool.cap, g->d_cnt, g->s);
         GReadCounters(g);

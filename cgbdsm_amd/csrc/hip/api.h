@@ -119,7 +119,7 @@ struct cgbdsm_query {
     std::deque<Resident> fifo;
     // final-DFS job table (one entry per query of a launch)
     DBuf<DfsJob> d_jobs;
-    DBuf<DfsOut> dfs_out;
+    DBuf<unsigned long long> dfs_out;  // block records of a launch (DfsOut)
     DBuf<unsigned long long> d_rowbase;
     std::vector<DfsJob> h_jobs;
     std::vector<unsigned long long> h_rowbase;

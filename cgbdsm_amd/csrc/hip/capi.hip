@@ -403,8 +403,10 @@ void RunDfsJobs(cgbdsm_query* q, uint32_t* tuples, uint64_t tup_cap) {
     q->st.last_dfs_lds_cache =
         q->dfs_cache_cap && q->dfs_cache_cap < sh.stab_cap ? q->dfs_cache_cap & ~63u : sh.stab_cap;
     const uint32_t grid = DfsGrid(sh, n, q->ctx->num_cus, q->dfs_bpc);
-    Ensure(q, q->dfs_out, grid);
-    LaunchDfs(q->d_jobs.p, (uint32_t)q->h_jobs.size(), q->d_rowbase.p, n, q->d_cnt, q->dfs_out.p,
+    Ensure(q, q->dfs_out, grid * kDfsOutWords);
+    const DfsOut outs{q->dfs_out.p, q->dfs_out.p + (size_t)grid * kDfsStats,
+                      (uint32_t*)(q->dfs_out.p + (size_t)grid * (kDfsStats + kDfsWaves * kMaxQE))};
+    LaunchDfs(q->d_jobs.p, (uint32_t)q->h_jobs.size(), q->d_rowbase.p, n, q->d_cnt, outs,
               MakeSteal(q, tuples == nullptr), tuples, tup_cap, sh, grid, q->dfs_grab, levels,
               q->st.last_dfs_lds_cache, batched, q->s);
     KEnd(q, k);

@@ -86,14 +86,15 @@ struct DfsJob {
 // per query its waves ended with (job[w], ~0: none), the counts per edge.
 constexpr int kDfsWaves = 4, kDfsStats = 8;
 struct DfsOut {
-    unsigned long long stat[kDfsStats];
-    uint32_t job[kDfsWaves];
-    unsigned long long pe[kDfsWaves][kMaxQE];
+    unsigned long long *stat, *pe;
+    uint32_t* job;
 };
 // LDS plan of a final-DFS launch (see DfsLdsShapeT in match.hip): survivor
 // stacks of surv_levels levels, a stable-intersection cache of stab_cap u32 per
 // wave.  batched: every job has kJobBatched.
 struct DfsShape {
+constexpr size_t kDfsOutWords = kDfsStats + kDfsWaves * kMaxQE + kDfsWaves / 2;  // u64 per block
+
     uint32_t blocks_per_cu, dyn_bytes, stab_cap;
 };
 DfsShape DfsLdsShape(uint32_t surv_levels, bool tuples, bool batched);
@@ -104,7 +105,7 @@ uint32_t DfsGrid(const DfsShape& sh, uint64_t n_rows, uint32_t num_cus, uint32_t
 // one record per block.  surv_levels >= qv - 1 of every job (survivor stacks in
 // LDS); stab_cap <= sh.stab_cap.
 void LaunchDfs(const DfsJob* jobs, uint32_t njobs, const unsigned long long* row_base, uint64_t n_rows, Counters* cnt,
-               DfsOut* outs, const StealQueue& Q, uint32_t* tuples, uint64_t tup_cap, const DfsShape& sh, uint32_t grid,
+               const DfsOut& outs, const StealQueue& Q, uint32_t* tuples, uint64_t tup_cap, const DfsShape& sh, uint32_t grid,
                uint32_t grab, uint32_t surv_levels, uint32_t stab_cap, bool batched, hipStream_t s);
 
 void LaunchCountDups(const uint64_t* k, uint64_t n, Counters* cnt, hipStream_t s);

@@ -431,6 +431,17 @@ __device__ __forceinline__ unsigned long long SatMul(unsigned long long a, unsig
     return __builtin_mul_overflow(a, b, &r) ? kCountSat : r;
 }
 
+// Saturating sum over the 64 lanes, in lane 63 (a DPP scan).
+__device__ __forceinline__ unsigned long long WaveSatScan(unsigned long long sum) {
+    sum = SatAdd(sum, DppMove64<kDppShr1>(sum));
+    sum = SatAdd(sum, DppMove64<kDppShr2>(sum));
+    sum = SatAdd(sum, DppMove64<kDppShr4>(sum));
+    sum = SatAdd(sum, DppMove64<kDppShr8>(sum));
+    sum = SatAdd(sum, DppMove64<kDppBcast15, 0xa>(sum));
+    sum = SatAdd(sum, DppMove64<kDppBcast31, 0xc>(sum));
+    return sum;
+}
+
 constexpr uint32_t kFull = 0xFFFFFFFFu;
 constexpr uint32_t kNoSel = 0xFFu;
 constexpr uint32_t kNoSkip = 0xFFu;
@@ -1259,15 +1270,7 @@ __device__ __forceinline__ unsigned long long BatchSuffix(const Ctx& X, const Ta
         const long long val = (long long)raw - (long long)hits;
         prod = val > 0 ? SatMul(prod, (unsigned long long)val) : 0ull;
     }
-    // Saturating sum over the lanes (a DPP scan; lane 63 holds the total).
-    unsigned long long sum = prod;
-    sum = SatAdd(sum, DppMove64<kDppShr1>(sum));
-    sum = SatAdd(sum, DppMove64<kDppShr2>(sum));
-    sum = SatAdd(sum, DppMove64<kDppShr4>(sum));
-    sum = SatAdd(sum, DppMove64<kDppShr8>(sum));
-    sum = SatAdd(sum, DppMove64<kDppBcast15, 0xa>(sum));
-    sum = SatAdd(sum, DppMove64<kDppBcast31, 0xc>(sum));
-    return ReadLane64(sum, kWave - 1);
+    return ReadLane64(WaveSatScan(prod), kWave - 1);
 }
 
 // Final DFS.  Work items are frontier rows (taken `grab` at a time from a
@@ -1289,7 +1292,7 @@ __global__ void __launch_bounds__(kThreads)
     __attribute__((amdgpu_waves_per_eu(CGD_DFS_BLOCKS))) KDfs(const DfsJob* __restrict__ jobs, uint32_t njobs,
                                                               const unsigned long long* __restrict__ row_base,
                                                               uint32_t grab, Counters* __restrict__ cnt,
-                                                              DfsOut* __restrict__ outs, StealQueue Q,
+                                                              DfsOut outs, StealQueue Q,
                                                               uint32_t* __restrict__ tuples, uint64_t tup_cap,
                                                               uint32_t surv_levels, uint32_t stab_cap) {
     constexpr bool kTuples = kMode == kDfsTuples, kLean = kMode == kDfsBatched;
@@ -1817,53 +1820,59 @@ __global__ void __launch_bounds__(kThreads)
     __syncthreads();
     // The block's record: statistics summed over its waves; per-edge counts
     // under the first wave of each query, the other waves' slots marked empty.
-    DfsOut* o = outs + blockIdx.x;
-    const uint32_t t = threadIdx.x;
+    // Records of one kind lie side by side (DfsOut), for KDfsFold to read.
+    const uint32_t t = threadIdx.x, nb = gridDim.x, bi = blockIdx.x;
     if (t < (uint32_t)kDfsStats) {
         unsigned long long v = 0;
         for (uint32_t w = 0; w < (uint32_t)kWpb; w++) v += ((const unsigned long long*)&s_stats[w])[t];
-        o->stat[t] = v;
+        outs.stat[t * nb + bi] = v;
     }
     for (uint32_t w = 0; w < (uint32_t)kWpb; w++) {
         bool first = s_job[w] != 0xFFFFFFFFu;
         for (uint32_t v = 0; v < w; v++) first = first && s_job[v] != s_job[w];
-        if (t == 0) o->job[w] = first ? s_job[w] : 0xFFFFFFFFu;
+        if (t == 0) outs.job[w * nb + bi] = first ? s_job[w] : 0xFFFFFFFFu;
         if (first && t < (uint32_t)kMaxQE) {
             unsigned long long v = s_pe[w][t];
             for (uint32_t u = w + 1; u < (uint32_t)kWpb; u++)
                 if (s_job[u] == s_job[w]) v = SatAdd(v, s_pe[u][t]);
-            o->pe[w][t] = v;
+            outs.pe[((uint64_t)w * kMaxQE + t) * nb + bi] = v;
         }
     }
 }
 
-// Adds the block records of a final-DFS launch to the counters: block j sums
-// the per-edge counts of query j, block 0 also the launch's statistics.
-__global__ void __launch_bounds__(kThreads) KDfsFold(const DfsJob* __restrict__ jobs, const DfsOut* __restrict__ outs,
-                                                     uint32_t n, Counters* __restrict__ cnt) {
+// Adds the n block records of a final-DFS launch to the counters: block j sums
+// the per-edge counts of query j (a wavefront per 64 records and edge), block 0
+// also the launch's statistics.
+constexpr int kFoldThreads = 1024;
+__global__ void __launch_bounds__(kFoldThreads) KDfsFold(const DfsJob* __restrict__ jobs, DfsOut outs, uint32_t n,
+                                                         Counters* __restrict__ cnt) {
     __shared__ unsigned long long s_sum[kMaxQE], s_stat[kDfsStats];
     __shared__ uint32_t s_wide;
-    const uint32_t t = threadIdx.x, j = blockIdx.x;
+    const uint32_t t = threadIdx.x, j = blockIdx.x, lane = LaneId();
     if (t < (uint32_t)kMaxQE) s_sum[t] = 0;
     if (t < (uint32_t)kDfsStats) s_stat[t] = 0;
     if (t == 0) s_wide = 0;
     __syncthreads();
     Counters* jc = jobs[j].cnt;
-    const uint32_t qe = jobs[j].T.qe;
-    for (uint32_t i = t; i < n * kWpb; i += kThreads) {
-        const DfsOut* o = outs + i / kWpb;
-        const uint32_t w = i % kWpb;
-        if (o->job[w] != j) continue;
+    const uint32_t qe = jobs[j].T.qe, chunks = (n + kWave - 1) / kWave;
+    for (uint32_t i = t / kWave; i < chunks * kWpb; i += kFoldThreads / kWave) {
+        const uint32_t w = i / chunks, b = (i % chunks) * kWave + lane;
+        const bool mine = b < n && outs.job[w * n + b] == j;
+        if (!__ballot(mine)) continue;
         for (uint32_t e = 0; e < qe; e++) {
-            const unsigned long long v = o->pe[w][e];
-            if (!v) continue;
-            const unsigned long long old = atomicAdd(&s_sum[e], v);
-            if (v == kCountSat || old + v < old) s_wide = 1;
+            const unsigned long long v = WaveSatScan(mine ? outs.pe[((uint64_t)w * kMaxQE + e) * n + b] : 0ull);
+            if (lane == kWave - 1 && v) {
+                const unsigned long long old = atomicAdd(&s_sum[e], v);
+                if (v == kCountSat || old + v < old) s_wide = 1;
+            }
         }
     }
     if (j == 0)
-        for (uint32_t i = t; i < n * kDfsStats; i += kThreads)
-            atomicAdd(&s_stat[i % kDfsStats], outs[i / kDfsStats].stat[i % kDfsStats]);
+        for (uint32_t i = t / kWave; i < chunks * kDfsStats; i += kFoldThreads / kWave) {
+            const uint32_t k = i / chunks, b = (i % chunks) * kWave + lane;
+            const unsigned long long v = WaveInclusiveScan(b < n ? outs.stat[k * n + b] : 0ull);
+            if (lane == kWave - 1) atomicAdd(&s_stat[k], v);
+        }
     __syncthreads();
     if (t < qe) {
         const unsigned long long a = jc->per_edge[t], v = s_sum[t];
@@ -2000,7 +2009,7 @@ uint32_t DfsGrid(const DfsShape& sh, uint64_t n_rows, uint32_t num_cus, uint32_t
 }
 
 void LaunchDfs(const DfsJob* jobs, uint32_t njobs, const unsigned long long* row_base, uint64_t n_rows, Counters* cnt,
-               DfsOut* outs, const StealQueue& Q, uint32_t* tuples, uint64_t tup_cap, const DfsShape& sh, uint32_t grid,
+               const DfsOut& outs, const StealQueue& Q, uint32_t* tuples, uint64_t tup_cap, const DfsShape& sh, uint32_t grid,
                uint32_t grab, uint32_t surv_levels, uint32_t stab_cap, bool batched, hipStream_t s) {
     if (!n_rows || !njobs) return;
     grab = grab < 1 ? 1 : grab;
@@ -2013,7 +2022,7 @@ void LaunchDfs(const DfsJob* jobs, uint32_t njobs, const unsigned long long* row
     else
         KDfs<kDfsGeneral><<<grid, kThreads, sh.dyn_bytes, s>>>(jobs, njobs, row_base, grab, cnt, outs, Q, nullptr, 0,
                                                                surv_levels, stab_cap);
-    KDfsFold<<<njobs, kThreads, 0, s>>>(jobs, outs, grid, cnt);
+    KDfsFold<<<njobs, kFoldThreads, 0, s>>>(jobs, outs, grid, cnt);
 }
 
 }  // namespace cgd

@@ -61,6 +61,7 @@ struct cgbdsm_query {
     DBuf<uint32_t> front[2];
     DBuf<uint64_t> ext_offs;  // BFS level: first candidate of each row
     DBuf<uint8_t> ext_sel;    // and its scanned backward neighbour
+    DBuf<uint64_t> exp_offs, exp_keys;  // index export: row offsets, a chunk of keys
     DBuf<unsigned long long> tag_hist;  // 2 * kMaxQE counters of the seed grouping
     uint64_t n_ins = 0, n_del = 0, n_upd = 0, u_rows_upper = 0;
     uint8_t edge_ok[kMaxQE] = {};

@@ -812,6 +812,8 @@ cgbdsm_status cgbdsm_query_destroy(cgbdsm_query* q) {
         Release(q, q->dfs_out);
         Release(q, q->ext_offs);
         Release(q, q->ext_sel);
+        Release(q, q->exp_offs);
+        Release(q, q->exp_keys);
         Release(q, q->d_rowbase);
         Release(q, q->tag_hist);
         for (auto& r : q->fifo) {
@@ -1600,41 +1602,42 @@ cgbdsm_status cgbdsm_kernel_times(cgbdsm_query* q, cgbdsm_ktime* out, int reset)
     });
 }
 
+static constexpr uint64_t kExportKeys = 4ull << 20, kExportKeep = 32ull << 20;
+
 cgbdsm_status cgbdsm_index_export(cgbdsm_query* q, int which, uint64_t* out, uint64_t cap, uint64_t* n_out) {
     return Guard([&] {
         if (!q) Throw(CGBDSM_ERR_INVALID, "null query");
         if (which == 0 && q->layout == CGBDSM_LAYOUT_GPMA && q->pma.stale) PmaExtract(q);
         const uint64_t nrows = (uint64_t)q->dv * q->ndir;
-        uint64_t* lens = (uint64_t*)DevAlloc(q->ctx, (nrows + 1) * 8);
-        void* scr = DevAlloc(q->ctx, ScanScratchBytes(nrows + 1) + 64);
-        uint64_t* tot = (uint64_t*)DevAlloc(q->ctx, 8);
-        uint64_t total = 0;
-        std::vector<uint64_t> h;
+        // The keys come in ascending order from the device, kExportKeys at a
+        // time: no sort on the host.  Scratch of up to kExportKeep bytes each
+        // stays with the query for the next call.
+        auto trim = [&] {
+            if (q->exp_offs.cap * 8 > kExportKeep) Release(q, q->exp_offs);
+            if (q->exp_keys.cap * 8 > kExportKeep) Release(q, q->exp_keys);
+        };
         try {
-            LaunchRowLens(MakeTables(q), nrows, which, lens, q->s);
-            ScanU64(lens, lens, nrows, tot, scr, q->s);
-            CGD_HIP(hipMemcpyAsync(&total, tot, 8, hipMemcpyDeviceToHost, q->s));
+            Ensure(q, q->exp_offs, nrows + 1);
+            Ensure(q, q->scan_scratch, ScanScratchBytes(nrows + 1) + 64);
+            uint64_t total = 0;
+            LaunchRowLens(MakeTables(q), nrows, which, q->exp_offs.p, q->s);
+            ScanU64(q->exp_offs.p, q->exp_offs.p, nrows, q->exp_offs.p + nrows, q->scan_scratch.p, q->s);
+            CGD_HIP(hipMemcpyAsync(&total, q->exp_offs.p + nrows, 8, hipMemcpyDeviceToHost, q->s));
             CGD_HIP(hipStreamSynchronize(q->s));
-            if (total) {
-                uint64_t* d = (uint64_t*)DevAlloc(q->ctx, total * 8);
-                LaunchExport(MakeTables(q), nrows, which, lens, q->ushift, d, q->s);
-                h.resize(total);
-                CGD_HIP(hipMemcpyAsync(h.data(), d, total * 8, hipMemcpyDeviceToHost, q->s));
+            if (n_out) *n_out = total;
+            const uint64_t n = out ? std::min(cap, total) : 0;
+            if (n) Ensure(q, q->exp_keys, std::min(n, kExportKeys));
+            for (uint64_t lo = 0; lo < n; lo += kExportKeys) {
+                const uint64_t hi = std::min(n, lo + kExportKeys);
+                LaunchExport(MakeTables(q), nrows, which, q->exp_offs.p, q->ushift, lo, hi, q->exp_keys.p, q->s);
+                CGD_HIP(hipMemcpyAsync(out + lo, q->exp_keys.p, (hi - lo) * 8, hipMemcpyDeviceToHost, q->s));
                 CGD_HIP(hipStreamSynchronize(q->s));
-                DevFree(q->ctx, d, total * 8);
             }
         } catch (...) {
-            DevFree(q->ctx, lens, (nrows + 1) * 8);
-            DevFree(q->ctx, scr, ScanScratchBytes(nrows + 1) + 64);
-            DevFree(q->ctx, tot, 8);
+            trim();
             throw;
         }
-        DevFree(q->ctx, lens, (nrows + 1) * 8);
-        DevFree(q->ctx, scr, ScanScratchBytes(nrows + 1) + 64);
-        DevFree(q->ctx, tot, 8);
-        std::sort(h.begin(), h.end());
-        if (n_out) *n_out = total;
-        if (out) memcpy(out, h.data(), std::min(cap, total) * 8);
+        trim();
     });
 }
 
@@ -1645,8 +1648,8 @@ cgbdsm_status cgbdsm_index_export_static(cgbdsm_query* q, int which, uint64_t* o
         // Refreshing stale GPMA flat lists must not grow the list pool.
         if (which == 0 && q->layout == CGBDSM_LAYOUT_GPMA && q->pma.stale) PmaExtract(q, false);
         const uint64_t nrows = (uint64_t)q->dv * q->ndir;
-        // Scratch layout (u64 words): row lengths then offsets [nrows + 1],
-        // the scan total, the scan's tile sums, then the exported keys.
+        // Scratch layout (u64 words): row lengths then offsets, the scan total
+        // after them [nrows + 1], the scan's tile sums, then the exported keys.
         const uint64_t w_total = nrows + 1;
         const uint64_t w_scan = w_total + 1;
         const uint64_t scan_words = (ScanScratchBytes(nrows + 1) + 64 + 7) / 8;
@@ -1655,7 +1658,7 @@ cgbdsm_status cgbdsm_index_export_static(cgbdsm_query* q, int which, uint64_t* o
             Throw(CGBDSM_ERR_LIMIT, "index has " + std::to_string(nrows) + " rows; the static export holds at most " +
                                         std::to_string(kStaticScratchWords * 8) + " bytes of scratch");
         uint64_t* lens = base;
-        uint64_t* tot = base + w_total;
+        uint64_t* tot = base + nrows;
         LaunchRowLens(MakeTables(q), nrows, which, lens, q->s);
         ScanU64(lens, lens, nrows, tot, base + w_scan, q->s);
         uint64_t total = 0;
@@ -1671,10 +1674,9 @@ cgbdsm_status cgbdsm_index_export_static(cgbdsm_query* q, int which, uint64_t* o
             Throw(CGBDSM_ERR_INVALID, "out holds " + std::to_string(cap) + " keys, the index has " +
                                           std::to_string(total) + " (*n_out is set)");
         if (total) {
-            LaunchExport(MakeTables(q), nrows, which, lens, q->ushift, base + w_keys, q->s);
+            LaunchExport(MakeTables(q), nrows, which, lens, q->ushift, 0, total, base + w_keys, q->s);
             CGD_HIP(hipMemcpyAsync(out, base + w_keys, total * 8, hipMemcpyDeviceToHost, q->s));
             CGD_HIP(hipStreamSynchronize(q->s));
-            std::sort(out, out + total);
         }
     });
 }

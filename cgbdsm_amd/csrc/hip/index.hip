@@ -745,29 +745,32 @@ __global__ void KInitValues(Tables T, const uint64_t* __restrict__ keys, const u
     }
 }
 
-// Export helpers: M/U as (row, v) pairs in boundary key form, row order.
-__global__ void KExportM(Tables T, const uint64_t* __restrict__ row_off, uint64_t nrows, uint32_t ushift,
-                         uint64_t* __restrict__ out) {
-    for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < nrows; r += (uint64_t)gridDim.x * blockDim.x) {
-        const MRec rec = T.m_rec[r];
-        const uint64_t e = r % T.ndir, u = r / T.ndir;
-        for (uint32_t j = 0; j < rec.len; j++)
-            out[row_off[r] + j] = (e << ushift) | (u << 32) | T.pool[rec.off + j];
+// Export of M (which 0) or U in ascending boundary keys: row i of the export
+// is direction i / dv of owner i % dv, so the rows laid end to end are sorted.
+__global__ void KRowLens(Tables T, uint64_t nrows, int which, uint64_t* __restrict__ lens) {
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nrows; i += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t r = (i % T.dv) * T.ndir + i / T.dv;
+        lens[i] = which ? T.u_rec[r].len : T.m_rec[r].len;
     }
 }
 
-__global__ void KRowLens(Tables T, uint64_t nrows, int which, uint64_t* __restrict__ lens) {
-    for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < nrows; r += (uint64_t)gridDim.x * blockDim.x)
-        lens[r] = which ? T.u_rec[r].len : T.m_rec[r].len;
-}
-
-__global__ void KExportU(Tables T, const uint64_t* __restrict__ row_off, uint64_t nrows, uint32_t ushift,
-                         uint64_t* __restrict__ out) {
-    for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < nrows; r += (uint64_t)gridDim.x * blockDim.x) {
-        const URec rec = T.u_rec[r];
-        const uint64_t e = r % T.ndir, u = r / T.ndir;
-        for (uint32_t j = 0; j < rec.len; j++)
-            out[row_off[r] + j] = (e << ushift) | (u << 32) | T.u_vals[rec.off + j];
+// Entries [lo, hi) of the export (offs = scanned row lengths, offs[nrows] =
+// all), one per lane: a lane per row left the hubs' rows to one lane each.
+__global__ void __launch_bounds__(kThreads) KExport(Tables T, const uint64_t* __restrict__ offs, uint64_t nrows,
+                                                    int which, uint32_t ushift, uint64_t lo, uint64_t hi,
+                                                    uint64_t* __restrict__ out) {
+    const uint64_t nw = (uint64_t)gridDim.x * (kThreads / kWave);
+    const uint64_t per = ((hi - lo + nw - 1) / nw + kWave - 1) & ~(uint64_t)(kWave - 1);
+    const uint64_t a = lo + ((uint64_t)blockIdx.x * (kThreads / kWave) + threadIdx.x / kWave) * per;
+    const uint64_t b = a + per < hi ? a + per : hi;
+    uint64_t p0 = a < b ? LbFirst(offs, nrows, a) : 0;
+    for (uint64_t it0 = a; it0 < b; it0 += kWave) {
+        const LbItem it = LbLocateFrom(offs, nrows, p0, it0, b);
+        if (it0 + kWave <= b) p0 = ReadLane64(it.p, kWave - 1);
+        if (!it.valid) continue;
+        const uint64_t e = it.p / T.dv, u = it.p % T.dv, r = u * T.ndir + e;
+        const uint32_t v = which ? T.u_vals[T.u_rec[r].off + it.j] : T.pool[T.m_rec[r].off + it.j];
+        out[it0 - lo + LaneId()] = (e << ushift) | (u << 32) | v;
     }
 }
 
@@ -864,13 +867,10 @@ void LaunchRowLens(const Tables& T, uint64_t nrows, int which, uint64_t* lens, h
     KRowLens<<<GridFor(nrows), 256, 0, s>>>(T, nrows, which, lens);
 }
 
-void LaunchExport(const Tables& T, uint64_t nrows, int which, const uint64_t* row_off, uint32_t ushift, uint64_t* out,
-                  hipStream_t s) {
-    if (!nrows) return;
-    if (which)
-        KExportU<<<GridFor(nrows), 256, 0, s>>>(T, row_off, nrows, ushift, out);
-    else
-        KExportM<<<GridFor(nrows), 256, 0, s>>>(T, row_off, nrows, ushift, out);
+void LaunchExport(const Tables& T, uint64_t nrows, int which, const uint64_t* offs, uint32_t ushift, uint64_t lo,
+                  uint64_t hi, uint64_t* out, hipStream_t s) {
+    if (hi <= lo) return;
+    KExport<<<GridFor(hi - lo, 4 * kThreads, 2048), kThreads, 0, s>>>(T, offs, nrows, which, ushift, lo, hi, out);
 }
 
 // Adjacent equal keys of a sorted key array into cnt->u_dups (0 means the

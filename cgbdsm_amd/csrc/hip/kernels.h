@@ -42,9 +42,11 @@ void LaunchInitCaps(const uint64_t* seg_start, const unsigned long long* n_segs,
 void LaunchInitLayout(const Tables& T, const uint64_t* keys, const unsigned long long* n_dev, uint64_t n_upper,
                       uint32_t vbits, const uint32_t* head_pos, const uint32_t* seg_row, const uint64_t* seg_start,
                       const unsigned long long* n_segs, const uint64_t* offs, Counters* cnt, hipStream_t s);
+// Export of M (which 0) or U in ascending boundary keys: row lengths, then
+// (offs = their exclusive scan, offs[nrows] = the total) entries [lo, hi).
 void LaunchRowLens(const Tables& T, uint64_t nrows, int which, uint64_t* lens, hipStream_t s);
-void LaunchExport(const Tables& T, uint64_t nrows, int which, const uint64_t* row_off, uint32_t ushift, uint64_t* out,
-                  hipStream_t s);
+void LaunchExport(const Tables& T, uint64_t nrows, int which, const uint64_t* offs, uint32_t ushift, uint64_t lo,
+                  uint64_t hi, uint64_t* out, hipStream_t s);
 
 // masks.hip
 void LaunchMaskClear(uint64_t* masks, uint64_t ei_words, const EiList& L, hipStream_t s);
@@ -81,20 +83,22 @@ struct DfsJob {
     uint32_t D;
     uint32_t opts;  // kJob* bits
 };
-// What one block of a final-DFS launch counted: its statistics (scanned,
-// probes, steps, step lanes, batched steps, donated, wave and idle ticks) and,
-// per query its waves ended with (job[w], ~0: none), the counts per edge.
+// What the n blocks of a final-DFS launch counted: per block its statistics
+// (stat[k * n + block]: scanned, probes, steps, step lanes, batched steps,
+// donated, wave and idle ticks) and, per query its waves ended with
+// (job[w * n + block], ~0: none), the counts per edge
+// (pe[(w * kMaxQE + e) * n + block]).
 constexpr int kDfsWaves = 4, kDfsStats = 8;
 struct DfsOut {
     unsigned long long *stat, *pe;
     uint32_t* job;
 };
+constexpr size_t kDfsOutWords = kDfsStats + kDfsWaves * kMaxQE + kDfsWaves / 2;  // u64 per block
+
 // LDS plan of a final-DFS launch (see DfsLdsShapeT in match.hip): survivor
 // stacks of surv_levels levels, a stable-intersection cache of stab_cap u32 per
 // wave.  batched: every job has kJobBatched.
 struct DfsShape {
-constexpr size_t kDfsOutWords = kDfsStats + kDfsWaves * kMaxQE + kDfsWaves / 2;  // u64 per block
-
     uint32_t blocks_per_cu, dyn_bytes, stab_cap;
 };
 DfsShape DfsLdsShape(uint32_t surv_levels, bool tuples, bool batched);
@@ -102,7 +106,7 @@ DfsShape DfsLdsShape(uint32_t surv_levels, bool tuples, bool batched);
 uint32_t DfsGrid(const DfsShape& sh, uint64_t n_rows, uint32_t num_cus, uint32_t blocks_per_cu);
 // Final DFS over the rows of njobs queries (row_base[j] = first global row of
 // job j, row_base[njobs] = all rows); `cnt` holds the shared work queue, outs
-// one record per block.  surv_levels >= qv - 1 of every job (survivor stacks in
+// room for one record per block.  surv_levels >= qv - 1 of every job (survivor stacks in
 // LDS); stab_cap <= sh.stab_cap.
 void LaunchDfs(const DfsJob* jobs, uint32_t njobs, const unsigned long long* row_base, uint64_t n_rows, Counters* cnt,
                const DfsOut& outs, const StealQueue& Q, uint32_t* tuples, uint64_t tup_cap, const DfsShape& sh, uint32_t grid,

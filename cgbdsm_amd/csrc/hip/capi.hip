@@ -1172,7 +1172,7 @@ cgbdsm_status cgbdsm_build_local_index(cgbdsm_query* q) {
                 const uint32_t ei = L.ei[k];
                 if (q->plan.rebuild_v[ei][q->plan.io_vs[ei][d]]) D.ei[D.n++] = (uint8_t)ei;
             }
-            LaunchMaskDepth(T, d, D, q->d_cnt, q->s);
+            LaunchMaskDepth(T, d, D, q->profile ? q->d_cnt : nullptr, q->s);
             tiles += D.n;
         }
         KEnd(q, kt);

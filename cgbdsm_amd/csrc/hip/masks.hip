@@ -47,9 +47,10 @@ __global__ void KMaskSeed(Tables T, const uint32_t* __restrict__ u_rows, const u
     }
 }
 
-// Algorithmic bytes counted into cnt->bytes: 4 per list entry read and 4 per
-// (backward neighbour, vertex) list size read; the tile write is added by
-// the host (ceil(dv/8) per rebuilt tile).
+// With cnt (profiling), the algorithmic bytes go to cnt->bytes: 4 per list
+// entry read and 4 per (backward neighbour, vertex) list size read; the tile
+// write is added by the host (ceil(dv/8) per rebuilt tile).  (Counted always,
+// an atomic per wavefront on one line took 0.1 ms of each launch.)
 __global__ void __launch_bounds__(256) KMaskDepth(Tables T, uint32_t d, EiList L, Counters* __restrict__ cnt) {
     const uint32_t ei = L.ei[blockIdx.y];
     const cgbdsm_plan& p = T.P->p;
@@ -87,6 +88,7 @@ __global__ void __launch_bounds__(256) KMaskDepth(Tables T, uint32_t d, EiList L
         const uint64_t word = __ballot(ok);
         if (lane == 0) out[w] = word;
     }
+    if (!cnt) return;
     const unsigned long long tot = ReadLane64(WaveInclusiveScan(reads), 63);
     if (lane == 0 && tot) atomicAdd(&cnt->bytes, 4ull * tot);
 }

@@ -53,6 +53,7 @@
 namespace cgd {
 
 constexpr uint32_t kCodeNone = 15;
+constexpr uint32_t kCheckUnroll = 4;
 constexpr uint32_t kSmallDeg = 48;  // pairs with longer lists are checked a wavefront each
 
 // Per-query constant tables, passed by value.
@@ -116,19 +117,41 @@ __device__ __forceinline__ void DeadSet(uint32_t* dead, uint32_t v, uint32_t ui,
     if (bits) atomicOr(&dead[i >> 1], bits << sh);
 }
 
-// Per-lane slots on a shared counter for `cnt` items (all lanes call).
-__device__ __forceinline__ uint64_t WaveReserve(uint32_t cnt, unsigned long long* counter) {
+// Per-thread slots on a shared counter for `cnt` items, with one atomic for
+// the whole block (every thread calls, in loops that all its waves run the same
+// number of times).  The work lists' counters share one line, whose atomics
+// serialize at about 8 ns: one per wavefront and query vertex took most of the
+// time of the kernels that fill the lists.
+__device__ __forceinline__ uint64_t BlockReserve(uint32_t cnt, unsigned long long* counter) {
+    __shared__ uint32_t s_sum[kWpb];
+    __shared__ unsigned long long s_base;
+    const uint32_t w = threadIdx.x / kWave;
     const uint32_t incl = WaveInclusiveScan(cnt);
-    const uint32_t total = ReadLane(incl, 63);
-    unsigned long long base = 0;
-    if (total && LaneId() == 63) base = atomicAdd(counter, (unsigned long long)total);
-    base = ReadLane64(base, 63);
-    return base + incl - cnt;
+    if (LaneId() == kWave - 1) s_sum[w] = incl;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t sum = 0;
+        for (int i = 0; i < kWpb; i++) sum += s_sum[i];
+        s_base = sum ? atomicAdd(counter, (unsigned long long)sum) : 0ull;
+    }
+    __syncthreads();
+    uint64_t at = s_base + incl - cnt;
+    for (uint32_t i = 0; i < w; i++) at += s_sum[i];
+    __syncthreads();
+    return at;
 }
 
-// Marks (v, u) queued; true for the lane that queued it first.
-__device__ __forceinline__ bool Enqueue(uint32_t* queued, uint32_t v, uint32_t u) {
-    return !((atomicOr(&queued[v], 1u << u) >> u) & 1u);
+// Appends the pairs (v, u), u in the bits of `want`, to a work list.
+__device__ __forceinline__ void PutPairs(uint32_t v, uint32_t want, uint32_t* __restrict__ out,
+                                         unsigned long long* __restrict__ n_out) {
+    uint64_t at = BlockReserve((uint32_t)__popc(want), n_out);
+    for (; want; want &= want - 1) out[at++] = (v << 4) | (uint32_t)(__ffs(want) - 1);
+}
+
+// Marks the pairs (v, u), u in the bits of `cand`, queued; returns those that
+// were not queued before.
+__device__ __forceinline__ uint32_t EnqueueAll(uint32_t* queued, uint32_t v, uint32_t cand) {
+    return cand ? cand & ~atomicOr(&queued[v], cand) : 0u;
 }
 
 // ---------------------------------------------------------------- graph kernels
@@ -216,13 +239,7 @@ __global__ void KS1ListPairs(const uint32_t* __restrict__ vstate, uint32_t n, QT
             const uint32_t s = vstate[v];
             bits = lit_only ? Lit(s) : (Code(s) == kCodeNone ? 0u : Q.by_code[Code(s)]);
         }
-        const uint64_t at = WaveReserve((uint32_t)__popc(bits), n_out);
-        uint32_t k = 0;
-        while (bits) {
-            const uint32_t u = __ffs(bits) - 1;
-            bits &= bits - 1;
-            out[at + k++] = ((uint32_t)v << 4) | u;
-        }
+        PutPairs((uint32_t)v, bits, out, n_out);
     }
 }
 
@@ -269,6 +286,31 @@ __device__ bool HallHolds(uint32_t S, const uint32_t (*lists)[kMaxQV], const uin
     return __ballot(!ok) == 0;
 }
 
+// One or more lit supporters of query neighbour u of ui were found (n of them,
+// n <= 64).  open: neighbours of ui that still need one -- or, sharing their
+// label with other neighbours, as many candidates as their label group has
+// members (then one is always free); cnt: 4-bit counts of the latter so far.
+// A pair passes the check once nothing is open, whatever else its list holds.
+__device__ __forceinline__ void Supported(const QTab& Q, uint32_t ui, uint32_t u, uint32_t n, uint32_t& open,
+                                          uint64_t& cnt) {
+    if ((Q.grp[ui] >> u) & 1u) {
+        const uint32_t had = (uint32_t)(cnt >> (4 * u)) & 15u, now = had + n < 15u ? had + n : 15u;
+        cnt += (uint64_t)(now - had) << (4 * u);
+        if (now < (uint32_t)((Q.gneed[ui] >> (4 * u)) & 15u)) return;
+    }
+    open &= ~(1u << u);
+}
+
+// The open neighbours without any supporter (the dead mask of a failing pair).
+__device__ __forceinline__ uint32_t Unsupported(uint32_t open, uint64_t cnt) {
+    uint32_t none = 0;
+    for (; open; open &= open - 1) {
+        const uint32_t u = __ffs(open) - 1;
+        if (!((cnt >> (4 * u)) & 15u)) none |= 1u << u;
+    }
+    return none;
+}
+
 // Exact check of list pairs, one lane per pair with a short adjacency list.
 // Failing pairs go to `died` with their dead mask (query neighbours without
 // a lit supporter); pairs with long lists, or whose distinct-representative
@@ -294,40 +336,26 @@ __global__ void __launch_bounds__(kThreads) KS1Check(GView G, QTab Q, SView S, c
                 tobig = true;
             } else {
                 const uint32_t* A = G.pool + r.off;
-                const uint32_t need = Q.nbr[ui], grp = Q.grp[ui];
-                uint32_t has = 0;
-                uint64_t cnt = 0;  // 4-bit saturating counts of group members
-                for (uint32_t k = 0; k < r.len; k++) {
+                const uint32_t need = Q.nbr[ui];
+                uint32_t open = need;
+                uint64_t cnt = 0;
+                for (uint32_t k = 0; k < r.len && open; k++) {
                     const uint32_t s = S.vstate[A[k]];
                     const uint32_t c = Code(s);
                     const uint32_t sup = c == kCodeNone ? 0u : (Lit(s) & Q.uj_of[ui][c]);
-                    has |= sup;
-                    uint32_t g = sup & grp;
-                    while (g) {
-                        const uint32_t u = __ffs(g) - 1;
-                        g &= g - 1;
-                        if (((cnt >> (4 * u)) & 15u) != 15u) cnt += 1ull << (4 * u);
-                    }
+                    for (uint32_t m = sup & open; m; m &= m - 1) Supported(Q, ui, __ffs(m) - 1, 1, open, cnt);
                 }
-                if ((has & need) != need) {
-                    fail = true;
-                    dbits = need & ~has;
-                } else if (grp) {
-                    uint32_t g = grp;
-                    while (g) {
-                        const uint32_t u = __ffs(g) - 1;
-                        g &= g - 1;
-                        if (((cnt >> (4 * u)) & 15u) < ((Q.gneed[ui] >> (4 * u)) & 15u)) tobig = true;
-                    }
-                }
+                dbits = Unsupported(open, cnt);
+                fail = dbits != 0;
+                tobig = !fail && open != 0;
             }
         }
-        const uint64_t at = WaveReserve(fail ? 1u : 0u, n_died);
+        const uint64_t at = BlockReserve(fail ? 1u : 0u, n_died);
         if (fail) {
             died[at] = p;
             died_bits[at] = (uint16_t)dbits;
         }
-        const uint64_t bt = WaveReserve(tobig ? 1u : 0u, n_big);
+        const uint64_t bt = BlockReserve(tobig ? 1u : 0u, n_big);
         if (tobig) big[bt] = p;
     }
 }
@@ -349,43 +377,34 @@ __global__ void __launch_bounds__(kThreads) KS1CheckWave(GView G, QTab Q, SView 
         const uint32_t v = p >> 4, ui = p & 15u;
         const MRec r = G.rec[v];
         const uint32_t* A = G.pool + r.off;
-        const uint32_t need = Q.nbr[ui], grp = Q.grp[ui];
-        uint32_t has = 0;
+        uint32_t open = Q.nbr[ui];
         uint64_t cnt = 0;
-        for (uint32_t k0 = 0; k0 < r.len; k0 += kWave) {
-            const uint32_t k = k0 + lane;
-            uint32_t sup = 0;
-            if (k < r.len) {
-                const uint32_t s = S.vstate[A[k]];
-                const uint32_t c = Code(s);
-                sup = c == kCodeNone ? 0u : (Lit(s) & Q.uj_of[ui][c]);
+        // kCheckUnroll chunks of 64 entries in flight; most pairs that pass are
+        // done with the first.
+        for (uint32_t k0 = 0; k0 < r.len && open; k0 += kWave * kCheckUnroll) {
+            uint32_t x[kCheckUnroll], sup[kCheckUnroll];
+#pragma unroll
+            for (uint32_t c = 0; c < kCheckUnroll; c++) {
+                const uint32_t k = k0 + c * kWave + lane;
+                x[c] = k < r.len ? A[k] : ~0u;
             }
-            uint32_t nb = need;
-            while (nb) {
-                const uint32_t u = __ffs(nb) - 1;
-                nb &= nb - 1;
-                const uint64_t b = __ballot((sup >> u) & 1u);
-                if (b) {
-                    has |= 1u << u;
-                    if ((grp >> u) & 1u) {
-                        const uint64_t c = ((cnt >> (4 * u)) & 15u) + (uint64_t)__popcll(b);
-                        cnt = (cnt & ~(15ull << (4 * u))) | ((c > 15 ? 15ull : c) << (4 * u));
-                    }
+#pragma unroll
+            for (uint32_t c = 0; c < kCheckUnroll; c++) {
+                const uint32_t s = x[c] != ~0u ? S.vstate[x[c]] : kCodeNone << 12;
+                sup[c] = Code(s) == kCodeNone ? 0u : (Lit(s) & Q.uj_of[ui][Code(s)]);
+            }
+#pragma unroll
+            for (uint32_t c = 0; c < kCheckUnroll; c++)
+                for (uint32_t m = open; m; m &= m - 1) {
+                    const uint32_t u = __ffs(m) - 1;
+                    const uint64_t b = __ballot((sup[c] >> u) & 1u);
+                    if (b) Supported(Q, ui, u, (uint32_t)__popcll(b), open, cnt);
                 }
-            }
         }
-        bool fail = false;
-        uint32_t dbits = 0;
-        if ((has & need) != need) {
-            fail = true;
-            dbits = need & ~has;
-        } else if (grp) {
-            uint32_t small = 0, g = grp;
-            while (g) {
-                const uint32_t u = __ffs(g) - 1;
-                g &= g - 1;
-                if (((cnt >> (4 * u)) & 15u) < ((Q.gneed[ui] >> (4 * u)) & 15u)) small |= 1u << u;
-            }
+        const uint32_t dbits = Unsupported(open, cnt);
+        bool fail = dbits != 0;
+        if (!fail) {
+            const uint32_t small = open;
             if (small) {
                 // Gather the small members' candidates (each fewer than its
                 // group size) and test Hall's condition on them; members
@@ -452,7 +471,7 @@ __global__ void KS1Apply(QTab Q, SView S, const uint32_t* __restrict__ died, con
             }
         }
         if (killed) {
-            const uint64_t at = WaveReserve(old_pair ? 1u : 0u, n_killed);
+            const uint64_t at = BlockReserve(old_pair ? 1u : 0u, n_killed);
             if (old_pair) killed[at] = p;
         }
     }
@@ -480,11 +499,7 @@ __global__ void KS1SeedDeleted(QTab Q, SView S, const uint64_t* __restrict__ dke
                 }
             }
         }
-        for (uint32_t u = 0; u < Q.qv; u++) {
-            const bool want = ((cand >> u) & 1u) && Enqueue(S.queued, a, u);
-            const uint64_t at = WaveReserve(want ? 1u : 0u, n_out);
-            if (want) out[at] = (a << 4) | u;
-        }
+        PutPairs(a, EnqueueAll(S.queued, a, cand), out, n_out);
     }
 }
 
@@ -517,7 +532,7 @@ __global__ void KS1DelEdgeKeys(QTab Q, SView S, const uint64_t* __restrict__ dke
                 }
             }
         }
-        uint64_t at = WaveReserve(cnt, n_keys);
+        uint64_t at = BlockReserve(cnt, n_keys);
         if (cnt) {
             if (at + cnt > cap) {
                 atomicOr(ovf, 1ull);
@@ -555,8 +570,8 @@ __global__ void __launch_bounds__(kThreads) KS1EmitKilled(GView G, QTab Q, SView
                                                           unsigned long long* __restrict__ ovf) {
     const uint64_t total = offs[np];
     const uint64_t nw = (uint64_t)gridDim.x * kWpb;
-    for (uint64_t t = (uint64_t)blockIdx.x * kWpb + threadIdx.x / kWave; t * kWave < total; t += nw) {
-        const LbItem it = LbLocate(offs, np, t * kWave, total);
+    for (uint64_t t = (uint64_t)blockIdx.x * kWpb; t * kWave < total; t += nw) {
+        const LbItem it = LbLocate(offs, np, (t + threadIdx.x / kWave) * kWave, total);
         uint32_t m = 0, v = 0, ui = 0, vj = 0;
         if (it.valid) {
             const uint32_t p = K[it.p];
@@ -570,7 +585,7 @@ __global__ void __launch_bounds__(kThreads) KS1EmitKilled(GView G, QTab Q, SView
             if (vj < v) m &= ~kb;
         }
         const uint32_t cnt = 2u * (uint32_t)__popc(m);
-        uint64_t at = WaveReserve(cnt, n_keys);
+        uint64_t at = BlockReserve(cnt, n_keys);
         if (cnt) {
             if (at + cnt > cap) {
                 atomicOr(ovf, 1ull);
@@ -614,8 +629,8 @@ __global__ void __launch_bounds__(kThreads) KS1Expand(GView G, QTab Q, SView S, 
                                                       unsigned long long* __restrict__ n_out) {
     const uint64_t total = offs[np];
     const uint64_t nw = (uint64_t)gridDim.x * kWpb;
-    for (uint64_t t = (uint64_t)blockIdx.x * kWpb + threadIdx.x / kWave; t * kWave < total; t += nw) {
-        const LbItem it = LbLocate(offs, np, t * kWave, total);
+    for (uint64_t t = (uint64_t)blockIdx.x * kWpb; t * kWave < total; t += nw) {
+        const LbItem it = LbLocate(offs, np, (t + threadIdx.x / kWave) * kWave, total);
         uint32_t cand = 0, vj = 0;
         if (it.valid) {
             const uint32_t p = D[it.p], v = p >> 4, ui = p & 15u;
@@ -624,11 +639,7 @@ __global__ void __launch_bounds__(kThreads) KS1Expand(GView G, QTab Q, SView S, 
             const uint32_t c = Code(s);
             cand = c == kCodeNone ? 0u : (Q.uj_of[ui][c] & Lit(s) & (opt_only ? Opt(s) : 0xFFFu));
         }
-        for (uint32_t u = 0; u < Q.qv; u++) {
-            const bool want = ((cand >> u) & 1u) && Enqueue(S.queued, vj, u);
-            const uint64_t at = WaveReserve(want ? 1u : 0u, n_out);
-            if (want) out[at] = (vj << 4) | u;
-        }
+        PutPairs(vj, EnqueueAll(S.queued, vj, cand), out, n_out);
     }
 }
 
@@ -648,18 +659,14 @@ __global__ void KS1TouchNew(QTab Q, SView S, const uint64_t* __restrict__ ekeys,
             cb = Code(S.vstate[b]);
             if (Code(sa) != kCodeNone && cb != kCodeNone) cand = Q.by_code[Code(sa)] & ~Lit(sa);
         }
-        for (uint32_t u = 0; u < Q.qv; u++) {
-            bool want = false;
-            if ((cand >> u) & 1u) {
-                const uint32_t m = Q.uj_of[u][cb];
-                if (m) {
-                    DeadClear(S.dead, a, u, Q.qv, m);
-                    want = Enqueue(S.queued, a, u);
-                }
-            }
-            const uint64_t at = WaveReserve(want ? 1u : 0u, n_out);
-            if (want) out[at] = (a << 4) | u;
+        uint32_t hit = 0;
+        for (; cand; cand &= cand - 1) {
+            const uint32_t u = __ffs(cand) - 1, m = Q.uj_of[u][cb];
+            if (!m) continue;
+            DeadClear(S.dead, a, u, Q.qv, m);
+            hit |= 1u << u;
         }
+        PutPairs(a, EnqueueAll(S.queued, a, hit), out, n_out);
     }
 }
 
@@ -683,9 +690,9 @@ __global__ void KS1Activate(QTab Q, SView S, const uint32_t* __restrict__ T, con
                 on = true;
             }
         }
-        const uint64_t at = WaveReserve(on ? 1u : 0u, n_act);
+        const uint64_t at = BlockReserve(on ? 1u : 0u, n_act);
         if (on) act[at] = p;
-        const uint64_t ot = WaveReserve(on ? 1u : 0u, n_opt);
+        const uint64_t ot = BlockReserve(on ? 1u : 0u, n_opt);
         if (on) opt[ot] = p;
     }
 }
@@ -696,8 +703,8 @@ __global__ void __launch_bounds__(kThreads) KS1Push(GView G, QTab Q, SView S, co
                                                     uint32_t* __restrict__ out, unsigned long long* __restrict__ n_out) {
     const uint64_t total = offs[np];
     const uint64_t nw = (uint64_t)gridDim.x * kWpb;
-    for (uint64_t t = (uint64_t)blockIdx.x * kWpb + threadIdx.x / kWave; t * kWave < total; t += nw) {
-        const LbItem it = LbLocate(offs, np, t * kWave, total);
+    for (uint64_t t = (uint64_t)blockIdx.x * kWpb; t * kWave < total; t += nw) {
+        const LbItem it = LbLocate(offs, np, (t + threadIdx.x / kWave) * kWave, total);
         uint32_t cand = 0, vj = 0, ui = 0;
         if (it.valid) {
             const uint32_t p = A[it.p], v = p >> 4;
@@ -707,15 +714,8 @@ __global__ void __launch_bounds__(kThreads) KS1Push(GView G, QTab Q, SView S, co
             const uint32_t c = Code(s);
             cand = c == kCodeNone ? 0u : (Q.uj_of[ui][c] & ~Lit(s));
         }
-        for (uint32_t u = 0; u < Q.qv; u++) {
-            bool want = false;
-            if ((cand >> u) & 1u) {
-                DeadClear(S.dead, vj, u, Q.qv, 1u << ui);
-                want = Enqueue(S.queued, vj, u);
-            }
-            const uint64_t at = WaveReserve(want ? 1u : 0u, n_out);
-            if (want) out[at] = (vj << 4) | u;
-        }
+        for (uint32_t c = cand; c; c &= c - 1) DeadClear(S.dead, vj, __ffs(c) - 1, Q.qv, 1u << ui);
+        PutPairs(vj, EnqueueAll(S.queued, vj, cand), out, n_out);
     }
 }
 
@@ -740,7 +740,7 @@ __global__ void KS1Survivors(SView S, const uint32_t* __restrict__ opt, const un
                 if (S.new_of[v] == ~0u) atomicOr(&newv[v >> 5], 1u << (v & 31));
             }
         }
-        const uint64_t at = WaveReserve(keep ? 1u : 0u, n_y);
+        const uint64_t at = BlockReserve(keep ? 1u : 0u, n_y);
         if (keep) Y[at] = p;
     }
 }
@@ -792,8 +792,8 @@ __global__ void __launch_bounds__(kThreads) KS1EmitPairs(GView G, QTab Q, SView 
                                                          unsigned long long* __restrict__ ovf) {
     const uint64_t total = offs[np];
     const uint64_t nw = (uint64_t)gridDim.x * kWpb;
-    for (uint64_t t = (uint64_t)blockIdx.x * kWpb + threadIdx.x / kWave; t * kWave < total; t += nw) {
-        const LbItem it = LbLocate(offs, np, t * kWave, total);
+    for (uint64_t t = (uint64_t)blockIdx.x * kWpb; t * kWave < total; t += nw) {
+        const LbItem it = LbLocate(offs, np, (t + threadIdx.x / kWave) * kWave, total);
         uint32_t m = 0, v = 0, ui = 0, vj = 0;
         if (it.valid) {
             const uint32_t p = Y[it.p];
@@ -806,7 +806,7 @@ __global__ void __launch_bounds__(kThreads) KS1EmitPairs(GView G, QTab Q, SView 
         }
         const uint32_t per = both ? 2u : 1u;
         const uint32_t cnt = (uint32_t)__popc(m) * per;
-        uint64_t at = WaveReserve(cnt, n_keys);
+        uint64_t at = BlockReserve(cnt, n_keys);
         if (cnt) {
             if (at + cnt > cap) {
                 atomicOr(ovf, 1ull);
@@ -853,7 +853,7 @@ __global__ void KS1EmitUpdates(QTab Q, SView S, const int32_t* __restrict__ ints
                 }
             }
         }
-        uint64_t at = WaveReserve(cnt, n_upd);
+        uint64_t at = BlockReserve(cnt, n_upd);
         if (cnt) {
             if (at + cnt > cap) {
                 atomicOr(ovf, 1ull);
@@ -1126,7 +1126,7 @@ void S1DeletionRounds(cgbdsm_query* q, int src, uint64_t n, bool opt_only, uint3
         S1Set(q, &S1Cnt::n_big, 0);
         KS1Check<<<Grid(n), kThreads, 0, q->s>>>(G, S->tab, V, S->L[cur].p, n_cur, S->L[2].p, S->died_bits.p,
                                                  &S->d_c->n_died, S->L[3].p, &S->d_c->n_big);
-        KS1CheckWave<<<Grid(n, kWpb, 16384), kThreads, 0, q->s>>>(G, S->tab, V, S->L[3].p, &S->d_c->n_big,
+        KS1CheckWave<<<Grid(n, kWpb, 2048), kThreads, 0, q->s>>>(G, S->tab, V, S->L[3].p, &S->d_c->n_big,
                                                                  S->L[2].p, S->died_bits.p, &S->d_c->n_died);
         // The deaths (at most n) are applied and their neighbours queued with
         // the device count: one host round trip per round.

@@ -53,7 +53,8 @@ struct cgbdsm_query {
     DBuf<URec> u_rec;
     DBuf<uint32_t> pool;
     Counters* d_cnt = nullptr;
-    Counters* h_cnt = nullptr;
+    Mailbox box;                // of d_cnt
+    Counters* h_cnt = nullptr;  // its data: the last read-back
     DBuf<uint64_t> k_ins, k_del, k_upd, k_usort, k_alt, seg_start, caps;
     DBuf<uint32_t> flags, seg_row, sc_val, sc_pos, rs_hist, u_vals, u_rows;
     DBuf<uint8_t> scan_scratch;

@@ -109,8 +109,8 @@ Tables MakeTables(cgbdsm_query* q) {
 }
 
 void ReadCounters(cgbdsm_query* q) {
-    CGD_HIP(hipMemcpyAsync(q->h_cnt, q->d_cnt, sizeof(Counters), hipMemcpyDeviceToHost, q->s));
-    CGD_HIP(hipStreamSynchronize(q->s));
+    q->box.Request(q->d_cnt, sizeof(Counters), q->s);
+    q->box.Wait(q->s);
 }
 
 unsigned long long* Cnt(cgbdsm_query* q, unsigned long long Counters::*f) { return &(q->d_cnt->*f); }
@@ -387,7 +387,10 @@ void RunDfsJobs(cgbdsm_query* q, uint32_t* tuples, uint64_t tup_cap) {
     }
     *(volatile uint32_t*)q->h_abort = 0;
     std::atomic_thread_fence(std::memory_order_seq_cst);
-    if (!n) return;
+    if (!n) {
+        ReadCounters(q);
+        return;
+    }
     Ensure(q, q->d_jobs, q->h_jobs.size());
     Ensure(q, q->d_rowbase, q->h_rowbase.size());
     CGD_HIP(hipMemcpyAsync(q->d_jobs.p, q->h_jobs.data(), q->h_jobs.size() * sizeof(DfsJob), hipMemcpyHostToDevice,
@@ -411,36 +414,44 @@ void RunDfsJobs(cgbdsm_query* q, uint32_t* tuples, uint64_t tup_cap) {
               q->st.last_dfs_lds_cache, batched, q->s);
     KEnd(q, k);
     CGD_HIP(hipGetLastError());
-    if (q->deadline_ms > 0) {
-        const auto t0 = std::chrono::steady_clock::now();
-        for (;;) {
-            hipError_t e = hipStreamQuery(q->s);
-            if (e == hipSuccess) break;
-            if (e != hipErrorNotReady) CGD_HIP(e);
-            const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-            if (ms > q->deadline_ms) {
-                *(volatile uint32_t*)q->h_abort = 1;
-                std::atomic_thread_fence(std::memory_order_seq_cst);
-                CGD_HIP(hipStreamSynchronize(q->s));
-                *(volatile uint32_t*)q->h_abort = 0;
-                ReadCounters(q);
-                unsigned long long part = 0;
-                for (uint32_t e = 0; e < q->qe; e++) part += q->h_cnt->per_edge[e];
-                Throw(CGBDSM_ERR_OVERFLOW, "final DFS exceeded the deadline of " + std::to_string(q->deadline_ms) +
-                                               " ms; count incomplete (partial " + std::to_string(part) +
-                                               " matches, " + std::to_string(q->h_cnt->scanned) + " candidates, " +
-                                               std::to_string(q->h_cnt->probes) + " probes, " + std::to_string(n) +
-                                               " rows at depth " + std::to_string(depth) + ", " +
-                                               std::to_string(q->h_cnt->q_rows.v) + " rows taken, " +
-                                               std::to_string(q->h_cnt->donated) + " donated; pending " +
-                                               std::to_string(q->h_cnt->q_pending.v) + ", idle " +
-                                               std::to_string(q->h_cnt->q_idle.v) + ", queue " +
-                                               std::to_string(q->h_cnt->q_head.v) + "/" +
-                                               std::to_string(q->h_cnt->q_tail.v) + ", flags " +
-                                               std::to_string(q->h_cnt->flags) + ")");
-            }
-            std::this_thread::sleep_for(std::chrono::microseconds(200));
+    // The counters come back with the launch.  The host watches for them
+    // without sleeping at first (a batch's launch is often over in 0.1 ms),
+    // then for a sixteenth of the time waited so far, 200 us at most.
+    q->box.Request(q->d_cnt, sizeof(Counters), q->s);
+    const auto t0 = std::chrono::steady_clock::now();
+    for (uint32_t i = 1; !q->box.Arrived(); i++) {
+        if (i & 63u) {
+            __builtin_ia32_pause();
+            continue;
         }
+        const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+        if (ms < 0.5) continue;
+        const hipError_t e = hipStreamQuery(q->s);
+        if (e != hipSuccess && e != hipErrorNotReady) CGD_HIP(e);
+        if (e == hipSuccess && !q->box.Arrived()) q->box.Wait(q->s);
+        if (q->deadline_ms > 0 && ms > q->deadline_ms) {
+            *(volatile uint32_t*)q->h_abort = 1;
+            std::atomic_thread_fence(std::memory_order_seq_cst);
+            CGD_HIP(hipStreamSynchronize(q->s));
+            *(volatile uint32_t*)q->h_abort = 0;
+            ReadCounters(q);
+            unsigned long long part = 0;
+            for (uint32_t e = 0; e < q->qe; e++) part += q->h_cnt->per_edge[e];
+            Throw(CGBDSM_ERR_OVERFLOW, "final DFS exceeded the deadline of " + std::to_string(q->deadline_ms) +
+                                           " ms; count incomplete (partial " + std::to_string(part) +
+                                           " matches, " + std::to_string(q->h_cnt->scanned) + " candidates, " +
+                                           std::to_string(q->h_cnt->probes) + " probes, " + std::to_string(n) +
+                                           " rows at depth " + std::to_string(depth) + ", " +
+                                           std::to_string(q->h_cnt->q_rows.v) + " rows taken, " +
+                                           std::to_string(q->h_cnt->donated) + " donated; pending " +
+                                           std::to_string(q->h_cnt->q_pending.v) + ", idle " +
+                                           std::to_string(q->h_cnt->q_idle.v) + ", queue " +
+                                           std::to_string(q->h_cnt->q_head.v) + "/" +
+                                           std::to_string(q->h_cnt->q_tail.v) + ", flags " +
+                                           std::to_string(q->h_cnt->flags) + ")");
+        }
+        std::this_thread::sleep_for(std::chrono::duration<double, std::milli>(std::min(0.2, ms / 16)));
+        i |= 63u;
     }
 }
 
@@ -761,8 +772,8 @@ cgbdsm_status cgbdsm_query_create(cgbdsm_ctx* ctx, const cgbdsm_plan* plan, cgbd
             CGD_HIP(hipEventCreateWithFlags(&q->fr_ev, hipEventDisableTiming));
             q->d_plan = (DevPlan*)DevAlloc(ctx, sizeof(DevPlan));
             q->d_cnt = (Counters*)DevAlloc(ctx, sizeof(Counters));
-            CGD_HIP(hipHostMalloc((void**)&q->h_cnt, sizeof(Counters), hipHostMallocDefault));
-            memset(q->h_cnt, 0, sizeof(Counters));
+            q->box.Alloc(sizeof(Counters));
+            q->h_cnt = (Counters*)q->box.data();
             CGD_HIP(hipHostMalloc((void**)&q->h_abort, 64, hipHostMallocMapped | hipHostMallocCoherent));
             *(volatile uint32_t*)q->h_abort = 0;
             CGD_HIP(hipHostGetDevicePointer((void**)&q->d_abort, q->h_abort, 0));
@@ -823,7 +834,6 @@ cgbdsm_status cgbdsm_query_destroy(cgbdsm_query* q) {
         }
         if (q->d_plan) DevFree(q->ctx, q->d_plan, sizeof(DevPlan));
         if (q->d_cnt) DevFree(q->ctx, q->d_cnt, sizeof(Counters));
-        if (q->h_cnt) (void)hipHostFree(q->h_cnt);
         if (q->h_abort) (void)hipHostFree(q->h_abort);
         if (q->steal_items) DevFree(q->ctx, q->steal_items, q->steal_cap * sizeof(StealItem));
         if (q->steal_seq) DevFree(q->ctx, q->steal_seq, q->steal_cap * sizeof(unsigned long long));
@@ -1361,7 +1371,6 @@ static void ResetDfsCounters(cgbdsm_query* q) {
 
 // Statistics of the final-DFS launch whose queue lived in `leader`.
 static void CheckDfs(cgbdsm_query* leader, uint64_t rows) {
-    ReadCounters(leader);
     const Counters* c = leader->h_cnt;
     if (c->flags & kFlagBadRow)
         Throw(CGBDSM_ERR_DEVICE, "final DFS read a frontier row with an out-of-range tag or vertex id");
@@ -1433,6 +1442,7 @@ cgbdsm_status cgbdsm_matching(cgbdsm_query* q, unsigned long long* num_matches, 
                 CGD_HIP(hipEventRecord(q->ev[6], q->s));
                 RunDfs(q, q->front[f.cur].p + k * f.depth, f.n - k, f.depth, nullptr, 0);
                 CGD_HIP(hipEventRecord(q->ev[7], q->s));
+                CGD_HIP(hipEventSynchronize(q->ev[7]));
                 CheckDfs(q, f.n - k);
             } catch (...) {
                 SplitJoin(q, true);
@@ -1480,11 +1490,11 @@ cgbdsm_status cgbdsm_matching_batch(cgbdsm_query* const* qs, int nq, unsigned lo
         for (int i = 0; i < nq; i++) ResetMatchCounters(qs[i], lead->s);
         ResetDfsCounters(lead);
         RunDfsJobs(lead, nullptr, 0);
-        // The other queries' counters come back on the launch's stream, with
-        // the lead's (CheckDfs): one wait instead of one per query.
+        // The other queries' counters come back on the launch's stream.
         for (int i = 0; i < nq; i++)
-            if (qs[i] != lead)
-                CGD_HIP(hipMemcpyAsync(qs[i]->h_cnt, qs[i]->d_cnt, sizeof(Counters), hipMemcpyDeviceToHost, lead->s));
+            if (qs[i] != lead) qs[i]->box.Request(qs[i]->d_cnt, sizeof(Counters), lead->s);
+        for (int i = 0; i < nq; i++)
+            if (qs[i] != lead) qs[i]->box.Wait(lead->s);
         CheckDfs(lead, lead->h_rowbase.back());
         for (int i = 0; i < nq; i++) {
             FinishMatching(qs[i], fr[i], lead, num_matches ? &num_matches[i] : nullptr,

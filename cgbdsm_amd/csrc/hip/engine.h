@@ -202,4 +202,27 @@ struct WordSet {
 void SetWords(uint64_t* base, const WordSet& ws, hipStream_t s);
 void FillU32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s);
 
+// Read-back of a small device block through coherent pinned host memory: a
+// kernel stores the block and then a sequence number there, and the host
+// watches the number.  (A copy into pinned memory and a stream synchronize cost
+// a copy kernel and about 20 us of the host's time for every size that decides
+// the next launch, over thirty times a batch.)
+class Mailbox {
+   public:
+    ~Mailbox() { Free(); }
+    void Alloc(size_t bytes);
+    void Free();
+    void* data() const { return host_ ? host_ + kHeader : nullptr; }
+    // Enqueues the read-back of `bytes` bytes (at most Alloc's) of src on s.
+    void Request(const void* src, size_t bytes, hipStream_t s);
+    bool Arrived() const;
+    // Waits for the last request, made on s.
+    void Wait(hipStream_t s) const;
+
+   private:
+    static constexpr size_t kHeader = 16;  // words before the data: the sequence number's own line
+    uint64_t *host_ = nullptr, *dev_ = nullptr;
+    uint64_t seq_ = 0;
+};
+
 }  // namespace cgd

@@ -2,6 +2,10 @@
 // stable LSD radix sort of u64 keys with 8-bit digits.  These replace the
 // thrust::sort / unique and CUB scan calls of the reference
 // (index/calig_helper_gamma.cu:304, 491-492, 573; graph/graph_gpu.cu:1395-1400).
+#include <atomic>
+#include <chrono>
+#include <cstring>
+
 #include "engine.h"
 #include "wave.h"
 
@@ -140,6 +144,16 @@ __global__ void KSetWords(uint64_t* base, WordSet ws) {
 __global__ void KFill32(uint32_t* p, uint32_t v, uint64_t n) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
         p[i] = v;
+}
+
+// Words of a device block, then the sequence number, into coherent host memory.
+__global__ void __launch_bounds__(256) KPublish(const uint64_t* __restrict__ src, uint32_t words, uint64_t* dst,
+                                                uint64_t* seq_at, uint64_t seq) {
+    for (uint32_t i = threadIdx.x; i < words; i += blockDim.x)
+        __hip_atomic_store(&dst[i], src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(seq_at, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------- radix sort
@@ -298,6 +312,41 @@ void FillU32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s) {
     if (!n) return;
     unsigned g = (unsigned)std::min<uint64_t>((n + 255) / 256, 4096);
     KFill32<<<g, 256, 0, s>>>(p, v, n);
+}
+
+void Mailbox::Alloc(size_t bytes) {
+    void *h = nullptr, *d = nullptr;
+    const size_t n = kHeader * 8 + bytes;
+    CGD_HIP(hipHostMalloc(&h, n, hipHostMallocMapped | hipHostMallocCoherent));
+    host_ = (uint64_t*)h;
+    memset(h, 0, n);
+    CGD_HIP(hipHostGetDevicePointer(&d, h, 0));
+    dev_ = (uint64_t*)d;
+}
+void Mailbox::Free() {
+    if (host_) (void)hipHostFree(host_);
+    host_ = dev_ = nullptr;
+}
+void Mailbox::Request(const void* src, size_t bytes, hipStream_t s) {
+    KPublish<<<1, 256, 0, s>>>((const uint64_t*)src, (uint32_t)(bytes / 8), dev_ + kHeader, dev_, ++seq_);
+    CGD_HIP(hipGetLastError());
+}
+bool Mailbox::Arrived() const {
+    if (*(volatile uint64_t*)host_ != seq_) return false;
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return true;
+}
+void Mailbox::Wait(hipStream_t s) const {
+    // Short waits by watching; a longer one leaves the processor to others.
+    const auto t0 = std::chrono::steady_clock::now();
+    for (uint32_t i = 0; !Arrived(); i++) {
+        if ((i & 63u) == 63u && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) {
+            CGD_HIP(hipStreamSynchronize(s));
+            if (!Arrived()) throw HipError(hipErrorUnknown, "counter read-back", __FILE__, __LINE__);
+            return;
+        }
+        __builtin_ia32_pause();
+    }
 }
 
 size_t RadixHistWords(uint64_t n) {

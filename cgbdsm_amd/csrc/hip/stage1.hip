@@ -923,7 +923,8 @@ struct cgbdsm_graph {
     DBuf<MRec> rec;
     DBuf<uint32_t> pool;
     Counters* d_cnt = nullptr;
-    Counters* h_cnt = nullptr;
+    Mailbox box;                // of d_cnt
+    Counters* h_cnt = nullptr;  // its data
     DBuf<int32_t> stream;          // update ints (two per pair; negative ids: deletions)
     uint64_t stream_ints = 0;
     uint64_t batches = 0;          // batches applied
@@ -958,7 +959,8 @@ struct S1Query {
     uint8_t neg_ok[kMaxQE] = {};       // edge_ok of the negative pass
     DBuf<uint64_t> sv_ins, sv_del, sv_upd;  // the positive batch's key buffers during the negative pass
     S1Cnt* d_c = nullptr;
-    S1Cnt* h_c = nullptr;
+    Mailbox box;           // of d_c
+    S1Cnt* h_c = nullptr;  // its data
     uint32_t dv = 0;
     // statistics of the last call
     double ms = 0;
@@ -991,8 +993,8 @@ void GRelease(cgbdsm_ctx* ctx, DBuf<T>& b) {
 }
 
 void GReadCounters(cgbdsm_graph* g) {
-    CGD_HIP(hipMemcpyAsync(g->h_cnt, g->d_cnt, sizeof(Counters), hipMemcpyDeviceToHost, g->s));
-    CGD_HIP(hipStreamSynchronize(g->s));
+    g->box.Request(g->d_cnt, sizeof(Counters), g->s);
+    g->box.Wait(g->s);
 }
 
 Tables GraphTables(cgbdsm_graph* g) {
@@ -1090,8 +1092,8 @@ void GraphMerge(cgbdsm_graph* g, const uint64_t* keys, uint64_t nk) {
 SView SV(S1Query* S) { return SView{S->vstate.p, S->queued.p, S->dead.p, S->new_of.p, S->old_of.p}; }
 
 void S1Read(cgbdsm_query* q) {
-    CGD_HIP(hipMemcpyAsync(q->s1->h_c, q->s1->d_c, sizeof(S1Cnt), hipMemcpyDeviceToHost, q->s));
-    CGD_HIP(hipStreamSynchronize(q->s));
+    q->s1->box.Request(q->s1->d_c, sizeof(S1Cnt), q->s);
+    q->s1->box.Wait(q->s);
 }
 
 void S1Set(cgbdsm_query* q, unsigned long long S1Cnt::*f, uint64_t v) {
@@ -1274,7 +1276,6 @@ void S1Free(cgbdsm_query* q) {
     Release(q, S->offs);
     for (auto* b : {&S->kd, &S->sv_ins, &S->sv_del, &S->sv_upd}) Release(q, *b);
     if (S->d_c) DevFree(q->ctx, S->d_c, sizeof(S1Cnt));
-    if (S->h_c) (void)hipHostFree(S->h_c);
     delete S;
     q->s1 = nullptr;
 }
@@ -1310,7 +1311,8 @@ cgbdsm_status cgbdsm_graph_create(cgbdsm_ctx* ctx, uint32_t n, const int32_t* la
             CGD_HIP(hipStreamCreateWithFlags(&g->s, hipStreamNonBlocking));
             CGD_HIP(hipEventCreateWithFlags(&g->ev, hipEventDisableTiming));
             g->d_cnt = (Counters*)DevAlloc(ctx, sizeof(Counters));
-            CGD_HIP(hipHostMalloc((void**)&g->h_cnt, sizeof(Counters), hipHostMallocDefault));
+            g->box.Alloc(sizeof(Counters));
+            g->h_cnt = (Counters*)g->box.data();
             FillU64((uint64_t*)g->d_cnt, 0, sizeof(Counters) / 8, g->s);
             GEnsure(g, g->labels, n);
             CGD_HIP(hipMemcpyAsync(g->labels.p, labels, (size_t)n * 4, hipMemcpyHostToDevice, g->s));
@@ -1367,7 +1369,6 @@ cgbdsm_status cgbdsm_graph_destroy(cgbdsm_graph* g) {
         for (auto* b : {&g->flags, &g->seg_row, &g->sc_val, &g->sc_pos, &g->hist}) GRelease(c, *b);
         GRelease(c, g->scan);
         if (g->d_cnt) DevFree(c, g->d_cnt, sizeof(Counters));
-        if (g->h_cnt) (void)hipHostFree(g->h_cnt);
         if (g->ev) (void)hipEventDestroy(g->ev);
         if (g->s) (void)hipStreamDestroy(g->s);
         delete g;
@@ -1461,7 +1462,8 @@ cgbdsm_status cgbdsm_calig_attach(cgbdsm_query* q, cgbdsm_graph* g, const int32_
             S->batches = g->batches;
             const uint32_t n = g->n;
             S->d_c = (S1Cnt*)DevAlloc(q->ctx, sizeof(S1Cnt));
-            CGD_HIP(hipHostMalloc((void**)&S->h_c, sizeof(S1Cnt), hipHostMallocDefault));
+            S->box.Alloc(sizeof(S1Cnt));
+            S->h_c = (S1Cnt*)S->box.data();
             FillU64((uint64_t*)S->d_c, 0, sizeof(S1Cnt) / 8, q->s);
             CGD_HIP(hipStreamWaitEvent(q->s, g->ev, 0));
             Ensure(q, S->vstate, n);

@@ -187,6 +187,35 @@ void DecodeSort(cgbdsm_query* q, const uint64_t* src, uint64_t* dst, uint64_t* a
     KAdd(q, CGBDSM_K_SORT, 0, n);
 }
 
+// The key set `in` of q (n keys, at most kKeySetMax) through one launch: sorted
+// (decode) and made unique into out, segments into q's scratch, counts into
+// n_unique and n_segs.
+KeySet MakeKeySet(cgbdsm_query* q, const uint64_t* in, uint64_t n, bool decode, bool unique, uint64_t* out) {
+    KeySet a{};
+    a.in = in;
+    a.n = (uint32_t)n;
+    a.decode = decode;
+    a.unique = unique;
+    a.ushift = q->ushift;
+    a.umask = q->umask;
+    a.ndir = q->ndir;
+    a.vbits = q->vbits;
+    a.bits = q->vbits + q->rbits;
+    a.out = out;
+    a.n_out = Cnt(q, &Counters::n_unique);
+    a.seg_row = q->seg_row.p;
+    a.seg_start = q->seg_start.p;
+    a.n_segs = Cnt(q, &Counters::n_segs);
+    return a;
+}
+
+void RunKeySet(cgbdsm_query* q, const KeySet& a) {
+    const int k = KBegin(q, CGBDSM_K_SORT);
+    LaunchKeySet(a, q->s);
+    KEnd(q, k);
+    KAdd(q, CGBDSM_K_SORT, 0, a.n);
+}
+
 void GrowPool(cgbdsm_query* q, uint64_t min_cap) {
     ReadCounters(q);
     uint64_t used = q->h_cnt->pool_top;
@@ -202,10 +231,13 @@ void GrowPool(cgbdsm_query* q, uint64_t min_cap) {
 }
 
 // M <- M u keys (sorted internal keys, unique), retrying after pool growth.
-void InsertSorted(cgbdsm_query* q, const uint64_t* keys, const unsigned long long* n_segs, uint64_t n_upper) {
+// zeroed: the counters are already reset.
+void InsertSorted(cgbdsm_query* q, const uint64_t* keys, const unsigned long long* n_segs, uint64_t n_upper,
+                  bool zeroed = false) {
     for (int attempt = 0;; attempt++) {
-        SetCounters(q, {{&Counters::flags, 0}, {&Counters::bytes, 0}, {&Counters::n_long, 0}, {&Counters::n_huge, 0}},
-                    q->s);
+        if (!zeroed || attempt)
+            SetCounters(q, {{&Counters::flags, 0}, {&Counters::bytes, 0}, {&Counters::n_long, 0},
+                            {&Counters::n_huge, 0}}, q->s);
         const int k = KBegin(q, CGBDSM_K_MERGE_INSERT);
         // q->flags (segment discovery's scan) is free again: long-list queue.
         LaunchMergeInsert(MakeTables(q), keys, q->vbits, q->seg_row.p, q->seg_start.p, n_segs, n_upper, q->sc_val.p,
@@ -1081,19 +1113,25 @@ cgbdsm_status cgbdsm_transfer_update_all(cgbdsm_query* q) {
         // The host mirror takes the batch's keys before the device's sort
         // reuses their buffers.
         if (q->split) SplitOnApply(q);
-        SetCounter(q, &Counters::bytes, 0);
-        SetCounter(q, &Counters::rows_touched, 0);
+        SetCounters(q, {{&Counters::bytes, 0}, {&Counters::rows_touched, 0}}, q->s);
         q->batch_idx_bytes = 0;
         if (q->layout == CGBDSM_LAYOUT_GPMA) {
             if (q->n_ins) {
-                DecodeSort(q, q->k_ins.p, q->k_alt.p, q->k_ins.p, q->n_ins);
-                LaunchUnique(q->k_alt.p, q->k_ins.p, q->n_ins, q->flags.p, q->scan_scratch.p,
-                             Cnt(q, &Counters::n_unique), q->s);
+                if (q->n_ins <= kKeySetMax) {
+                    RunKeySet(q, MakeKeySet(q, q->k_ins.p, q->n_ins, true, true, q->k_ins.p));
+                } else {
+                    DecodeSort(q, q->k_ins.p, q->k_alt.p, q->k_ins.p, q->n_ins);
+                    LaunchUnique(q->k_alt.p, q->k_ins.p, q->n_ins, q->flags.p, q->scan_scratch.p,
+                                 Cnt(q, &Counters::n_unique), q->s);
+                }
                 ReadCounters(q);
                 PmaInsert(q, q->k_ins.p, q->h_cnt->n_unique);
             }
             if (q->n_del) {
-                DecodeSort(q, q->k_del.p, q->k_alt.p, q->k_del.p, q->n_del);
+                if (q->n_del <= kKeySetMax)
+                    RunKeySet(q, MakeKeySet(q, q->k_del.p, q->n_del, true, false, q->k_alt.p));
+                else
+                    DecodeSort(q, q->k_del.p, q->k_alt.p, q->k_del.p, q->n_del);
                 PmaDelete(q, q->k_alt.p, q->n_del);
             }
             PmaExtract(q);
@@ -1101,19 +1139,32 @@ cgbdsm_status cgbdsm_transfer_update_all(cgbdsm_query* q) {
             return;
         }
         if (q->n_ins) {
-            DecodeSort(q, q->k_ins.p, q->k_alt.p, q->k_ins.p, q->n_ins);
-            LaunchUnique(q->k_alt.p, q->k_ins.p, q->n_ins, q->flags.p, q->scan_scratch.p, Cnt(q, &Counters::n_unique),
-                         q->s);
-            LaunchSegments(q->k_ins.p, Cnt(q, &Counters::n_unique), q->n_ins, q->vbits, q->flags.p, q->seg_row.p,
-                           q->seg_start.p, Cnt(q, &Counters::n_segs), q->scan_scratch.p, q->s);
-            InsertSorted(q, q->k_ins.p, Cnt(q, &Counters::n_segs), q->n_ins);
+            const bool small = q->n_ins <= kKeySetMax;
+            if (small) {
+                KeySet a = MakeKeySet(q, q->k_ins.p, q->n_ins, true, true, q->k_ins.p);
+                a.zero = q->d_cnt;
+                RunKeySet(q, a);
+            } else {
+                DecodeSort(q, q->k_ins.p, q->k_alt.p, q->k_ins.p, q->n_ins);
+                LaunchUnique(q->k_alt.p, q->k_ins.p, q->n_ins, q->flags.p, q->scan_scratch.p,
+                             Cnt(q, &Counters::n_unique), q->s);
+                LaunchSegments(q->k_ins.p, Cnt(q, &Counters::n_unique), q->n_ins, q->vbits, q->flags.p,
+                               q->seg_row.p, q->seg_start.p, Cnt(q, &Counters::n_segs), q->scan_scratch.p, q->s);
+            }
+            InsertSorted(q, q->k_ins.p, Cnt(q, &Counters::n_segs), q->n_ins, small);
         }
         if (q->n_del) {
-            DecodeSort(q, q->k_del.p, q->k_alt.p, q->k_del.p, q->n_del);
-            SetCounter(q, &Counters::n_unique, q->n_del);
-            LaunchSegments(q->k_alt.p, Cnt(q, &Counters::n_unique), q->n_del, q->vbits, q->flags.p, q->seg_row.p,
-                           q->seg_start.p, Cnt(q, &Counters::n_segs), q->scan_scratch.p, q->s);
-            SetCounters(q, {{&Counters::bytes, 0}, {&Counters::n_long, 0}, {&Counters::n_huge, 0}}, q->s);
+            if (q->n_del <= kKeySetMax) {
+                KeySet a = MakeKeySet(q, q->k_del.p, q->n_del, true, false, q->k_alt.p);
+                a.zero = q->d_cnt;
+                RunKeySet(q, a);
+            } else {
+                DecodeSort(q, q->k_del.p, q->k_alt.p, q->k_del.p, q->n_del);
+                SetCounter(q, &Counters::n_unique, q->n_del);
+                LaunchSegments(q->k_alt.p, Cnt(q, &Counters::n_unique), q->n_del, q->vbits, q->flags.p,
+                               q->seg_row.p, q->seg_start.p, Cnt(q, &Counters::n_segs), q->scan_scratch.p, q->s);
+                SetCounters(q, {{&Counters::bytes, 0}, {&Counters::n_long, 0}, {&Counters::n_huge, 0}}, q->s);
+            }
             const int k = KBegin(q, CGBDSM_K_MERGE_REMOVE);
             LaunchMergeRemove(MakeTables(q), q->k_alt.p, q->vbits, q->seg_row.p, q->seg_start.p,
                               Cnt(q, &Counters::n_segs), q->n_del, q->flags.p, q->d_cnt, q->s);
@@ -1131,11 +1182,26 @@ cgbdsm_status cgbdsm_transfer_update_index(cgbdsm_query* q, int* nonempty) {
     return Guard([&] {
         if (!q || q->phase != 2) Throw(CGBDSM_ERR_INVALID, "transfer_update_index must follow transfer_update_all");
         if (q->split) SplitOnUpdateIndex(q);
-        LaunchClearU(q->u_rec.p, q->u_rows.p, Cnt(q, &Counters::u_rows), q->u_rows_upper, q->s);
-        SetCounter(q, &Counters::u_rows, 0);
-        q->u_rows_upper = 0;
         q->u_nonempty = q->n_upd > 0;
-        if (q->n_upd) {
+        // Small sets in one launch, which also clears the last batch's rows
+        // (a block clears them at about 20 per microsecond).
+        const bool small = q->n_upd && q->n_upd <= kKeySetMax && q->u_rows_upper <= 4 * kKeySetMax;
+        if (!small) {
+            LaunchClearU(q->u_rec.p, q->u_rows.p, Cnt(q, &Counters::u_rows), q->u_rows_upper, q->s);
+            if (q->u_rows_upper) SetCounter(q, &Counters::u_rows, 0);
+            q->u_rows_upper = 0;
+        }
+        if (small) {
+            KeySet a = MakeKeySet(q, q->k_upd.p, q->n_upd, true, false, q->k_usort.p);
+            a.n_dups = Cnt(q, &Counters::u_dups);
+            a.u_rec = q->u_rec.p;
+            a.u_vals = q->u_vals.p;
+            a.u_rows = q->u_rows.p;
+            a.u_rows_count = Cnt(q, &Counters::u_rows);
+            RunKeySet(q, a);
+            KAdd(q, CGBDSM_K_UPDATE_INDEX, 12ull * q->n_upd, q->n_upd);
+            q->u_rows_upper = q->n_upd;
+        } else if (q->n_upd) {
             DecodeSort(q, q->k_upd.p, q->k_usort.p, q->k_alt.p, q->n_upd);
             SetCounter(q, &Counters::u_dups, 0);
             LaunchCountDups(q->k_usort.p, q->n_upd, q->d_cnt, q->s);
@@ -1539,16 +1605,24 @@ cgbdsm_status cgbdsm_batch_update_global_index(cgbdsm_query* q) {
             Throw(CGBDSM_ERR_INVALID, "batch_update_global_index must follow transfer_update_index");
         if (q->split) SplitOnCommit(q);
         if (q->n_upd) {
-            LaunchUnique(q->k_usort.p, q->k_alt.p, q->n_upd, q->flags.p, q->scan_scratch.p, Cnt(q, &Counters::n_unique),
-                         q->s);
+            const bool small = q->n_upd <= kKeySetMax;
+            if (small) {
+                KeySet a = MakeKeySet(q, q->k_usort.p, q->n_upd, false, true, q->k_alt.p);
+                a.zero = q->d_cnt;
+                RunKeySet(q, a);
+            } else {
+                LaunchUnique(q->k_usort.p, q->k_alt.p, q->n_upd, q->flags.p, q->scan_scratch.p,
+                             Cnt(q, &Counters::n_unique), q->s);
+            }
             if (q->layout == CGBDSM_LAYOUT_GPMA) {
                 ReadCounters(q);
                 PmaInsert(q, q->k_alt.p, q->h_cnt->n_unique);
                 q->pma.stale = true;
             } else {
-                LaunchSegments(q->k_alt.p, Cnt(q, &Counters::n_unique), q->n_upd, q->vbits, q->flags.p, q->seg_row.p,
-                               q->seg_start.p, Cnt(q, &Counters::n_segs), q->scan_scratch.p, q->s);
-                InsertSorted(q, q->k_alt.p, Cnt(q, &Counters::n_segs), q->n_upd);
+                if (!small)
+                    LaunchSegments(q->k_alt.p, Cnt(q, &Counters::n_unique), q->n_upd, q->vbits, q->flags.p,
+                                   q->seg_row.p, q->seg_start.p, Cnt(q, &Counters::n_segs), q->scan_scratch.p, q->s);
+                InsertSorted(q, q->k_alt.p, Cnt(q, &Counters::n_segs), q->n_upd, small);
             }
         }
         q->st.batches++;

@@ -26,6 +26,7 @@
 //      merged list is written to a fresh pool block of CapFor(len) slots.
 //   3. B' values are scattered to their recorded positions.
 // Removal is an in-place ballot compaction starting at the first deleted value.
+#include "blocksort.h"
 #include "engine.h"
 #include "kernels.h"
 #include "wave.h"
@@ -75,6 +76,84 @@ __global__ void KWriteSegs(const uint64_t* __restrict__ keys, const unsigned lon
         }
         if (i == n - 1) seg_start[*n_segs] = n;
     }
+}
+
+// The steps of one small key set (at most kKeySetMax keys) in one block:
+// decode, sort, unique, list segments, and the update index (KeySet).  A batch
+// of a few thousand keys spent ten launches of one or two microseconds on each
+// of its four key sets, and most of that time between them.
+__global__ void __launch_bounds__(kBsThreads) KKeySet(KeySet a) {
+    __shared__ BsLds L;
+    const uint32_t t = threadIdx.x, n = a.n;
+    const uint64_t vmask = (1ull << a.vbits) - 1ull;
+    for (uint32_t i = t; i < n; i += kBsThreads) {
+        const uint64_t k = a.in[i];
+        const uint64_t e = k >> a.ushift, u = (k >> 32) & a.umask, v = (uint32_t)k;
+        L.key[i] = a.decode ? ((u * a.ndir + e) << a.vbits) | v : k;
+    }
+    // Rows of the last update index go first.
+    if (a.u_rec) {
+        const uint64_t old = *a.u_rows_count;
+        for (uint64_t i = t; i < old; i += kBsThreads) a.u_rec[a.u_rows[i]] = URec{0, 0};
+    }
+    if (a.zero && t == 0) a.zero->flags = a.zero->bytes = a.zero->n_long = a.zero->n_huge = 0;
+    if (a.decode) BlockSort(L, n, a.bits);
+    else __syncthreads();
+    // Four consecutive keys per thread: first of its value, first of its row.
+    uint64_t k[kBsItems];
+    uint32_t mark = 0, dups = 0;
+#pragma unroll
+    for (int j = 0; j < kBsItems; j++) {
+        const uint32_t i = t * kBsItems + j;
+        k[j] = i < n ? L.key[i] : 0ull;
+        const uint64_t prev = i > 0 && i < n ? L.key[i - 1] : ~0ull;
+        const bool fresh = i < n && (i == 0 || k[j] != prev);
+        const bool head = i < n && (i == 0 || (k[j] >> a.vbits) != (prev >> a.vbits));
+        dups += i < n && !fresh;
+        mark |= (fresh ? 1u << j : 0u) | (head ? 16u << j : 0u);
+    }
+    uint32_t total;
+    const uint32_t ex = BsScan(L, (uint32_t)__popc(mark & 15u) | ((uint32_t)__popc(mark >> 4) << 16), &total);
+    const uint32_t n_fresh = total & 0xFFFFu, n_heads = total >> 16;
+    uint32_t* s_start = &L.cnt[0][0];  // first key of each segment (kBsTile entries)
+    uint32_t f = ex & 0xFFFFu, h = ex >> 16;
+#pragma unroll
+    for (int j = 0; j < kBsItems; j++) {
+        const uint32_t i = t * kBsItems + j;
+        if (i >= n) break;
+        const bool fresh = (mark >> j) & 1u, head = (mark >> (4 + j)) & 1u;
+        const uint32_t at = a.unique ? f : i;
+        if (head) {
+            s_start[h] = at;
+            a.seg_row[h] = (uint32_t)(k[j] >> a.vbits);
+            a.seg_start[h] = at;
+            h++;
+        }
+        if (a.out && (!a.unique || fresh)) a.out[at] = k[j];
+        if (a.u_vals) a.u_vals[i] = (uint32_t)(k[j] & vmask);
+        f += fresh;
+    }
+    const uint32_t n_out = a.unique ? n_fresh : n;
+    if (a.n_dups) {
+        uint32_t all;
+        __syncthreads();  // L.sum is read above
+        (void)BsScan(L, dups, &all);
+        if (t == 0) *a.n_dups = all;
+    }
+    if (t == 0) {
+        *a.n_out = n_out;
+        *a.n_segs = n_heads;
+        a.seg_start[n_heads] = n_out;
+    }
+    if (!a.u_rec) return;
+    __syncthreads();
+    for (uint32_t i = t; i < n_heads; i += kBsThreads) {
+        const uint32_t at = s_start[i], end = i + 1 < n_heads ? s_start[i + 1] : n_out;
+        const uint32_t row = a.seg_row[i];
+        a.u_rec[row] = URec{at, end - at};
+        a.u_rows[i] = row;
+    }
+    if (t == 0) *a.u_rows_count = n_heads;
 }
 
 __device__ __forceinline__ uint32_t LowerBoundKeys(const uint64_t* __restrict__ k, uint32_t n, uint32_t v,
@@ -786,6 +865,11 @@ void LaunchDecode(const uint64_t* in, uint64_t* out, uint64_t n, uint32_t ushift
                   uint32_t vbits, hipStream_t s) {
     if (!n) return;
     KDecode<<<GridFor(n), 256, 0, s>>>(in, out, n, ushift, umask, ndir, vbits);
+}
+
+void LaunchKeySet(const KeySet& a, hipStream_t s) {
+    KKeySet<<<1, kBsThreads, 0, s>>>(a);
+    CGD_HIP(hipGetLastError());
 }
 
 void LaunchUnique(const uint64_t* in, uint64_t* out, uint64_t n, uint32_t* flags, void* scan_scratch,

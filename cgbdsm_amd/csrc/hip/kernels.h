@@ -17,6 +17,26 @@ struct EiSeedInfo {
 // index.hip
 void LaunchDecode(const uint64_t* in, uint64_t* out, uint64_t n, uint32_t ushift, uint32_t umask, uint32_t ndir,
                   uint32_t vbits, hipStream_t s);
+// One key set of at most kKeySetMax keys (n >= 1) in one launch.
+constexpr uint64_t kKeySetMax = 4096;
+struct KeySet {
+    const uint64_t* in;                  // boundary keys, or with decode = 0 sorted index keys
+    uint32_t n, decode, unique;          // unique: `out` and the segments drop repeated keys
+    uint32_t ushift, umask, ndir, vbits, bits;
+    uint64_t* out;                       // sorted index keys (may be `in`), or null
+    unsigned long long* n_out;           // keys of the segments
+    unsigned long long* n_dups;          // repeated keys, or null
+    uint32_t* seg_row;                   // lists touched: row, first key, one past the last key
+    uint64_t* seg_start;
+    unsigned long long* n_segs;
+    Counters* zero;                      // flags, bytes, n_long and n_huge zeroed here, or null
+    // Update index: the last one's rows (u_rows, *u_rows_count) cleared, then
+    // values, records and rows of this one; null u_rec: none.
+    URec* u_rec;
+    uint32_t *u_vals, *u_rows;
+    unsigned long long* u_rows_count;
+};
+void LaunchKeySet(const KeySet& a, hipStream_t s);
 void LaunchUnique(const uint64_t* in, uint64_t* out, uint64_t n, uint32_t* flags, void* scan_scratch,
                   unsigned long long* n_out_dev, hipStream_t s);
 void LaunchSegments(const uint64_t* keys, const unsigned long long* n_dev, uint64_t n_upper, uint32_t vbits,

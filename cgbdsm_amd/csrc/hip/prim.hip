@@ -6,6 +6,7 @@
 #include <chrono>
 #include <cstring>
 
+#include "blocksort.h"
 #include "engine.h"
 #include "wave.h"
 
@@ -157,136 +158,64 @@ __global__ void __launch_bounds__(256) KPublish(const uint64_t* __restrict__ src
 }
 
 // ---------------------------------------------------------------- radix sort
-constexpr int kRsThreads = 256;
-constexpr int kRsItems = 16;
-constexpr int kRsTile = kRsThreads * kRsItems;  // 4096 keys per block
+constexpr int kRsTile = kBsTile;  // keys per block
 
-__global__ void __launch_bounds__(kRsThreads) KRsHist(const uint64_t* keys, uint64_t n, uint32_t shift,
+__global__ void __launch_bounds__(kBsThreads) KRsHist(const uint64_t* keys, uint64_t n, uint32_t shift,
                                                        uint32_t* hist, uint32_t nblocks) {
     __shared__ uint32_t h[256];
-    h[threadIdx.x] = 0;
+    if (threadIdx.x < 256) h[threadIdx.x] = 0;
     __syncthreads();
     const uint64_t base = (uint64_t)blockIdx.x * kRsTile;
-#pragma unroll 4
-    for (int i = 0; i < kRsItems; i++) {
-        uint64_t idx = base + (uint64_t)i * kRsThreads + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < kBsItems; i++) {
+        uint64_t idx = base + (uint64_t)i * kBsThreads + threadIdx.x;
         if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & 255u], 1u);
     }
     __syncthreads();
-    hist[(uint64_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
+    if (threadIdx.x < 256) hist[(uint64_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
 }
 
-// Stable scatter: within a block, keys are ranked round by round (256 keys
-// per round, in index order); inside a wave the rank among equal digits comes
-// from 8 ballots, across waves from per-wave digit counts in LDS.
-__global__ void __launch_bounds__(kRsThreads) KRsScatter(const uint64_t* in, uint64_t* out, uint64_t n,
+// Stable scatter of one tile: each wave ranks its own run of 256 keys among
+// equal digits (BsRank, no block synchronisation between its rounds), the
+// waves' digit counts give the rank across them.  With 256 threads and a block
+// round of 256 keys (four barriers each) a tile took 14 us, this takes 5.
+__global__ void __launch_bounds__(kBsThreads) KRsScatter(const uint64_t* in, uint64_t* out, uint64_t n,
                                                           uint32_t shift, const uint32_t* offs, uint32_t nblocks) {
-    __shared__ uint32_t run[256];
-    __shared__ uint32_t wcnt[kRsThreads / kWave][256];
-    const int tid = threadIdx.x, w = tid / kWave;
-    const uint32_t lane = tid & (kWave - 1);
-    run[tid] = offs[(uint64_t)tid * nblocks + blockIdx.x];
+    __shared__ uint32_t cnt[kBsWaves][256];
+    const uint32_t t = threadIdx.x, w = t / kWave, lane = LaneId();
     const uint64_t base = (uint64_t)blockIdx.x * kRsTile;
-    for (int r = 0; r < kRsItems; r++) {
+    uint64_t k[kBsItems];
+    uint32_t pos[kBsItems], valid = 0;
 #pragma unroll
-        for (int ww = 0; ww < kRsThreads / kWave; ww++) wcnt[ww][tid] = 0;
-        __syncthreads();
-        const uint64_t idx = base + (uint64_t)r * kRsThreads + tid;
-        const bool valid = idx < n;
-        const uint64_t key = valid ? in[idx] : 0;
-        const uint32_t d = (uint32_t)(key >> shift) & 255u;
-        uint64_t m = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            uint64_t bb = __ballot((d >> b) & 1u);
-            m &= ((d >> b) & 1u) ? bb : ~bb;
-        }
-        const uint32_t rank = __popcll(m & LaneMaskLt(lane));
-        if (valid && rank == 0) wcnt[w][d] = __popcll(m);
-        __syncthreads();
-        if (valid) {
-            uint32_t pre = run[d];
-            for (int ww = 0; ww < w; ww++) pre += wcnt[ww][d];
-            out[pre + rank] = key;
-        }
-        __syncthreads();
-        uint32_t add = 0;
-#pragma unroll
-        for (int ww = 0; ww < kRsThreads / kWave; ww++) add += wcnt[ww][tid];
-        run[tid] += add;
-        __syncthreads();
+    for (int r = 0; r < kBsItems; r++) {
+        const uint64_t i = base + w * (kBsItems * kWave) + r * kWave + lane;
+        k[r] = i < n ? in[i] : 0ull;
+        valid |= i < n ? 1u << r : 0u;
     }
+    for (uint32_t i = t; i < (uint32_t)kBsWaves * 256; i += kBsThreads) (&cnt[0][0])[i] = 0;
+    __syncthreads();
+    BsRank<kBsItems>(cnt[w], kBsItems, k, valid, shift, pos);
+    __syncthreads();
+    if (t < 256) {
+        uint32_t all = offs[(uint64_t)t * nblocks + blockIdx.x];
+        for (int i = 0; i < kBsWaves; i++) {
+            const uint32_t c = cnt[i][t];
+            cnt[i][t] = all;
+            all += c;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kBsItems; r++)
+        if ((valid >> r) & 1u) out[cnt[w][(uint32_t)(k[r] >> shift) & 255u] + pos[r]] = k[r];
 }
 
-// Whole sort of at most one tile (kRsTile keys) in one block: the keys stay
-// in LDS across the digit passes; each pass takes the digit histogram, its
-// exclusive scan, then the same stable round-by-round scatter as KRsScatter
-// (the block's keys held in registers while LDS is rewritten).  One launch
-// instead of three per digit for the small key sets of most batches.
-__global__ void __launch_bounds__(kRsThreads) KRsSortTile(uint64_t* keys, uint32_t n, uint32_t bits) {
-    __shared__ uint64_t buf[kRsTile];
-    __shared__ uint32_t run[256];
-    __shared__ uint32_t wcnt[kRsThreads / kWave][256];
-    const int tid = threadIdx.x, w = tid / kWave;
-    const uint32_t lane = tid & (kWave - 1);
-    for (uint32_t i = tid; i < n; i += kRsThreads) buf[i] = keys[i];
-    __syncthreads();
-    for (uint32_t shift = 0; shift < bits; shift += 8) {
-        run[tid] = 0;
-        __syncthreads();
-        for (uint32_t i = tid; i < n; i += kRsThreads) atomicAdd(&run[(uint32_t)(buf[i] >> shift) & 255u], 1u);
-        __syncthreads();
-        // exclusive scan of the 256 digit counts (Hillis-Steele in LDS)
-        uint32_t v = run[tid];
-        const uint32_t own = v;
-        for (int o = 1; o < 256; o <<= 1) {
-            __syncthreads();
-            const uint32_t add = tid >= o ? run[tid - o] : 0u;
-            __syncthreads();
-            v += add;
-            run[tid] = v;
-        }
-        __syncthreads();
-        run[tid] = v - own;
-        uint64_t k[kRsItems];
-#pragma unroll
-        for (int r = 0; r < kRsItems; r++) {
-            const uint32_t idx = (uint32_t)r * kRsThreads + tid;
-            k[r] = idx < n ? buf[idx] : 0;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < kRsItems; r++) {
-#pragma unroll
-            for (int ww = 0; ww < kRsThreads / kWave; ww++) wcnt[ww][tid] = 0;
-            __syncthreads();
-            const uint32_t idx = (uint32_t)r * kRsThreads + tid;
-            const bool valid = idx < n;
-            const uint64_t key = k[r];
-            const uint32_t d = (uint32_t)(key >> shift) & 255u;
-            uint64_t m = __ballot(valid);
-#pragma unroll
-            for (int b = 0; b < 8; b++) {
-                uint64_t bb = __ballot((d >> b) & 1u);
-                m &= ((d >> b) & 1u) ? bb : ~bb;
-            }
-            const uint32_t rank = __popcll(m & LaneMaskLt(lane));
-            if (valid && rank == 0) wcnt[w][d] = __popcll(m);
-            __syncthreads();
-            if (valid) {
-                uint32_t pre = run[d];
-                for (int ww = 0; ww < w; ww++) pre += wcnt[ww][d];
-                buf[pre + rank] = key;
-            }
-            __syncthreads();
-            uint32_t add = 0;
-#pragma unroll
-            for (int ww = 0; ww < kRsThreads / kWave; ww++) add += wcnt[ww][tid];
-            run[tid] += add;
-            __syncthreads();
-        }
-    }
-    for (uint32_t i = tid; i < n; i += kRsThreads) keys[i] = buf[i];
+// Whole sort of at most one tile in one block.
+__global__ void __launch_bounds__(kBsThreads) KRsSortTile(uint64_t* keys, uint32_t n, uint32_t bits) {
+    __shared__ BsLds L;
+    for (uint32_t i = threadIdx.x; i < n; i += kBsThreads) L.key[i] = keys[i];
+    BlockSort(L, n, bits);
+    for (uint32_t i = threadIdx.x; i < n; i += kBsThreads) keys[i] = L.key[i];
 }
 
 }  // namespace
@@ -359,7 +288,7 @@ size_t RadixHistWords(uint64_t n) {
 void RadixSortU64(uint64_t* keys, uint64_t* alt, uint64_t n, uint32_t bits, uint32_t* hist, hipStream_t s) {
     if (n < 2) return;
     if (n <= (uint64_t)kRsTile) {
-        KRsSortTile<<<1, kRsThreads, 0, s>>>(keys, (uint32_t)n, bits);
+        KRsSortTile<<<1, kBsThreads, 0, s>>>(keys, (uint32_t)n, bits);
         CGD_HIP(hipGetLastError());
         return;
     }
@@ -370,9 +299,9 @@ void RadixSortU64(uint64_t* keys, uint64_t* alt, uint64_t n, uint32_t bits, uint
     uint64_t* src = keys;
     uint64_t* dst = alt;
     for (uint32_t shift = 0; shift < bits; shift += 8) {
-        KRsHist<<<nb, kRsThreads, 0, s>>>(src, n, shift, hist, nb);
+        KRsHist<<<nb, kBsThreads, 0, s>>>(src, n, shift, hist, nb);
         ScanU32(hist, hist, hn, nullptr, scan_scratch, s);
-        KRsScatter<<<nb, kRsThreads, 0, s>>>(src, dst, n, shift, hist, nb);
+        KRsScatter<<<nb, kBsThreads, 0, s>>>(src, dst, n, shift, hist, nb);
         std::swap(src, dst);
     }
     if (src != keys) CGD_HIP(hipMemcpyAsync(keys, src, n * sizeof(uint64_t), hipMemcpyDeviceToDevice, s));

@@ -1215,6 +1215,9 @@ cgbdsm_status cgbdsm_transfer_update_index(cgbdsm_query* q, int* nonempty) {
             KAdd(q, CGBDSM_K_UPDATE_INDEX, 12ull * q->n_upd, q->n_upd);
             q->u_rows_upper = q->n_upd;
         }
+        // The duplicates of the update lists are wanted when the frontier is
+        // built: on their way from here on.
+        if (q->n_upd) q->box.Request(q->d_cnt, sizeof(Counters), q->s);
         if (nonempty) *nonempty = q->u_nonempty ? 1 : 0;
         q->phase = 3;
     });
@@ -1336,7 +1339,7 @@ static const Frontier& BuildFrontier(cgbdsm_query* q) {
     // that depend on v0 alone are computed once per v0, not once per (v0, v1).
     bool seed1 = false;
     if (q->hplan.sfx_batch && q->dfs_suffix && q->hplan.cp_start == 2 && q->qv > 2) {
-        ReadCounters(q);
+        q->box.Wait(q->s);  // requested when the update index was built
         seed1 = q->h_cnt->u_dups == 0;
     }
     const uint32_t words = seed1 ? 1u : 2u;

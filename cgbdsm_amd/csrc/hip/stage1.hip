@@ -48,6 +48,7 @@
 #include <mutex>
 
 #include "api.h"
+#include "blocksort.h"
 #include "wave.h"
 
 namespace cgd {
@@ -172,6 +173,108 @@ __global__ void KGraphPairKeys(const int32_t* __restrict__ ints, uint64_t start,
         const bool del = a < 0 && b < 0 && x < (int64_t)n && y < (int64_t)n && x != y;
         dkeys[2 * i] = del ? ((uint64_t)x << vbits) | (uint64_t)y : ~0ull;
         dkeys[2 * i + 1] = del ? ((uint64_t)y << vbits) | (uint64_t)x : ~0ull;
+    }
+}
+
+// What becomes of one kind of stream pair in a small batch (KGraphBatch).
+struct GraphSet {
+    uint64_t* edges;  // the directed edges that take effect, sorted (src << vbits) | dst
+    uint32_t* seg_row;
+    uint64_t* seg_start;
+    unsigned long long *n, *n_segs;
+};
+
+// A batch of at most kBsTile / 2 pairs in one launch: block 0 takes its
+// insertions (edges absent from the graph), block 1 its deletions (edges in
+// it); each sorts its directed keys, drops repeats and those the graph decides
+// against, and lists the adjacency lists they touch.
+__global__ void __launch_bounds__(kBsThreads) KGraphBatch(const int32_t* __restrict__ ints, uint64_t start,
+                                                          uint32_t np, uint32_t n, uint32_t vbits, GView G,
+                                                          GraphSet ins, GraphSet del) {
+    __shared__ BsLds L;
+    __shared__ uint32_t s_n;
+    const uint32_t t = threadIdx.x;
+    const bool dels = blockIdx.x != 0;
+    const GraphSet out = dels ? del : ins;
+    const uint64_t vmask = (1ull << vbits) - 1ull;
+    if (t == 0) s_n = 0;
+    __syncthreads();
+    for (uint32_t i = t; i < np; i += kBsThreads) {
+        const int64_t a = ints[start + 2 * (uint64_t)i], b = ints[start + 2 * (uint64_t)i + 1];
+        const int64_t x = dels ? -a - 1 : a, y = dels ? -b - 1 : b;
+        if (x >= 0 && y >= 0 && x < (int64_t)n && y < (int64_t)n && x != y) {
+            const uint32_t at = atomicAdd(&s_n, 2u);
+            L.key[at] = ((uint64_t)x << vbits) | (uint64_t)y;
+            L.key[at + 1] = ((uint64_t)y << vbits) | (uint64_t)x;
+        }
+    }
+    __syncthreads();
+    const uint32_t nk = s_n;
+    BlockSort(L, nk, 2 * vbits);
+    // The four keys of a thread are looked up side by side: their searches'
+    // loads are in flight together.
+    uint64_t k[kBsItems];
+    const uint32_t* A[kBsItems];
+    uint32_t lo[kBsItems], hi[kBsItems], keep = 0;
+#pragma unroll
+    for (int j = 0; j < kBsItems; j++) {
+        const uint32_t i = t * kBsItems + j;
+        k[j] = i < nk ? L.key[i] : 0ull;
+        const bool fresh = i < nk && (i == 0 || k[j] != L.key[i - 1]);
+        const MRec r = G.rec[fresh ? (uint32_t)(k[j] >> vbits) : 0u];
+        A[j] = G.pool + r.off;
+        lo[j] = 0;
+        hi[j] = fresh ? r.len : 0u;
+        keep |= fresh ? 1u << j : 0u;
+    }
+    uint32_t len[kBsItems];
+#pragma unroll
+    for (int j = 0; j < kBsItems; j++) len[j] = hi[j];
+    while (lo[0] < hi[0] || lo[1] < hi[1] || lo[2] < hi[2] || lo[3] < hi[3]) {
+        uint32_t v[kBsItems];
+#pragma unroll
+        for (int j = 0; j < kBsItems; j++) v[j] = lo[j] < hi[j] ? A[j][(lo[j] + hi[j]) >> 1] : 0u;
+#pragma unroll
+        for (int j = 0; j < kBsItems; j++) {
+            const uint32_t m = (lo[j] + hi[j]) >> 1;
+            if (lo[j] < hi[j]) {
+                if (v[j] < (uint32_t)(k[j] & vmask)) lo[j] = m + 1;
+                else hi[j] = m;
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kBsItems; j++) {
+        const bool in = lo[j] < len[j] && A[j][lo[j]] == (uint32_t)(k[j] & vmask);
+        if (in != dels) keep &= ~(1u << j);
+    }
+    uint32_t total;
+    uint32_t at = BsScan(L, (uint32_t)__popc(keep), &total);
+    __syncthreads();  // the keys are in registers, L.sum is read
+#pragma unroll
+    for (int j = 0; j < kBsItems; j++)
+        if ((keep >> j) & 1u) {
+            L.key[at] = k[j];
+            out.edges[at++] = k[j];
+        }
+    __syncthreads();
+    uint32_t head = 0;
+#pragma unroll
+    for (int j = 0; j < kBsItems; j++) {
+        const uint32_t i = t * kBsItems + j;
+        if (i < total && (i == 0 || (L.key[i] >> vbits) != (L.key[i - 1] >> vbits))) head |= 1u << j;
+    }
+    uint32_t segs;
+    uint32_t h = BsScan(L, (uint32_t)__popc(head), &segs);
+    for (; head; head &= head - 1, h++) {
+        const uint32_t i = t * kBsItems + (uint32_t)__ffs(head) - 1;
+        out.seg_row[h] = (uint32_t)(L.key[i] >> vbits);
+        out.seg_start[h] = i;
+    }
+    if (t == 0) {
+        *out.n = total;
+        *out.n_segs = segs;
+        out.seg_start[segs] = total;
     }
 }
 
@@ -610,6 +713,38 @@ __global__ void KS1ClearKilled(SView S, const uint32_t* __restrict__ K, const un
     }
 }
 
+// KS1Deg and its exclusive scan for a short list, in one block: offs[n] = total.
+constexpr uint64_t kDegScanMax = 4 * kBsThreads;
+__global__ void __launch_bounds__(kBsThreads) KS1DegScan(GView G, const uint32_t* __restrict__ L, uint64_t n_upper,
+                                                         const unsigned long long* __restrict__ n_dev,
+                                                         uint64_t* __restrict__ offs) {
+    __shared__ unsigned long long s_sum[kBsWaves];
+    const uint32_t t = threadIdx.x, w = t / kWave;
+    const uint64_t n = n_dev ? *n_dev : n_upper;
+    unsigned long long v[4], mine = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) {
+        const uint64_t i = (uint64_t)t * 4 + j;
+        v[j] = i < n && i < n_upper ? G.rec[L[i] >> 4].len : 0u;
+        mine += v[j];
+    }
+    const unsigned long long incl = WaveInclusiveScan(mine);
+    if (LaneId() == kWave - 1) s_sum[w] = incl;
+    __syncthreads();
+    unsigned long long at = incl - mine, total = 0;
+    for (uint32_t i = 0; i < (uint32_t)kBsWaves; i++) {
+        at += i < w ? s_sum[i] : 0ull;
+        total += s_sum[i];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) {
+        const uint64_t i = (uint64_t)t * 4 + j;
+        if (i < n_upper) offs[i] = at;
+        at += v[j];
+    }
+    if (t == 0) offs[n_upper] = total;
+}
+
 // offs[i] = adjacency length of the vertex of pair i (before the scan); with
 // n_dev, entries from *n_dev up to n_upper are 0 (pairs the list does not hold).
 __global__ void KS1Deg(GView G, const uint32_t* __restrict__ L, uint64_t n_upper,
@@ -933,7 +1068,8 @@ struct cgbdsm_graph {
     uint64_t n_new = 0;
     DBuf<uint64_t> dele, kd;       // its deleted directed edges (sorted, as newe); deletion key scratch
     uint64_t n_dele = 0;
-    DBuf<uint64_t> k, alt, seg_start;
+    DBuf<uint64_t> k, alt, seg_start, del_seg_start;  // del_*: a small batch's deletions
+    DBuf<uint32_t> del_seg_row;
     DBuf<uint32_t> flags, seg_row, sc_val, sc_pos, hist;
     DBuf<uint8_t> scan;
     hipEvent_t ev = nullptr;       // latest batch applied on s
@@ -1048,31 +1184,33 @@ void GraphLayout(cgbdsm_graph* g, uint64_t nk) {
                      g->alt.p, g->d_cnt, g->s);
 }
 
-// Removes the sorted deleted-edge keys (all present) from the adjacency lists.
-void GraphRemove(cgbdsm_graph* g, const uint64_t* keys, uint64_t nk) {
-    if (!nk) return;
-    unsigned long long* n_s = &g->d_cnt->n_segs;
+// Touched lists of nk sorted keys into the graph's segment scratch.
+void GraphSegments(cgbdsm_graph* g, const uint64_t* keys, uint64_t nk) {
     FillU64((uint64_t*)&g->d_cnt->n_unique, nk, 1, g->s);
-    LaunchSegments(keys, &g->d_cnt->n_unique, nk, g->vbits, g->flags.p, g->seg_row.p, g->seg_start.p, n_s, g->scan.p,
-                   g->s);
-    FillU64((uint64_t*)&g->d_cnt->n_long, 0, 2, g->s);  // and n_huge
-    LaunchMergeRemove(GraphTables(g), keys, g->vbits, g->seg_row.p, g->seg_start.p, n_s, nk, g->flags.p, g->d_cnt,
-                      g->s);
+    LaunchSegments(keys, &g->d_cnt->n_unique, nk, g->vbits, g->flags.p, g->seg_row.p, g->seg_start.p,
+                   &g->d_cnt->n_segs, g->scan.p, g->s);
 }
 
-// Inserts the sorted new-edge keys into the adjacency lists (pool grows and
-// the merge is relaunched on overflow; merged lists see nothing left).
+// Removes the nk sorted deleted-edge keys (all present), whose touched lists
+// are seg_row / seg_start / *n_segs, from the adjacency lists.
+void GraphRemove(cgbdsm_graph* g, const uint64_t* keys, uint64_t nk, const uint32_t* seg_row,
+                 const uint64_t* seg_start, const unsigned long long* n_segs) {
+    if (!nk) return;
+    FillU64((uint64_t*)&g->d_cnt->n_long, 0, 2, g->s);  // and n_huge
+    LaunchMergeRemove(GraphTables(g), keys, g->vbits, seg_row, seg_start, n_segs, nk, g->flags.p, g->d_cnt, g->s);
+}
+
+// Inserts the nk sorted new-edge keys, whose touched lists are in the graph's
+// segment scratch, into the adjacency lists (pool grows and the merge is
+// relaunched on overflow; merged lists see nothing left).
 void GraphMerge(cgbdsm_graph* g, const uint64_t* keys, uint64_t nk) {
     if (!nk) return;
-    unsigned long long* n_s = &g->d_cnt->n_segs;
-    FillU64((uint64_t*)&g->d_cnt->n_unique, nk, 1, g->s);
-    LaunchSegments(keys, &g->d_cnt->n_unique, nk, g->vbits, g->flags.p, g->seg_row.p, g->seg_start.p, n_s, g->scan.p,
-                   g->s);
     for (int attempt = 0;; attempt++) {
-        FillU64((uint64_t*)&g->d_cnt->flags, 0, 1, g->s);
-        FillU64((uint64_t*)&g->d_cnt->n_long, 0, 2, g->s);  // and n_huge
-        LaunchMergeInsert(GraphTables(g), keys, g->vbits, g->seg_row.p, g->seg_start.p, n_s, nk, g->sc_val.p,
-                          g->sc_pos.p, g->flags.p, g->pool.cap, g->d_cnt, g->s);
+        WordSet ws{3, {offsetof(Counters, flags) / 8, offsetof(Counters, n_long) / 8, offsetof(Counters, n_huge) / 8},
+                   {}};
+        SetWords((uint64_t*)g->d_cnt, ws, g->s);
+        LaunchMergeInsert(GraphTables(g), keys, g->vbits, g->seg_row.p, g->seg_start.p, &g->d_cnt->n_segs, nk,
+                          g->sc_val.p, g->sc_pos.p, g->flags.p, g->pool.cap, g->d_cnt, g->s);
         GReadCounters(g);
         if (!(g->h_cnt->flags & kFlagPool)) return;
         if (attempt >= 4) Throw(CGBDSM_ERR_OOM, "graph adjacency pool overflow after growth");
@@ -1100,12 +1238,26 @@ void S1Set(cgbdsm_query* q, unsigned long long S1Cnt::*f, uint64_t v) {
     FillU64((uint64_t*)&(q->s1->d_c->*f), v, 1, q->s);
 }
 
+// Several counters in one launch.
+void S1SetMany(cgbdsm_query* q, std::initializer_list<std::pair<const unsigned long long*, uint64_t>> fv) {
+    WordSet ws{};
+    for (const auto& [f, v] : fv) {
+        ws.off[ws.n] = (uint32_t)(f - (const unsigned long long*)q->s1->d_c);
+        ws.val[ws.n++] = v;
+    }
+    SetWords((uint64_t*)q->s1->d_c, ws, q->s);
+}
+
 // Offsets of the adjacency items of list L[0..n): offs[n] = total items.
 // With n_dev, the list holds *n_dev <= n pairs (the rest count as empty).
 void S1Offsets(cgbdsm_query* q, const uint32_t* L, uint64_t n, const unsigned long long* n_dev = nullptr) {
     S1Query* S = q->s1;
     Ensure(q, S->offs, n + 1);
     Ensure(q, q->scan_scratch, ScanScratchBytes(n + 2) + 64);
+    if (n && n <= kDegScanMax) {
+        KS1DegScan<<<1, kBsThreads, 0, q->s>>>(View(S->g), L, n, n_dev, S->offs.p);
+        return;
+    }
     if (n) KS1Deg<<<Grid(n), 256, 0, q->s>>>(View(S->g), L, n, n_dev, S->offs.p);
     ScanU64(S->offs.p, S->offs.p, n, S->offs.p + n, q->scan_scratch.p, q->s);
 }
@@ -1124,8 +1276,8 @@ void S1DeletionRounds(cgbdsm_query* q, int src, uint64_t n, bool opt_only, uint3
     uint64_t rounds = 0, killed = 0;
     while (n) {
         unsigned long long* n_cur = &S->d_c->n_list[cur];
-        S1Set(q, &S1Cnt::n_died, 0);
-        S1Set(q, &S1Cnt::n_big, 0);
+        const int nxt = cur == 0 ? 1 : 0;
+        S1SetMany(q, {{&S->d_c->n_died, 0}, {&S->d_c->n_big, 0}, {&S->d_c->n_list[nxt], 0}});
         KS1Check<<<Grid(n), kThreads, 0, q->s>>>(G, S->tab, V, S->L[cur].p, n_cur, S->L[2].p, S->died_bits.p,
                                                  &S->d_c->n_died, S->L[3].p, &S->d_c->n_big);
         KS1CheckWave<<<Grid(n, kWpb, 2048), kThreads, 0, q->s>>>(G, S->tab, V, S->L[3].p, &S->d_c->n_big,
@@ -1135,8 +1287,6 @@ void S1DeletionRounds(cgbdsm_query* q, int src, uint64_t n, bool opt_only, uint3
         KS1Apply<<<Grid(n), 256, 0, q->s>>>(S->tab, V, S->L[2].p, S->died_bits.p, &S->d_c->n_died,
                                             killed_list, &S->d_c->n_killed);
         S1Offsets(q, S->L[2].p, n, &S->d_c->n_died);
-        const int nxt = cur == 0 ? 1 : 0;
-        FillU64((uint64_t*)&S->d_c->n_list[nxt], 0, 1, q->s);
         KS1Expand<<<LbGrid(q), kThreads, 0, q->s>>>(G, S->tab, V, S->L[2].p, S->offs.p, n, opt_only ? 1u : 0u,
                                                    S->L[nxt].p, &S->d_c->n_list[nxt]);
         S1Read(q);
@@ -1157,8 +1307,7 @@ uint64_t S1EmitPairs(cgbdsm_query* q, const uint32_t* Y, uint64_t n, bool both) 
     S1Query* S = q->s1;
     S1Offsets(q, Y, n);
     for (int attempt = 0;; attempt++) {
-        S1Set(q, &S1Cnt::n_keys, 0);
-        S1Set(q, &S1Cnt::ovf, 0);
+        S1SetMany(q, {{&S->d_c->n_keys, 0}, {&S->d_c->ovf, 0}});
         if (n)
             KS1EmitPairs<<<LbGrid(q), kThreads, 0, q->s>>>(View(S->g), S->tab, SV(S), Y, S->offs.p, n, both ? 1u : 0u,
                                                           q->k_ins.p, q->k_ins.cap, &S->d_c->n_keys, &S->d_c->ovf);
@@ -1177,9 +1326,7 @@ uint64_t S1EmitDelEdges(cgbdsm_query* q) {
     const cgbdsm_graph* g = S->g;
     Ensure(q, S->kd, std::max<uint64_t>(S->kd.cap, 1024));
     for (int attempt = 0;; attempt++) {
-        S1Set(q, &S1Cnt::n_keys, 0);
-        S1Set(q, &S1Cnt::ovf, 0);
-        FillU64((uint64_t*)&S->d_c->dirmask[0], 0, 2, q->s);
+        S1SetMany(q, {{&S->d_c->n_keys, 0}, {&S->d_c->ovf, 0}, {&S->d_c->dirmask[0], 0}, {&S->d_c->dirmask[1], 0}});
         KS1DelEdgeKeys<<<Grid(g->n_dele), 256, 0, q->s>>>(S->tab, SV(S), g->dele.p, g->n_dele, g->vbits, S->kd.p,
                                                           S->kd.cap, &S->d_c->n_keys, &S->d_c->ovf,
                                                           &S->d_c->dirmask[0]);
@@ -1202,8 +1349,7 @@ uint64_t S1EmitKilled(cgbdsm_query* q, uint64_t base, uint64_t nk) {
     S1Offsets(q, S->L2[1].p, nk);
     uint64_t end = base;
     for (int attempt = 0;; attempt++) {
-        FillU64((uint64_t*)&S->d_c->n_keys, base, 1, q->s);
-        S1Set(q, &S1Cnt::ovf, 0);
+        S1SetMany(q, {{&S->d_c->n_keys, base}, {&S->d_c->ovf, 0}});
         KS1EmitKilled<<<LbGrid(q), kThreads, 0, q->s>>>(View(S->g), S->tab, SV(S), S->L2[1].p, S->offs.p, nk, S->kd.p,
                                                        S->kd.cap, &S->d_c->n_keys, &S->d_c->ovf);
         S1Read(q);
@@ -1404,7 +1550,20 @@ cgbdsm_status cgbdsm_graph_apply_range(cgbdsm_graph* g, uint64_t start, uint64_t
         GEnsure(g, g->newe, std::max<uint64_t>(nk, 1));
         GEnsure(g, g->dele, std::max<uint64_t>(nk, 1));
         uint64_t n_new = 0, n_dele = 0;
-        if (np) {
+        if (np && nk <= (uint64_t)kBsTile) {
+            GEnsure(g, g->del_seg_row, nk + 1);
+            GEnsure(g, g->del_seg_start, nk + 2);
+            // Both kinds are judged against the graph before the batch, as below.
+            KGraphBatch<<<2, kBsThreads, 0, g->s>>>(
+                g->stream.p, start, (uint32_t)np, g->n, g->vbits, View(g),
+                GraphSet{g->newe.p, g->seg_row.p, g->seg_start.p, &g->d_cnt->rows_out, &g->d_cnt->n_segs},
+                GraphSet{g->dele.p, g->del_seg_row.p, g->del_seg_start.p, &g->d_cnt->u_rows, &g->d_cnt->u_dups});
+            GReadCounters(g);
+            n_new = g->h_cnt->rows_out;
+            n_dele = g->h_cnt->u_rows;
+            GraphRemove(g, g->dele.p, n_dele, g->del_seg_row.p, g->del_seg_start.p, &g->d_cnt->u_dups);
+            GraphMerge(g, g->newe.p, n_new);
+        } else if (np) {
             KGraphPairKeys<<<Grid(np), 256, 0, g->s>>>(g->stream.p, start, np, g->n, g->vbits, g->k.p, g->kd.p);
             // Both kinds are judged against the graph before the batch
             // (calig.cpp:980-998): insertions of absent edges, deletions of
@@ -1425,8 +1584,14 @@ cgbdsm_status cgbdsm_graph_apply_range(cgbdsm_graph* g, uint64_t start, uint64_t
             GReadCounters(g);
             n_new = g->h_cnt->n_segs;
             n_dele = g->h_cnt->u_rows;
-            GraphRemove(g, g->dele.p, n_dele);
-            GraphMerge(g, g->newe.p, n_new);
+            if (n_dele) {
+                GraphSegments(g, g->dele.p, n_dele);
+                GraphRemove(g, g->dele.p, n_dele, g->seg_row.p, g->seg_start.p, &g->d_cnt->n_segs);
+            }
+            if (n_new) {
+                GraphSegments(g, g->newe.p, n_new);
+                GraphMerge(g, g->newe.p, n_new);
+            }
         }
         g->n_new = n_new;
         g->n_dele = n_dele;
@@ -1560,12 +1725,11 @@ cgbdsm_status cgbdsm_calig_update(cgbdsm_query* q) {
         // deleted, the pairs from before the batch that lost one (then any
         // lit pair may die, so every lit neighbour of a death is re-checked).
         if (n_opt) CGD_HIP(hipMemcpyAsync(S->L[0].p, S->L[5].p, n_opt * 4, hipMemcpyDeviceToDevice, q->s));
-        FillU64((uint64_t*)&S->d_c->n_list[0], n_opt, 1, q->s);
+        S1SetMany(q, {{&S->d_c->n_list[0], n_opt}, {&S->d_c->n_killed, 0}});
         uint64_t n_chk = n_opt;
         if (nd) {
             KS1SeedDeleted<<<Grid(nd), 256, 0, q->s>>>(S->tab, V, g->dele.p, nd, g->vbits, S->L[0].p,
                                                        &S->d_c->n_list[0]);
-            S1Set(q, &S1Cnt::n_killed, 0);
             S1Read(q);
             n_chk = S->h_c->n_list[0];
         }
@@ -1575,8 +1739,7 @@ cgbdsm_status cgbdsm_calig_update(cgbdsm_query* q) {
             if (nk) n_kd = S1EmitKilled(q, n_kd, nk);
         }
         // 3. Survivors, new compressed ids, keys.
-        FillU64((uint64_t*)&S->d_c->n_list[3], 0, 1, q->s);
-        FillU64((uint64_t*)&S->d_c->n_list[2], n_opt, 1, q->s);
+        S1SetMany(q, {{&S->d_c->n_list[3], 0}, {&S->d_c->n_list[2], n_opt}});
         if (n_opt)
             KS1Survivors<<<Grid(n_opt), 256, 0, q->s>>>(V, S->L[5].p, &S->d_c->n_list[2], S->L[4].p,
                                                         &S->d_c->n_list[3], S->newv.p);
@@ -1590,9 +1753,7 @@ cgbdsm_status cgbdsm_calig_update(cgbdsm_query* q) {
         Ensure(q, q->k_del, cap_u);
         uint64_t n_upd = 0;
         for (int attempt = 0;; attempt++) {
-            S1Set(q, &S1Cnt::n_upd, 0);
-            S1Set(q, &S1Cnt::ovf, 0);
-            FillU64((uint64_t*)&S->d_c->dirmask[0], 0, 2, q->s);
+            S1SetMany(q, {{&S->d_c->n_upd, 0}, {&S->d_c->ovf, 0}, {&S->d_c->dirmask[0], 0}, {&S->d_c->dirmask[1], 0}});
             if (np)
                 KS1EmitUpdates<<<Grid(np), 256, 0, q->s>>>(S->tab, V, g->stream.p, g->b_start, np, g->n, q->k_upd.p,
                                                            q->k_del.p, std::min(q->k_upd.cap, q->k_del.cap),

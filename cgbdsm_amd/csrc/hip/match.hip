@@ -1077,12 +1077,21 @@ struct BxLds {
 // to end over the 64 lanes, each entry tested against j's other lists (or
 // the cached stable intersection) and its support mask, and counted per
 // sibling in LDS.  Equal to SuffixCount per sibling (identical counts).
+//
+// A step over hub lists can hold a million entries, milliseconds of one
+// wavefront's time that nobody can take over: it then ends at the sibling lane
+// `used` where kStepEntries entries are reached (kWave if all were counted),
+// and the caller goes on from there, where it can also hand out the rest.
+// The 250 000-edge batch's dense 4-vertex query spent 46 % of its wavefront
+// time waiting for such steps (38.2 ms; 22.9 ms with them cut here, 27 ms at 16384).
+constexpr uint32_t kStepEntries = 2048;
 template <bool kLean>
 __device__ __forceinline__ unsigned long long BatchSuffix(const Ctx& X, const Tables& T, uint32_t p, const uint32_t* matched,
                                           uint64_t m, uint32_t x, uint32_t* csize, uint32_t& cvalid, StabCache& sc,
-                                          BxLds& B, uint32_t& scanned, uint32_t& probes, uint32_t wmin) {
+                                          BxLds& B, uint32_t& used, uint32_t& scanned, uint32_t& probes, uint32_t wmin) {
     const uint32_t lane = LaneId();
     const uint32_t qv = X.qv;
+    used = kWave;
     const uint32_t pcls = Cls(X, p);
     unsigned long long prod = ((m >> lane) & 1ull) ? 1ull : 0ull;
     // Cheap positions first (sizes independent of the sibling, or a single
@@ -1190,9 +1199,20 @@ __device__ __forceinline__ unsigned long long BatchSuffix(const Ctx& X, const Ta
                 const uint32_t depth_v = 32u - (uint32_t)__builtin_clz(len | 1u);
                 from_src = use_sc ? (uint64_t)nmin * (depth_v + 1) < 4ull * len : nmin < len;
             }
-            const uint32_t ne = prod ? (from_src ? nmin : len) : 0u;
+            uint32_t ne = prod ? (from_src ? nmin : len) : 0u;
             const uint32_t incl = WaveInclusiveScan(ne);
-            const uint32_t total = ReadLane(incl, kWave - 1);
+            uint32_t total = ReadLane(incl, kWave - 1);
+            if (total > kStepEntries) {
+                const uint64_t over = __ballot(ne && incl > kStepEntries && incl != ne);
+                if (over) {
+                    used = (uint32_t)__builtin_ctzll(over);  // never lane 0, whose incl is ne
+                    if (lane >= used) {
+                        prod = 0;
+                        ne = 0;
+                    }
+                    total = ReadLane(incl, used - 1);
+                }
+            }
             B.base[lane] = Ls.base;
             B.app[lane] = Ls.app;
             B.bl[lane] = Ls.bl;
@@ -1616,6 +1636,7 @@ __global__ void __launch_bounds__(kThreads)
         if (lane == 0) lvl[D0] = DfsLevel{lo0, 0, 0, hi0, sel0};
         WaveSync();
         unsigned long long count = 0;
+        uint32_t bstep = kWave;  // candidates the last step at the batched level got through
         uint32_t d = Uniform(D0);
         for (;;) {
             // (every iteration at the batched level, whose steps are long:
@@ -1712,7 +1733,7 @@ __global__ void __launch_bounds__(kThreads)
             // into, so its ranges are split down to one step each (smaller
             // pieces would repeat the per-item set-up of the suffix sizes).
             const bool blev = (kLean || bsfx) && d + 1 == cps;
-            const uint32_t rmin = blev ? kWave : Q.range_min;
+            const uint32_t rmin = blev ? bstep : Q.range_min;
             if (Q.donate_min && idl_hint > 0 && limit - off >= 2 * rmin) {
                 unsigned long long h = 0, t = 0;
                 if (lane == 0) {
@@ -1725,7 +1746,8 @@ __global__ void __launch_bounds__(kThreads)
                 uint32_t parts = (uint32_t)(idl_hint < 15 ? idl_hint + 1 : 16);
                 if (parts > rem / rmin) parts = rem / rmin;
                 if (parts >= 2 && (long long)(t - h) + (long long)parts <= (long long)(Q.cap / 2)) {
-                    const uint32_t piece = ((rem + parts - 1) / parts + kWave - 1) & ~(uint32_t)(kWave - 1);
+                    uint32_t piece = (rem + parts - 1) / parts;
+                    if (rmin >= (uint32_t)kWave) piece = (piece + kWave - 1) & ~(uint32_t)(kWave - 1);
                     const uint32_t k = (rem - 1) / piece;  // donated pieces after the kept one
                     unsigned long long t0 = 0;
                     if (lane == 0) {
@@ -1771,12 +1793,13 @@ __global__ void __launch_bounds__(kThreads)
             // Last position before the product suffix: count the suffix of
             // every survivor of this step at once instead of descending.
             if (blev) {
+                bstep = kWave;
                 if (m) {
-                    count = SatAdd(count, BatchSuffix<kLean>(X, T, d, matched, m, c, s_csize[wv], cvalid, sc, s_bx[wv],
+                    count = SatAdd(count, BatchSuffix<kLean>(X, T, d, matched, m, c, s_csize[wv], cvalid, sc, s_bx[wv], bstep,
                                                       my_scanned, my_probes, wsearch ? wmin : 0u));
                     StatAdd(ws->batched, 1);
                 }
-                if (lane == 0) lvl[d].off = off + kWave;
+                if (lane == 0) lvl[d].off = off + bstep;
                 WaveSync();
                 continue;
             }

@@ -307,8 +307,10 @@ PlanLds MakePlanLds(const DevPlan& h) {
     PlanLds L{};
     for (uint32_t d = 0; d < p.qv; d++) {
         const uint32_t nbn = p.go_bni_offs[d + 1] - p.go_bni_offs[d];
+        L.vary[d] = 0xFFu;
         for (uint32_t k = 0; k < nbn && k < (uint32_t)kMaxQV; k++) {
             const uint32_t bq = p.go_bni[p.go_bni_offs[d] + k];
+            if (d >= h.cp_start && bq + 1 == h.cp_start) L.vary[d] = k;
             L.pair[d][k] = (uint16_t)(p.eidx[p.go_vs[bq] * kMaxQV + p.go_vs[d]] | (bq << 8));
         }
         L.dep_mask[d] = h.dep_mask[d];

@@ -110,6 +110,8 @@ struct PlanLds {
     uint32_t own[kMaxQE];           // edge tag ei: its two dirs, sa | sb << 8
     uint32_t dep_mask[kMaxQV];      // positions whose candidate set has position x as backward neighbour
     uint64_t vs, cls, nbn;          // per position, 4 bits each: query vertex, label class, backward neighbours
+    uint32_t vary[kMaxQV];          // suffix position: which backward neighbour is the position
+                                    // before the suffix (0xFF: none)
 };
 static_assert(sizeof(PlanLds) % 8 == 0, "copied as 64-bit words");
 

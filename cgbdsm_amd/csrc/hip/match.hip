@@ -486,6 +486,8 @@ struct Hint {
     uint32_t idle, stop;  // waves waiting for work; the launch was asked to stop
 };
 
+typedef __attribute__((address_space(3))) Hint LdsHint;
+
 // Frontier rows a block has taken and not yet given to its waves, the rows its
 // waves are done with, and the waves still taking rows.
 struct RowRange {
@@ -755,10 +757,10 @@ __device__ __forceinline__ bool InListLanes(const List& L, uint32_t c, bool act,
 // backward neighbour k1 (kNoSel: none) is given, with its pivots.
 __device__ __forceinline__ bool AcceptSelWave(const Ctx& X, const Tables& T, uint32_t d, const uint32_t* matched,
                                               uint32_t c, bool act, uint32_t skip, uint32_t k1, const List& L1,
-                                              uint32_t held1, uint32_t ninj, uint32_t& probes, uint32_t wmin) {
+                                              uint32_t held1, uint32_t inj, uint32_t& probes, uint32_t wmin) {
     bool ok = act && TileBit(X, T, Vs(X, d), c);
-    for (uint32_t i = 0; i < ninj; i++)
-        if (matched[i] == c) ok = false;
+    for (uint32_t b = inj; b; b &= b - 1)
+        if (matched[__builtin_ctz(b)] == c) ok = false;
     if (k1 != kNoSkip && __ballot(ok)) ok = InListHeld(L1, held1, c, ok, probes, wmin);
     const uint32_t nbn = Nbn(X, d);
     for (uint32_t k = 0; k < nbn; k++) {
@@ -1484,7 +1486,7 @@ __global__ void __launch_bounds__(kThreads)
         s_rows = RowRange{0, 0, 0, 0, 0, (uint32_t)kWpb};
     }
     __syncthreads();
-    volatile Hint* hint = &s_hint;
+    volatile LdsHint* hint = (volatile LdsHint*)&s_hint;
     long long t_idle0 = 0, idle_sum = 0;
     uint32_t idl_hint = 0;
     // Returns true when the kernel is asked to stop.
@@ -1765,6 +1767,8 @@ __global__ void __launch_bounds__(kThreads)
                 L1 = BnList(X, T, d, k1, matched);
                 held1 = LoadHeld(L1, wmin);
             }
+            // Only a position of the same label class can hold the candidate.
+            const uint32_t inj = (uint32_t)__ballot(lane < d && (!blev || Cls(X, lane) == Cls(X, d)));
             SfxLevel S{1, 0, kNoSkip, 0, ~0u, {nullptr, nullptr, 0, 0}};
             bool have_level = false;
             unsigned long long lsum = 0;  // per lane
@@ -1823,7 +1827,7 @@ __global__ void __launch_bounds__(kThreads)
                     my_cand++;
                 }
                 if (kLean || wsearch)
-                    ok = AcceptSelWave(X, T, d, matched, c, i < limit, sel, k1, L1, held1, d, my_probes, wmin);
+                    ok = AcceptSelWave(X, T, d, matched, c, i < limit, sel, k1, L1, held1, inj, my_probes, wmin);
                 else if (i < limit)
                     ok = AcceptSel(X, T, d, matched, c, sel, d, my_probes);
                 m = __ballot(ok);

@@ -105,6 +105,7 @@ Tables MakeTables(cgbdsm_query* q) {
     T.qe = q->qe;
     T.dv = q->dv;
     T.W = q->W;
+    T.stride = q->dv_cap;
     return T;
 }
 
@@ -132,21 +133,58 @@ void SetCounters(cgbdsm_query* q, std::initializer_list<std::pair<unsigned long 
     SetWords((uint64_t*)q->d_cnt, ws, s);
 }
 
+// The records of every direction from rows at stride `from` to rows at stride
+// `to`, in a larger buffer, the new rows zero.
+template <class T>
+void Restride(cgbdsm_query* q, DBuf<T>& b, uint32_t from, uint32_t to) {
+    const size_t n = (size_t)to * q->ndir;
+    T* np = (T*)DevAlloc(q->ctx, n * sizeof(T));
+    FillU64((uint64_t*)np, 0, n * sizeof(T) / 8, q->s);
+    if (b.p) {
+        if (from)
+            CGD_HIP(hipMemcpy2DAsync(np, (size_t)to * sizeof(T), b.p, (size_t)from * sizeof(T),
+                                     (size_t)from * sizeof(T), q->ndir, hipMemcpyDeviceToDevice, q->s));
+        CGD_HIP(hipStreamSynchronize(q->s));
+        DevFree(q->ctx, b.p, b.cap * sizeof(T));
+    }
+    b.p = np;
+    b.cap = n;
+}
+
 void GrowDV(cgbdsm_query* q, uint32_t dv) {
     if (dv > q->dv_cap) {
-        uint32_t nc = std::max<uint32_t>({dv, q->dv_cap + q->dv_cap / 2, 1024});
-        const size_t old_rows = (size_t)q->dv_cap * q->ndir, new_rows = (size_t)nc * q->ndir;
-        Ensure(q, q->m_rec, new_rows, true, old_rows);
-        Ensure(q, q->u_rec, new_rows, true, old_rows);
-        // zero the new tail (records are pairs / quads of u32)
-        FillU64((uint64_t*)(q->m_rec.p + old_rows), 0, (q->m_rec.cap - old_rows) * 2, q->s);
-        FillU64((uint64_t*)(q->u_rec.p + old_rows), 0, (q->u_rec.cap - old_rows), q->s);
-        q->dv_cap = (uint32_t)std::min<size_t>(q->m_rec.cap, q->u_rec.cap) / q->ndir;
+        const uint32_t from = q->dv_cap;
+        // (row numbers fit 32 bits: owners take at most 32 - ebits of them)
+        const uint32_t to = std::max<uint32_t>(
+            dv, (uint32_t)std::min<uint64_t>(std::max<uint64_t>(from + from / 2ull, 1024), 1ull << (32 - q->ebits)));
+        Restride(q, q->m_rec, from, to);
+        try {
+            Restride(q, q->u_rec, from, to);
+        } catch (...) {
+            // No room for U: M goes back to the old rows (through the host;
+            // the larger buffer stays).
+            if (from) {
+                std::vector<MRec> rows((size_t)from * q->ndir);
+                CGD_HIP(hipMemcpy2DAsync(rows.data(), (size_t)from * sizeof(MRec), q->m_rec.p,
+                                         (size_t)to * sizeof(MRec), (size_t)from * sizeof(MRec), q->ndir,
+                                         hipMemcpyDeviceToHost, q->s));
+                CGD_HIP(hipStreamSynchronize(q->s));
+                CGD_HIP(hipMemcpyAsync(q->m_rec.p, rows.data(), rows.size() * sizeof(MRec), hipMemcpyHostToDevice, q->s));
+                CGD_HIP(hipStreamSynchronize(q->s));
+            }
+            throw;
+        }
+        q->dv_cap = to;
+        // rows kept from one batch to the next
+        if (from && q->u_rows_upper)
+            LaunchMoveRows(q->u_rows.p, Cnt(q, &Counters::u_rows), q->u_rows_upper, from, to, q->s);
+        if (from && q->pma.nleaves)
+            LaunchPmaMoveRows(q->pma.slot.p, q->pma.lo.p, q->pma.nleaves, from, to, q->s);
     }
     if (dv > q->dv) q->dv = dv;
     q->W = (q->dv + 63) / 64;
     q->vbits = BitsFor(std::max<uint32_t>(q->dv, 2));
-    q->rbits = BitsFor((uint64_t)std::max<uint32_t>(q->dv, 1) * q->ndir);
+    q->rbits = BitsFor((uint64_t)std::max<uint32_t>(q->dv_cap, 1) * q->ndir);
 }
 
 void EnsureKeyScratch(cgbdsm_query* q, uint64_t n) {
@@ -181,7 +219,7 @@ void KAdd(cgbdsm_query* q, int cls, uint64_t bytes, uint64_t items);
 
 void DecodeSort(cgbdsm_query* q, const uint64_t* src, uint64_t* dst, uint64_t* alt, uint64_t n) {
     const int k = KBegin(q, CGBDSM_K_SORT);
-    LaunchDecode(src, dst, n, q->ushift, q->umask, q->ndir, q->vbits, q->s);
+    LaunchDecode(src, dst, n, q->ushift, q->umask, q->dv_cap, q->vbits, q->s);
     RadixSortU64(dst, alt, n, q->vbits + q->rbits, q->rs_hist.p, q->s);
     KEnd(q, k);
     KAdd(q, CGBDSM_K_SORT, 0, n);
@@ -198,7 +236,7 @@ KeySet MakeKeySet(cgbdsm_query* q, const uint64_t* in, uint64_t n, bool decode, 
     a.unique = unique;
     a.ushift = q->ushift;
     a.umask = q->umask;
-    a.ndir = q->ndir;
+    a.stride = q->dv_cap;
     a.vbits = q->vbits;
     a.bits = q->vbits + q->rbits;
     a.out = out;
@@ -577,7 +615,7 @@ void PmaExtract(cgbdsm_query* q, bool may_grow = true) {
         q->pool.cap = want;
     }
     LaunchPmaFlat(P.slot.p, P.cnt.p, P.gpos.p, P.nleaves, P.shadow.p, q->s);
-    const uint64_t rows = (uint64_t)q->dv * q->ndir;
+    const uint64_t rows = (uint64_t)q->dv_cap * q->ndir;
     LaunchPmaRows(P.shadow.p, n, q->pool.p, q->m_rec.p, rows, q->s);
     KEnd(q, k);
     KAdd(q, CGBDSM_K_GPMA_EXTRACT, 8ull * (uint64_t)P.nleaves * kPmaLeaf + 12ull * n + 16ull * rows, n);

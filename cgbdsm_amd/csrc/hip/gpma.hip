@@ -13,7 +13,7 @@
 // kernel and the window choice is a sum tree walked per dirty leaf.
 //
 // Layout: one array of nleaves * kLeaf u64 keys, key = (row << 27) | v
-// (row = owner * ndir + dir), each leaf left-packed (sorted keys, then
+// (row = dir * stride + owner), each leaf left-packed (sorted keys, then
 // kEmpty).  lo[leaf] is the leaf's separator: a key belongs to the last leaf
 // whose separator is <= the key; lo is non-decreasing and lo[0] = 0.
 #include "engine.h"
@@ -387,6 +387,15 @@ __global__ void KPmaRows(const uint64_t* __restrict__ flat, uint64_t n, uint32_t
     }
 }
 
+// A larger stride moves every row by a multiple of its direction: the keys'
+// order, and so their places, stay.
+__global__ void KPmaMoveRows(uint64_t* __restrict__ keys, uint64_t n, uint32_t from, uint32_t to) {
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t k = keys[i], row = k >> kPmaVBits;
+        if (k != kEmpty) keys[i] = k + ((row / from * (uint64_t)(to - from)) << kPmaVBits);
+    }
+}
+
 unsigned GridFor64(uint64_t n, unsigned per = 256, unsigned cap = 16384) {
     const uint64_t g = (n + per - 1) / per;
     return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(g, cap));
@@ -449,6 +458,12 @@ void LaunchPmaFlat(const uint64_t* slot, const uint32_t* cnt, const uint32_t* gp
                    hipStream_t s) {
     KPmaFlat<<<GridFor64((uint64_t)nleaves * kPmaLeaf), 256, 0, s>>>(slot, cnt, gpos, nleaves, flat);
 }
+void LaunchPmaMoveRows(uint64_t* slot, uint64_t* lo, uint32_t nleaves, uint32_t from, uint32_t to, hipStream_t s) {
+    if (!nleaves) return;
+    KPmaMoveRows<<<GridFor64((uint64_t)nleaves * kPmaLeaf), 256, 0, s>>>(slot, (uint64_t)nleaves * kPmaLeaf, from, to);
+    KPmaMoveRows<<<GridFor64(nleaves), 256, 0, s>>>(lo, nleaves, from, to);
+}
+
 void LaunchPmaRows(const uint64_t* flat, uint64_t n, uint32_t* pool, MRec* m_rec, uint64_t rows, hipStream_t s) {
     if (rows) KPmaClearRecs<<<GridFor64(rows), 256, 0, s>>>(m_rec, rows);
     if (n) KPmaRows<<<GridFor64(n), 256, 0, s>>>(flat, n, pool, m_rec);

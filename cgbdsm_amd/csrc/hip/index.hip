@@ -38,11 +38,11 @@ namespace {
 constexpr int kThreads = 256;
 
 __global__ void KDecode(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n, uint32_t ushift,
-                        uint32_t umask, uint32_t ndir, uint32_t vbits) {
+                        uint32_t umask, uint32_t stride, uint32_t vbits) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
         uint64_t k = in[i];
         uint64_t e = k >> ushift, u = (k >> 32) & umask, v = (uint32_t)k;
-        out[i] = ((u * ndir + e) << vbits) | v;
+        out[i] = ((e * stride + u) << vbits) | v;
     }
 }
 
@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(kBsThreads) KKeySet(KeySet a) {
     for (uint32_t i = t; i < n; i += kBsThreads) {
         const uint64_t k = a.in[i];
         const uint64_t e = k >> a.ushift, u = (k >> 32) & a.umask, v = (uint32_t)k;
-        L.key[i] = a.decode ? ((u * a.ndir + e) << a.vbits) | v : k;
+        L.key[i] = a.decode ? ((e * a.stride + u) << a.vbits) | v : k;
     }
     // Rows of the last update index go first.
     if (a.u_rec) {
@@ -772,6 +772,13 @@ __global__ void KClearU(URec* __restrict__ u_rec, const uint32_t* __restrict__ u
         u_rec[u_rows[i]] = URec{0, 0};
 }
 
+__global__ void KMoveRows(uint32_t* __restrict__ u_rows, const unsigned long long* __restrict__ n_dev, uint32_t from,
+                          uint32_t to) {
+    const uint64_t n = *n_dev;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+        u_rows[i] = u_rows[i] / from * to + u_rows[i] % from;
+}
+
 __global__ void KBuildUValues(const uint64_t* __restrict__ keys, uint64_t n, uint32_t vbits, uint32_t* __restrict__ vals) {
     const uint64_t vmask = (1ull << vbits) - 1ull;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
@@ -806,7 +813,7 @@ __global__ void KInitRecs(Tables T, const uint32_t* __restrict__ seg_row, const 
         const uint32_t row = seg_row[s];
         const uint32_t len = (uint32_t)(seg_start[s + 1] - seg_start[s]);
         T.m_rec[row] = MRec{offs[s], len, CapFor(len)};
-        const uint32_t e = row % T.ndir;
+        const uint32_t e = row / T.stride;
         atomicAdd(&cnt->card[e], (unsigned long long)len);
         atomicAdd(&cnt->nodes[e], 1ull);
     }
@@ -828,7 +835,7 @@ __global__ void KInitValues(Tables T, const uint64_t* __restrict__ keys, const u
 // is direction i / dv of owner i % dv, so the rows laid end to end are sorted.
 __global__ void KRowLens(Tables T, uint64_t nrows, int which, uint64_t* __restrict__ lens) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nrows; i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t r = (i % T.dv) * T.ndir + i / T.dv;
+        const uint64_t r = i / T.dv * T.stride + i % T.dv;
         lens[i] = which ? T.u_rec[r].len : T.m_rec[r].len;
     }
 }
@@ -847,7 +854,7 @@ __global__ void __launch_bounds__(kThreads) KExport(Tables T, const uint64_t* __
         const LbItem it = LbLocateFrom(offs, nrows, p0, it0, b);
         if (it0 + kWave <= b) p0 = ReadLane64(it.p, kWave - 1);
         if (!it.valid) continue;
-        const uint64_t e = it.p / T.dv, u = it.p % T.dv, r = u * T.ndir + e;
+        const uint64_t e = it.p / T.dv, u = it.p % T.dv, r = e * T.stride + u;
         const uint32_t v = which ? T.u_vals[T.u_rec[r].off + it.j] : T.pool[T.m_rec[r].off + it.j];
         out[it0 - lo + LaneId()] = (e << ushift) | (u << 32) | v;
     }
@@ -861,10 +868,10 @@ unsigned GridFor(uint64_t n, unsigned per_block = 256, unsigned cap = 8192) {
 
 }  // namespace
 
-void LaunchDecode(const uint64_t* in, uint64_t* out, uint64_t n, uint32_t ushift, uint32_t umask, uint32_t ndir,
+void LaunchDecode(const uint64_t* in, uint64_t* out, uint64_t n, uint32_t ushift, uint32_t umask, uint32_t stride,
                   uint32_t vbits, hipStream_t s) {
     if (!n) return;
-    KDecode<<<GridFor(n), 256, 0, s>>>(in, out, n, ushift, umask, ndir, vbits);
+    KDecode<<<GridFor(n), 256, 0, s>>>(in, out, n, ushift, umask, stride, vbits);
 }
 
 void LaunchKeySet(const KeySet& a, hipStream_t s) {
@@ -923,6 +930,11 @@ void LaunchClearU(URec* u_rec, const uint32_t* u_rows, const unsigned long long*
                   hipStream_t s) {
     if (!n_upper) return;
     KClearU<<<GridFor(n_upper), 256, 0, s>>>(u_rec, u_rows, n_dev);
+}
+
+void LaunchMoveRows(uint32_t* u_rows, const unsigned long long* n_dev, uint64_t n_upper, uint32_t from, uint32_t to,
+                    hipStream_t s) {
+    if (n_upper) KMoveRows<<<GridFor(n_upper), 256, 0, s>>>(u_rows, n_dev, from, to);
 }
 
 void LaunchBuildU(URec* u_rec, const uint64_t* keys, uint64_t n, uint32_t vbits, uint32_t* vals,

@@ -15,14 +15,14 @@ struct EiSeedInfo {
 };
 
 // index.hip
-void LaunchDecode(const uint64_t* in, uint64_t* out, uint64_t n, uint32_t ushift, uint32_t umask, uint32_t ndir,
+void LaunchDecode(const uint64_t* in, uint64_t* out, uint64_t n, uint32_t ushift, uint32_t umask, uint32_t stride,
                   uint32_t vbits, hipStream_t s);
 // One key set of at most kKeySetMax keys (n >= 1) in one launch.
 constexpr uint64_t kKeySetMax = 4096;
 struct KeySet {
     const uint64_t* in;                  // boundary keys, or with decode = 0 sorted index keys
     uint32_t n, decode, unique;          // unique: `out` and the segments drop repeated keys
-    uint32_t ushift, umask, ndir, vbits, bits;
+    uint32_t ushift, umask, stride, vbits, bits;
     uint64_t* out;                       // sorted index keys (may be `in`), or null
     unsigned long long* n_out;           // keys of the segments
     unsigned long long* n_dups;          // repeated keys, or null
@@ -52,6 +52,9 @@ void LaunchMergeInsert(const Tables& T, const uint64_t* keys, uint32_t vbits, co
 void LaunchMergeRemove(const Tables& T, const uint64_t* keys, uint32_t vbits, const uint32_t* seg_row,
                        const uint64_t* seg_start, const unsigned long long* n_segs, uint64_t n_upper,
                        uint32_t* long_segs, Counters* cnt, hipStream_t s);
+// Rows u_rows[0, *n_dev) from stride `from` to stride `to` (GrowDV).
+void LaunchMoveRows(uint32_t* u_rows, const unsigned long long* n_dev, uint64_t n_upper, uint32_t from, uint32_t to,
+                    hipStream_t s);
 void LaunchClearU(URec* u_rec, const uint32_t* u_rows, const unsigned long long* n_dev, uint64_t n_upper,
                   hipStream_t s);
 void LaunchBuildU(URec* u_rec, const uint64_t* keys, uint64_t n, uint32_t vbits, uint32_t* vals,
@@ -165,6 +168,8 @@ void LaunchPmaDelete(const uint64_t* dkeys, const uint32_t* dleaf, uint64_t n, u
                      hipStream_t s);
 void LaunchPmaFlat(const uint64_t* slot, const uint32_t* cnt, const uint32_t* gpos, uint32_t nleaves, uint64_t* flat,
                    hipStream_t s);
+// The keys of the array from row stride `from` to stride `to`: their order stays.
+void LaunchPmaMoveRows(uint64_t* slot, uint64_t* lo, uint32_t nleaves, uint32_t from, uint32_t to, hipStream_t s);
 void LaunchPmaRows(const uint64_t* flat, uint64_t n, uint32_t* pool, MRec* m_rec, uint64_t rows, hipStream_t s);
 
 }  // namespace cgd

@@ -35,7 +35,7 @@ __global__ void KMaskSeed(Tables T, const uint32_t* __restrict__ u_rows, const u
     const uint64_t n = *n_dev;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t row = u_rows[i];
-        const uint32_t e = row % T.ndir, u = row / T.ndir;
+        const uint32_t e = row / T.stride, u = row % T.stride;
         const uint64_t bit = 1ull << (u & 63);
         for (uint32_t k = 0; k < info.n; k++) {
             const uint32_t ei = info.ei[k];
@@ -69,7 +69,7 @@ __global__ void __launch_bounds__(256) KMaskDepth(Tables T, uint32_t d, EiList L
             const bool up_vis = p.dir_to_edge[bwd] <= ei;
             bool sat = false;
             if (ok) {
-                const uint64_t r = (uint64_t)v * T.ndir + bwd;
+                const uint64_t r = (uint64_t)bwd * T.stride + v;
                 const MRec m = T.m_rec[r];
                 const uint32_t* L0 = T.pool + m.off;
                 uint32_t j = 0;

@@ -133,7 +133,7 @@ __device__ __forceinline__ MRec LdMRec(const MRec* p) {
 // with U appended when that direction's undirected edge precedes the tag.
 __device__ __forceinline__ List Resolve(const Ctx& X, const Tables& T, uint32_t dir, uint32_t owner) {
     List L;
-    const uint64_t r = (uint64_t)owner * T.ndir + dir;
+    const uint64_t r = (uint64_t)dir * T.stride + owner;
     if (dir == X.sa || dir == X.sb) {
         const URec u = LdURec(T.u_rec + r);
         L.base = T.u_vals + u.off;
@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(kThreads) KSeed(Tables T, EiList EL, uint32_t*
         }
         if (v >= T.dv) m0 = 0;
         if (!__ballot(m0 != 0)) continue;
-        const uint64_t r = (uint64_t)v * T.ndir + idx;
+        const uint64_t r = (uint64_t)idx * T.stride + v;
         uint32_t lm = 0, lu = 0, ou = 0;
         uint64_t om = 0;
         if (m0 & use_m) {
@@ -339,7 +339,7 @@ __global__ void __launch_bounds__(kThreads) KSeed1(Tables T, EiList EL, uint32_t
         }
         if (v >= T.dv) m0 = 0;
         if (!__ballot(m0 != 0)) continue;
-        const uint64_t r = (uint64_t)v * T.ndir + idx;
+        const uint64_t r = (uint64_t)idx * T.stride + v;
         uint64_t emit = 0;
         if ((m0 & use_m) && LdMRec(T.m_rec + r).len) emit |= m0 & use_m;
         if ((m0 & use_u) && LdURec(T.u_rec + r).len) emit |= m0 & use_u;
@@ -549,7 +549,7 @@ __device__ __forceinline__ bool InList(const List& L, uint32_t c, uint32_t& prob
 // (Resolve with a tag of each lane's own).
 __device__ __forceinline__ List ResolveTag(LdsPlan* L, const Tables& T, uint32_t ei, uint32_t dir, uint32_t owner) {
     List l{nullptr, nullptr, 0, 0};
-    const uint64_t r = (uint64_t)owner * T.ndir + dir;
+    const uint64_t r = (uint64_t)dir * T.stride + owner;
     const uint32_t own = L->own[ei];
     const bool mine = dir == (own & 0xFFu) || dir == own >> 8;
     const bool app = (L->app[ei][dir >> 6] >> (dir & 63u)) & 1ull;

@@ -1138,7 +1138,7 @@ Tables GraphTables(cgbdsm_graph* g) {
     T.m_rec = g->rec.p;
     T.pool = g->pool.p;
     T.ndir = 1;
-    T.dv = g->n;
+    T.dv = T.stride = g->n;
     return T;
 }
 

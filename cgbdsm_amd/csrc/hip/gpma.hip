@@ -311,7 +311,14 @@ __global__ void KPmaFinalize(const uint32_t* __restrict__ win_of, const PmaWin* 
 // Deletes: one wavefront per leaf that holds delete keys (a wave per sorted
 // delete key, which goes on only when its key is the first of its leaf), so
 // that scattered deletes compact their leaves in parallel rather than up to
-// 64 leaves one after another per wave.
+// 64 leaves one after another per wave.  A leaf takes two round trips: its
+// keys, eight per lane, and its delete keys, 64 per round, each compared with
+// the keys held (a leaf mostly has a few; finding their end and every key by
+// binary search took over twenty: 214 -> 107 us per call on the 250 000-edge batch).
+constexpr uint32_t kLeafRounds = kPmaLeaf / kWave;
+// Up to this many delete keys are compared one by one (8 comparisons each);
+// more of them cost less by rank (8 times 7 shuffles for 64).
+constexpr uint32_t kLeafFew = 16;
 __global__ void __launch_bounds__(256) KPmaDelete(const uint64_t* __restrict__ dkeys, const uint32_t* __restrict__ dleaf,
                                                   uint64_t n, uint64_t* __restrict__ slot, uint32_t* __restrict__ cnt) {
     const uint32_t lane = LaneId();
@@ -319,38 +326,46 @@ __global__ void __launch_bounds__(256) KPmaDelete(const uint64_t* __restrict__ d
     for (uint64_t h = (uint64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; h < n; h += nw) {
         const uint32_t leaf = Uniform(dleaf[h]);
         if (h > 0 && Uniform(dleaf[h - 1]) == leaf) continue;
-        uint64_t e = h;  // end of this leaf's delete keys
-        {
-            uint64_t lo = h, hi = n;
-            while (lo < hi) {
-                const uint64_t m = (lo + hi) >> 1;
-                if (dleaf[m] <= leaf) lo = m + 1;
-                else hi = m;
-            }
-            e = lo;
-        }
         uint64_t* L = slot + (uint64_t)leaf * kPmaLeaf;
         const uint32_t c = Uniform(cnt[leaf]);
-        uint32_t w = 0;
-        for (uint32_t k = 0; k < c; k += kWave) {
-            const uint32_t t = k + lane;
-            const bool valid = t < c;
-            const uint64_t key = valid ? L[t] : kEmpty;
-            bool del = false;
-            if (valid) {
-                const uint64_t p = h + LowerBoundU64(dkeys + h, e - h, key);
-                del = p < e && dkeys[p] == key;
+        uint64_t key[kLeafRounds];
+        uint32_t del = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kLeafRounds; j++) key[j] = j * kWave + lane < c ? L[j * kWave + lane] : kEmpty;
+        for (uint64_t d0 = h; d0 < n; d0 += kWave) {
+            const bool mine = d0 + lane < n && dleaf[d0 + lane] == leaf;
+            const uint64_t dk = mine ? dkeys[d0 + lane] : kEmpty;
+            const uint32_t k = (uint32_t)__popcll(__ballot(mine));
+            if (k <= kLeafFew) {
+                for (uint32_t i = 0; i < k; i++) {
+                    const uint64_t x = ReadLane64(dk, (int)i);
+#pragma unroll
+                    for (uint32_t j = 0; j < kLeafRounds; j++) del |= key[j] == x ? 1u << j : 0u;
+                }
+            } else {
+                // (sorted, kEmpty past the end: each key's rank by shuffles)
+#pragma unroll
+                for (uint32_t j = 0; j < kLeafRounds; j++) {
+                    uint32_t pos = 0;
+#pragma unroll
+                    for (uint32_t step = 32; step >= 1; step >>= 1)
+                        if ((uint64_t)__shfl((unsigned long long)dk, (int)(pos + step - 1), kWave) < key[j]) pos += step;
+                    const uint64_t at = __shfl((unsigned long long)dk, (int)pos, kWave);
+                    del |= at == key[j] && at != kEmpty ? 1u << j : 0u;
+                }
             }
-            const bool keep = valid && !del;
+            if (k < (uint32_t)kWave) break;
+        }
+        uint32_t w = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kLeafRounds; j++) {
+            const bool keep = j * kWave + lane < c && !((del >> j) & 1u);
             const uint64_t m = __ballot(keep);
-            WaveSync();
-            if (keep) L[w + RankBelow(m)] = key;
-            WaveSync();
+            if (keep) L[w + RankBelow(m)] = key[j];
             w += (uint32_t)__popcll(m);
         }
         for (uint32_t t = w + lane; t < c; t += kWave) L[t] = kEmpty;
         if (lane == 0) cnt[leaf] = w;
-        WaveSync();
     }
 }
 
@@ -370,20 +385,45 @@ __global__ void KPmaClearRecs(MRec* __restrict__ m_rec, uint64_t rows) {
         m_rec[r] = MRec{0, 0, 0};
 }
 
-// Flat keys -> list values in the pool and one record per non-empty row
-// (written by the thread holding the row's last key).
-__global__ void KPmaRows(const uint64_t* __restrict__ flat, uint64_t n, uint32_t* __restrict__ pool,
-                         MRec* __restrict__ m_rec) {
+// Flat keys -> list values in the pool and one record per non-empty row,
+// written by the lane holding the row's last key.  The row's first key is in
+// the same 64 keys or found by steps that double backwards from them (a binary
+// search over all keys took 25 dependent loads for every row: 292 -> 170 us per
+// call on the 250 000-edge batch).
+__global__ void __launch_bounds__(256) KPmaRows(const uint64_t* __restrict__ flat, uint64_t n,
+                                                uint32_t* __restrict__ pool, MRec* __restrict__ m_rec) {
     const uint64_t vmask = (1ull << kPmaVBits) - 1ull;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t k = flat[i];
-        pool[i] = (uint32_t)(k & vmask);
+    const uint32_t lane = LaneId();
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    const uint64_t t0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint64_t b = t0 - lane; b < n; b += stride) {  // the wave's 64 keys: all lanes stay for the ballot
+        const uint64_t i = b + lane;
+        const bool valid = i < n;
+        const uint64_t k = valid ? flat[i] : kEmpty;
+        if (valid) pool[i] = (uint32_t)(k & vmask);
         const uint64_t row = k >> kPmaVBits;
-        if (i + 1 == n || (flat[i + 1] >> kPmaVBits) != row) {
-            const uint64_t start = LowerBoundU64(flat, i + 1, row << kPmaVBits);
-            const uint32_t len = (uint32_t)(i + 1 - start);
-            m_rec[row] = MRec{start, len, len};
+        const bool head = valid && (i == 0 || (flat[i - 1] >> kPmaVBits) != row);
+        const uint64_t heads = __ballot(head) & (~0ull >> (63 - lane));  // at or below this lane
+        if (!valid || (i + 1 < n && (flat[i + 1] >> kPmaVBits) == row)) continue;
+        uint64_t start;
+        if (heads) {
+            start = b + (63u - (uint32_t)__builtin_clzll(heads));
+        } else {
+            // the row's keys reach below b: lo is below the row (or 0), hi in it
+            uint64_t lo = 0, hi = b, step = 1;
+            while (step <= hi) {
+                const uint64_t at = hi - step;
+                if ((flat[at] >> kPmaVBits) != row) {
+                    lo = at + 1;
+                    break;
+                }
+                hi = at;
+                step <<= 1;
+            }
+            start = lo + LowerBoundU64(flat + lo, hi - lo, row << kPmaVBits);
         }
+        const uint32_t len = (uint32_t)(i + 1 - start);
+        m_rec[row] = MRec{start, len, len};
     }
 }
 

@@ -33,11 +33,13 @@
 #include "wave.h"
 
 // Resident blocks per CU (= waves per SIMD) of the final DFS, a build-time
-// tuning knob.  Its loops' carried values are scalar (87 to 92 VGPRs, nothing
+// tuning knob.  Its loops' carried values are scalar (66 to 96 VGPRs, nothing
 // spilled to memory); what decides is latency hiding against the LDS left for
 // the stable-intersection cache and the waves that share the work queue's
-// lines.  DFS ms per launch at 3 / 4 / 5 blocks: scale-21 four-query batch 152
-// / 133 / 126; scale-20 dense 6-vertex query 29.2 / 23.9 / 21.3; 8-query mix
+// lines.  DFS ms per launch at 3 / 4 / 5 blocks, when every step still looked
+// its lists up (6 blocks: 5-vertex path 7 % and dense 6-vertex query 8 % faster,
+// walk batch 12 % and dense 5-vertex query 3 % slower): scale-21 four-query batch
+// 152 / 133 / 126; scale-20 dense 6-vertex query 29.2 / 23.9 / 21.3; 8-query mix
 // 25.9 / 21.3 / 18.7; a 50 000-edge 5-vertex walk batch 4.26 / 4.07 / 4.35.
 #ifndef CGD_DFS_BLOCKS
 #define CGD_DFS_BLOCKS 5

@@ -1234,10 +1234,6 @@ void S1Read(cgbdsm_query* q) {
     q->s1->box.Wait(q->s);
 }
 
-void S1Set(cgbdsm_query* q, unsigned long long S1Cnt::*f, uint64_t v) {
-    FillU64((uint64_t*)&(q->s1->d_c->*f), v, 1, q->s);
-}
-
 // Several counters in one launch.
 void S1SetMany(cgbdsm_query* q, std::initializer_list<std::pair<const unsigned long long*, uint64_t>> fv) {
     WordSet ws{};

@@ -1507,8 +1507,8 @@ cgbdsm_status cgbdsm_graph_destroy(cgbdsm_graph* g) {
         GRelease(c, g->pool);
         GRelease(c, g->stream);
         GRelease(c, g->newe);
-        for (auto* b : {&g->k, &g->alt, &g->seg_start, &g->dele, &g->kd}) GRelease(c, *b);
-        for (auto* b : {&g->flags, &g->seg_row, &g->sc_val, &g->sc_pos, &g->hist}) GRelease(c, *b);
+        for (auto* b : {&g->k, &g->alt, &g->seg_start, &g->del_seg_start, &g->dele, &g->kd}) GRelease(c, *b);
+        for (auto* b : {&g->flags, &g->seg_row, &g->del_seg_row, &g->sc_val, &g->sc_pos, &g->hist}) GRelease(c, *b);
         GRelease(c, g->scan);
         if (g->d_cnt) DevFree(c, g->d_cnt, sizeof(Counters));
         if (g->ev) (void)hipEventDestroy(g->ev);

@@ -64,3 +64,17 @@ def test_graph_batch(pairs):
     g.close()
     want.close()
     eng.close()
+
+
+@pytest.mark.parametrize("pairs", [16, 5000])
+def test_closed_graph_gives_its_memory_back(pairs):
+    print(f"case graph memory {pairs}", flush=True)
+    rng = np.random.default_rng(pairs)
+    eng = Engine(0)
+    held = eng.memory()[0]
+    g = eng.graph(rng.integers(0, 2, 900).astype(np.int32), rng.integers(0, 900, (4000, 2)))
+    g.set_stream(rng.integers(0, 900, (pairs, 2)))
+    g.apply_range(0, 2 * pairs)
+    g.close()
+    assert eng.memory()[0] == held
+    eng.close()

@@ -84,6 +84,9 @@ struct cgbdsm_query {
     // always held one entry per lane when on).  Default 64.
     uint32_t dfs_wsearch = 6;
     double deadline_ms = 120000;  // safety net; cgbdsm_set_deadline_ms(0) disables
+    // Scratch that is being read or written (kScratch* bits): the rest of it
+    // is given back when an allocation fails (QueryAlloc).
+    uint32_t scratch_used = 0;
     StealItem* steal_items = nullptr;
     unsigned long long* steal_seq = nullptr;
     uint64_t steal_cap = 1ull << 20;
@@ -172,11 +175,21 @@ cgbdsm_status Guard(F&& f) {
 void CheckCanStage(const cgbdsm_query* q);
 void* DevAlloc(cgbdsm_ctx* ctx, size_t bytes);
 void DevFree(cgbdsm_ctx* ctx, void* p, size_t bytes);
+// DevAlloc for a query, which first gives back the scratch it does not need
+// when there is no room.
+void* QueryAlloc(cgbdsm_query* q, size_t bytes);
+enum : uint32_t { kScratchLevels = 1, kScratchExport = 2 };
+struct ScratchUse {
+    cgbdsm_query* q;
+    uint32_t bit;
+    ScratchUse(cgbdsm_query* query, uint32_t b) : q(query), bit(b) { q->scratch_used |= bit; }
+    ~ScratchUse() { q->scratch_used &= ~bit; }
+};
 template <class T>
 void Ensure(cgbdsm_query* q, DBuf<T>& b, size_t n, bool keep = false, size_t keep_n = 0) {
     if (n <= b.cap) return;
     size_t nc = std::max<size_t>({n, b.cap + b.cap / 2, 1024});
-    T* np = (T*)DevAlloc(q->ctx, nc * sizeof(T));
+    T* np = (T*)QueryAlloc(q, nc * sizeof(T));
     if (keep && b.p && keep_n)
         CGD_HIP(hipMemcpyAsync(np, b.p, std::min(keep_n, b.cap) * sizeof(T), hipMemcpyDeviceToDevice, q->s));
     if (b.p) {

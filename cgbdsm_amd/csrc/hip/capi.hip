@@ -92,6 +92,37 @@ void DevFree(cgbdsm_ctx* ctx, void* p, size_t bytes) {
     }
 }
 
+// Scratch kept from one call to the next and not in use now: the export's,
+// the BFS levels' and the frontier buffer that holds no rows to be counted.
+static bool GiveBack(cgbdsm_query* q) {
+    size_t bytes = 0;
+    auto drop = [&](auto& b) {
+        bytes += b.cap;
+        Release(q, b);
+    };
+    if (q->s) CGD_HIP(hipStreamSynchronize(q->s));
+    if (!(q->scratch_used & kScratchExport)) {
+        drop(q->exp_offs);
+        drop(q->exp_keys);
+    }
+    if (!(q->scratch_used & kScratchLevels)) {
+        drop(q->ext_offs);
+        drop(q->ext_sel);
+        for (uint32_t i = 0; i < 2; i++)
+            if (!q->fr_ready || q->fr.cur != i) drop(q->front[i]);
+    }
+    return bytes != 0;
+}
+
+void* QueryAlloc(cgbdsm_query* q, size_t bytes) {
+    try {
+        return DevAlloc(q->ctx, bytes);
+    } catch (const ApiError& e) {
+        if (e.code != CGBDSM_ERR_OOM || !GiveBack(q)) throw;
+    }
+    return DevAlloc(q->ctx, bytes);
+}
+
 Tables MakeTables(cgbdsm_query* q) {
     Tables T;
     T.P = q->d_plan;
@@ -138,7 +169,7 @@ void SetCounters(cgbdsm_query* q, std::initializer_list<std::pair<unsigned long 
 template <class T>
 void Restride(cgbdsm_query* q, DBuf<T>& b, uint32_t from, uint32_t to) {
     const size_t n = (size_t)to * q->ndir;
-    T* np = (T*)DevAlloc(q->ctx, n * sizeof(T));
+    T* np = (T*)QueryAlloc(q, n * sizeof(T));
     FillU64((uint64_t*)np, 0, n * sizeof(T) / 8, q->s);
     if (b.p) {
         if (from)
@@ -258,7 +289,7 @@ void GrowPool(cgbdsm_query* q, uint64_t min_cap) {
     ReadCounters(q);
     uint64_t used = q->h_cnt->pool_top;
     uint64_t nc = std::max<uint64_t>({min_cap, q->pool.cap * 2, used + (64ull << 20)});
-    uint32_t* np = (uint32_t*)DevAlloc(q->ctx, nc * sizeof(uint32_t));
+    uint32_t* np = (uint32_t*)QueryAlloc(q, nc * sizeof(uint32_t));
     if (q->pool.p && used)
         CGD_HIP(hipMemcpyAsync(np, q->pool.p, std::min<uint64_t>(used, q->pool.cap) * sizeof(uint32_t),
                                hipMemcpyDeviceToDevice, q->s));
@@ -611,7 +642,7 @@ void PmaExtract(cgbdsm_query* q, bool may_grow = true) {
         }
         Release(q, q->pool);
         const uint64_t want = n + n / 2 + (16ull << 20);
-        q->pool.p = (uint32_t*)DevAlloc(q->ctx, want * sizeof(uint32_t));
+        q->pool.p = (uint32_t*)QueryAlloc(q, want * sizeof(uint32_t));
         q->pool.cap = want;
     }
     LaunchPmaFlat(P.slot.p, P.cnt.p, P.gpos.p, P.nleaves, P.shadow.p, q->s);
@@ -633,7 +664,7 @@ void PmaRebuild(cgbdsm_query* q, const uint64_t* extra, uint64_t n_extra) {
     const uint64_t n_old = q->h_cnt->n_segs, n = n_old + n_extra;
     // The extra keys live in P.keys2: copy them out before P.keys grows.
     DBuf<uint64_t> tmp;
-    tmp.p = (uint64_t*)DevAlloc(q->ctx, std::max<uint64_t>(n_extra, 1) * sizeof(uint64_t));
+    tmp.p = (uint64_t*)QueryAlloc(q, std::max<uint64_t>(n_extra, 1) * sizeof(uint64_t));
     tmp.cap = std::max<uint64_t>(n_extra, 1);
     if (n_extra) CGD_HIP(hipMemcpyAsync(tmp.p, extra, n_extra * 8, hipMemcpyDeviceToDevice, q->s));
     Ensure(q, P.keys, std::max<uint64_t>(n, 1));
@@ -733,7 +764,7 @@ void IndexInitDevice(cgbdsm_query* q, uint64_t n, uint32_t dv_count, uint32_t* c
     const uint64_t want = std::max<uint64_t>(total + total / 2 + (16ull << 20), 1ull << 24);
     if (q->pool.cap < want) {
         Release(q, q->pool);
-        q->pool.p = (uint32_t*)DevAlloc(q->ctx, want * sizeof(uint32_t));
+        q->pool.p = (uint32_t*)QueryAlloc(q, want * sizeof(uint32_t));
         q->pool.cap = want;
     }
     LaunchInitLayout(MakeTables(q), q->k_ins.p, Cnt(q, &Counters::n_unique), n, q->vbits, q->flags.p,
@@ -1378,6 +1409,7 @@ static constexpr uint64_t kExtendWords = 16ull << 20;
 // on another query's stream to wait on.
 static const Frontier& BuildFrontier(cgbdsm_query* q) {
     if (q->fr_ready) return q->fr;
+    const ScratchUse in_use(q, kScratchLevels);
     const EiList L = ActiveEdges(q);
     SetCounters(q, {{&Counters::rows_out, 0}, {&Counters::flags, 0}, {&Counters::tuples, 0}}, q->s);
     const Tables T = MakeTables(q);
@@ -1437,11 +1469,12 @@ static const Frontier& BuildFrontier(cgbdsm_query* q) {
         uint64_t want_rows = fixed_cap ? q->frontier_cap_rows
                              : wide    ? std::min<uint64_t>(n * 4, kExtendWords / (depth + 1))
                                        : std::min<uint64_t>(std::max<uint64_t>(n * 64, 1u << 20), 1ull << 28);
-        bool done = false;
+        bool done = false, have_scratch = false;
         try {
             Ensure(q, q->ext_offs, n + 1);
             Ensure(q, q->ext_sel, n);
             Ensure(q, q->scan_scratch, ScanScratchBytes(n + 1) + 64);
+            have_scratch = true;
             for (int attempt = 0;; attempt++) {
                 Ensure(q, q->front[cur ^ 1], want_rows * (depth + 1));
                 SetCounters(q, {{&Counters::rows_out, 0}, {&Counters::flags, 0}}, q->s);
@@ -1461,9 +1494,18 @@ static const Frontier& BuildFrontier(cgbdsm_query* q) {
                 if (!wide || attempt || want_rows * (depth + 1) > kExtendWords) break;
             }
         } catch (const ApiError& e) {
-            if (e.code != CGBDSM_ERR_OOM || !wide) throw;
+            if (e.code != CGBDSM_ERR_OOM || (!wide && have_scratch)) throw;
         }
-        if (!done) break;  // keep this level, count it by DFS
+        if (!done) {  // keep this level, count it by DFS
+            if (wide) {
+                CGD_HIP(hipStreamSynchronize(q->s));  // (without memory: the grouping may still read the seeds)
+                Release(q, q->ext_offs);
+                Release(q, q->ext_sel);
+                if (cur) Release(q, q->front[0]);  // (the seeds' buffer grows to what they need)
+                else Release(q, q->front[1]);
+            }
+            break;
+        }
         n = q->h_cnt->rows_out;
         cur ^= 1;
         depth++;
@@ -1627,7 +1669,7 @@ cgbdsm_status cgbdsm_match_tuples(cgbdsm_query* q, uint32_t* out, uint64_t cap, 
     return Guard([&] {
         if (!q || q->phase != 5) Throw(CGBDSM_ERR_INVALID, "match_tuples must follow matching");
         const uint64_t words = (q->qv + 1) * std::max<uint64_t>(cap, 1);
-        uint32_t* d_out = (uint32_t*)DevAlloc(q->ctx, words * 4);
+        uint32_t* d_out = (uint32_t*)QueryAlloc(q, words * 4);
         try {
             SetCounter(q, &Counters::tuples, 0);
             SetCounter(q, &Counters::flags, 0);
@@ -1745,6 +1787,7 @@ cgbdsm_status cgbdsm_index_export(cgbdsm_query* q, int which, uint64_t* out, uin
     return Guard([&] {
         if (!q) Throw(CGBDSM_ERR_INVALID, "null query");
         if (which == 0 && q->layout == CGBDSM_LAYOUT_GPMA && q->pma.stale) PmaExtract(q);
+        const ScratchUse in_use(q, kScratchExport);
         const uint64_t nrows = (uint64_t)q->dv * q->ndir;
         // The keys come in ascending order from the device, kExportKeys at a
         // time: no sort on the host.  Scratch of up to kExportKeep bytes each

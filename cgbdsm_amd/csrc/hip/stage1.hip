@@ -1622,7 +1622,7 @@ cgbdsm_status cgbdsm_calig_attach(cgbdsm_query* q, cgbdsm_graph* g, const int32_
             S->tab = MakeQTab(q, qlabels);
             S->batches = g->batches;
             const uint32_t n = g->n;
-            S->d_c = (S1Cnt*)DevAlloc(q->ctx, sizeof(S1Cnt));
+            S->d_c = (S1Cnt*)QueryAlloc(q, sizeof(S1Cnt));
             S->box.Alloc(sizeof(S1Cnt));
             S->h_c = (S1Cnt*)S->box.data();
             FillU64((uint64_t*)S->d_c, 0, sizeof(S1Cnt) / 8, q->s);
@@ -1839,7 +1839,7 @@ cgbdsm_status cgbdsm_calig_export_lit(cgbdsm_query* q, uint32_t* li, uint32_t n)
     return Guard([&] {
         if (!q || !q->s1 || !li) Throw(CGBDSM_ERR_INVALID, "null argument or no device Stage 1");
         if (n != q->s1->g->n) Throw(CGBDSM_ERR_INVALID, "n must be the graph's vertex count");
-        uint32_t* d = (uint32_t*)DevAlloc(q->ctx, (size_t)n * 4);
+        uint32_t* d = (uint32_t*)QueryAlloc(q, (size_t)n * 4);
         KS1ExportLit<<<Grid(n), 256, 0, q->s>>>(q->s1->vstate.p, n, d);
         CGD_HIP(hipMemcpyAsync(li, d, (size_t)n * 4, hipMemcpyDeviceToHost, q->s));
         CGD_HIP(hipStreamSynchronize(q->s));

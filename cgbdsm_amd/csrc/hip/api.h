@@ -34,10 +34,12 @@ struct cgbdsm_ctx {
 constexpr uint64_t kBfsRowLimit = 65536;  // default of cgbdsm_set_match_params
 
 // Rows left for the final DFS after seeds and BFS levels: count, depth and
-// which of the two frontier buffers holds them.
+// which of the two frontier buffers holds them; and what the levels above the
+// row limit took of the deadline (until a count has been charged with it).
 struct Frontier {
     uint64_t n = 0;
     uint32_t depth = 0, cur = 0;
+    double ms = 0;
 };
 
 struct cgbdsm_query {
@@ -84,6 +86,10 @@ struct cgbdsm_query {
     // always held one entry per lane when on).  Default 64.
     uint32_t dfs_wsearch = 6;
     double deadline_ms = 120000;  // safety net; cgbdsm_set_deadline_ms(0) disables
+    double spent_ms = 0;          // of it, by the frontier of the count that runs
+    // Rows at a depth from which a BFS level above the row limit is not tried
+    // (0: no limit): it did not fit lately.
+    uint64_t wide_from[kMaxQV] = {};
     // Scratch that is being read or written (kScratch* bits): the rest of it
     // is given back when an allocation fails (QueryAlloc).
     uint32_t scratch_used = 0;

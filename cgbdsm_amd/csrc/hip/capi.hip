@@ -469,6 +469,46 @@ StealQueue MakeSteal(cgbdsm_query* q, bool donate) {
     return Q;
 }
 
+// Waits for the counters requested last on q's stream.  The host watches for
+// them without sleeping at first (a batch's launch is often over in 0.1 ms),
+// then for a sixteenth of the time waited so far, 200 us at most.  Past
+// limit_ms (0: none) it raises the abort flag that the kernels poll, waits for
+// the stream, reads the counters again and returns false.
+bool WatchCounters(cgbdsm_query* q, double limit_ms) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (uint32_t i = 1; !q->box.Arrived(); i++) {
+        if (i & 63u) {
+            __builtin_ia32_pause();
+            continue;
+        }
+        const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+        const bool late = limit_ms > 0 && ms > limit_ms;
+        if (ms < 0.5 && !late) continue;
+        const hipError_t e = hipStreamQuery(q->s);
+        if (e != hipSuccess && e != hipErrorNotReady) CGD_HIP(e);
+        if (e == hipSuccess) {
+            q->box.Wait(q->s);
+            break;
+        }
+        if (late) {
+            *(volatile uint32_t*)q->h_abort = 1;
+            std::atomic_thread_fence(std::memory_order_seq_cst);
+            CGD_HIP(hipStreamSynchronize(q->s));
+            *(volatile uint32_t*)q->h_abort = 0;
+            ReadCounters(q);
+            return false;
+        }
+        std::this_thread::sleep_for(std::chrono::duration<double, std::milli>(std::min(0.2, ms / 16)));
+        i |= 63u;
+    }
+    return true;
+}
+
+// What `spent` ms leave of q's deadline (0: none), for WatchCounters.
+double DeadlineLeft(const cgbdsm_query* q, double spent) {
+    return q->deadline_ms > 0 ? std::max(q->deadline_ms - spent, 1e-3) : 0.0;
+}
+
 // Final DFS over the rows of the jobs in q->h_jobs (job j owns rows
 // [h_rowbase[j], h_rowbase[j+1])), on q's stream with q's work queue; waits
 // for it while honouring q's deadline: past the deadline the host raises the
@@ -517,45 +557,23 @@ void RunDfsJobs(cgbdsm_query* q, uint32_t* tuples, uint64_t tup_cap) {
               q->st.last_dfs_lds_cache, batched, q->s);
     KEnd(q, k);
     CGD_HIP(hipGetLastError());
-    // The counters come back with the launch.  The host watches for them
-    // without sleeping at first (a batch's launch is often over in 0.1 ms),
-    // then for a sixteenth of the time waited so far, 200 us at most.
+    // The counters come back with the launch.
     q->box.Request(q->d_cnt, sizeof(Counters), q->s);
-    const auto t0 = std::chrono::steady_clock::now();
-    for (uint32_t i = 1; !q->box.Arrived(); i++) {
-        if (i & 63u) {
-            __builtin_ia32_pause();
-            continue;
-        }
-        const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-        if (ms < 0.5) continue;
-        const hipError_t e = hipStreamQuery(q->s);
-        if (e != hipSuccess && e != hipErrorNotReady) CGD_HIP(e);
-        if (e == hipSuccess && !q->box.Arrived()) q->box.Wait(q->s);
-        if (q->deadline_ms > 0 && ms > q->deadline_ms) {
-            *(volatile uint32_t*)q->h_abort = 1;
-            std::atomic_thread_fence(std::memory_order_seq_cst);
-            CGD_HIP(hipStreamSynchronize(q->s));
-            *(volatile uint32_t*)q->h_abort = 0;
-            ReadCounters(q);
-            unsigned long long part = 0;
-            for (uint32_t e = 0; e < q->qe; e++) part += q->h_cnt->per_edge[e];
-            Throw(CGBDSM_ERR_OVERFLOW, "final DFS exceeded the deadline of " + std::to_string(q->deadline_ms) +
-                                           " ms; count incomplete (partial " + std::to_string(part) +
-                                           " matches, " + std::to_string(q->h_cnt->scanned) + " candidates, " +
-                                           std::to_string(q->h_cnt->probes) + " probes, " + std::to_string(n) +
-                                           " rows at depth " + std::to_string(depth) + ", " +
-                                           std::to_string(q->h_cnt->q_rows.v) + " rows taken, " +
-                                           std::to_string(q->h_cnt->donated) + " donated; pending " +
-                                           std::to_string(q->h_cnt->q_pending.v) + ", idle " +
-                                           std::to_string(q->h_cnt->q_idle.v) + ", queue " +
-                                           std::to_string(q->h_cnt->q_head.v) + "/" +
-                                           std::to_string(q->h_cnt->q_tail.v) + ", flags " +
-                                           std::to_string(q->h_cnt->flags) + ")");
-        }
-        std::this_thread::sleep_for(std::chrono::duration<double, std::milli>(std::min(0.2, ms / 16)));
-        i |= 63u;
-    }
+    if (WatchCounters(q, DeadlineLeft(q, q->spent_ms))) return;
+    unsigned long long part = 0;
+    for (uint32_t e = 0; e < q->qe; e++) part += q->h_cnt->per_edge[e];
+    Throw(CGBDSM_ERR_OVERFLOW, "final DFS exceeded the deadline of " + std::to_string(q->deadline_ms) +
+                                   " ms; count incomplete (partial " + std::to_string(part) + " matches, " +
+                                   std::to_string(q->h_cnt->scanned) + " candidates, " +
+                                   std::to_string(q->h_cnt->probes) + " probes, " + std::to_string(n) +
+                                   " rows at depth " + std::to_string(depth) + ", " +
+                                   std::to_string(q->h_cnt->q_rows.v) + " rows taken, " +
+                                   std::to_string(q->h_cnt->donated) + " donated; pending " +
+                                   std::to_string(q->h_cnt->q_pending.v) + ", idle " +
+                                   std::to_string(q->h_cnt->q_idle.v) + ", queue " +
+                                   std::to_string(q->h_cnt->q_head.v) + "/" +
+                                   std::to_string(q->h_cnt->q_tail.v) + ", flags " +
+                                   std::to_string(q->h_cnt->flags) + ")");
 }
 
 // q's share of a final-DFS launch; its frontier has been built, so h_cnt
@@ -740,6 +758,7 @@ void PmaDelete(cgbdsm_query* q, const uint64_t* keys, uint64_t n) {
 
 void IndexInitDevice(cgbdsm_query* q, uint64_t n, uint32_t dv_count, uint32_t* card, float* avg) {
     SplitInvalidate(q);
+    memset(q->wide_from, 0, sizeof(q->wide_from));
     GrowDV(q, std::max<uint32_t>(dv_count, 1));
     q->dv = dv_count;
     q->W = (q->dv + 63) / 64;
@@ -1050,6 +1069,7 @@ cgbdsm_status cgbdsm_query_set_plan(cgbdsm_query* q, const cgbdsm_plan* plan) {
             q->hplan.dep_mask[x] = m;
         }
         q->hplan.lds = MakePlanLds(q->hplan);
+        memset(q->wide_from, 0, sizeof(q->wide_from));
         UploadPlan(q);
         q->have_order = true;
     });
@@ -1461,11 +1481,20 @@ static const Frontier& BuildFrontier(cgbdsm_query* q) {
     // than the level written out (dense 6-vertex query on scale 20: 49 ms of
     // DFS from depth 2; dense 5-vertex 25 ms; a 6-vertex cycle on scale 17 24
     // ms).  So with the default limit or a larger one the levels go on to it
-    // while a level fits kExtendWords.
+    // while a level fits kExtendWords.  They are part of the work that the
+    // deadline bounds.
     const bool to_suffix = batched_suffix && !fixed_cap && q->bfs_row_limit >= kBfsRowLimit;
+    double spent = 0;
     while (n > 0 && depth + 1 < q->qv && !(batched_suffix && depth + 2 > q->hplan.cp_start)) {
         const bool wide = n >= q->bfs_row_limit;
-        if (wide && !(to_suffix && n * (depth + 1) <= kExtendWords)) break;
+        if (wide) {
+            if (!to_suffix || n * (depth + 1) > kExtendWords) break;
+            uint64_t& from = q->wide_from[depth];
+            if (from && n >= from) {
+                from += from / 32 + 1;  // tried again after some 20 batches of the size that failed
+                break;
+            }
+        }
         uint64_t want_rows = fixed_cap ? q->frontier_cap_rows
                              : wide    ? std::min<uint64_t>(n * 4, kExtendWords / (depth + 1))
                                        : std::min<uint64_t>(std::max<uint64_t>(n * 64, 1u << 20), 1ull << 28);
@@ -1478,12 +1507,24 @@ static const Frontier& BuildFrontier(cgbdsm_query* q) {
             for (int attempt = 0;; attempt++) {
                 Ensure(q, q->front[cur ^ 1], want_rows * (depth + 1));
                 SetCounters(q, {{&Counters::rows_out, 0}, {&Counters::flags, 0}}, q->s);
+                const uint64_t cap_rows = q->front[cur ^ 1].cap / (depth + 1);
+                // (a wide level's rows are counted on past the buffer, up to
+                // the largest size that the second attempt may take)
+                const LevelStop stop{wide ? std::max<uint64_t>(cap_rows, kExtendWords / (depth + 1)) : cap_rows,
+                                     q->d_abort, (long long)q->ctx->wall_khz / 2};
+                const auto t0 = std::chrono::steady_clock::now();
                 const int ke = KBegin(q, CGBDSM_K_EXTEND);
                 LaunchExtend(T, q->front[cur].p, n, depth, q->h_cnt->u_dups == 0, q->ext_offs.p, q->ext_sel.p,
-                             q->scan_scratch.p, q->front[cur ^ 1].p, q->front[cur ^ 1].cap / (depth + 1), q->d_cnt,
-                             q->s);
+                             q->scan_scratch.p, q->front[cur ^ 1].p, cap_rows, stop, q->d_cnt, q->s);
                 KEnd(q, ke);
-                ReadCounters(q);
+                if (wide) {
+                    q->box.Request(q->d_cnt, sizeof(Counters), q->s);
+                    const bool in_time = WatchCounters(q, DeadlineLeft(q, spent));
+                    spent += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+                    if (!in_time) break;
+                } else {
+                    ReadCounters(q);
+                }
                 KAdd(q, CGBDSM_K_EXTEND, 0, n);
                 if (!(q->h_cnt->flags & kFlagFrontier)) {
                     done = true;
@@ -1498,6 +1539,7 @@ static const Frontier& BuildFrontier(cgbdsm_query* q) {
         }
         if (!done) {  // keep this level, count it by DFS
             if (wide) {
+                q->wide_from[depth] = std::max<uint64_t>(n / 2, 1);
                 CGD_HIP(hipStreamSynchronize(q->s));  // (without memory: the grouping may still read the seeds)
                 Release(q, q->ext_offs);
                 Release(q, q->ext_sel);
@@ -1511,7 +1553,7 @@ static const Frontier& BuildFrontier(cgbdsm_query* q) {
         depth++;
     }
     CGD_HIP(hipEventRecord(q->fr_ev, q->s));
-    q->fr = Frontier{n, depth, cur};
+    q->fr = Frontier{n, depth, cur, spent};
     q->fr_ready = true;
     return q->fr;
 }
@@ -1592,6 +1634,8 @@ cgbdsm_status cgbdsm_matching(cgbdsm_query* q, unsigned long long* num_matches, 
     return Guard([&] {
         if (!q || (q->phase != 4 && q->phase != 5)) Throw(CGBDSM_ERR_INVALID, "matching must follow build_local_index");
         const Frontier f = BuildFrontier(q);
+        q->spent_ms = f.ms;
+        q->fr.ms = 0;
         // Step 5: final DFS count from the current level.
         ResetMatchCounters(q, q->s);
         ResetDfsCounters(q);
@@ -1633,11 +1677,19 @@ cgbdsm_status cgbdsm_matching_batch(cgbdsm_query* const* qs, int nq, unsigned lo
         // Seeds and BFS levels, one query after another, for queries whose
         // frontier cgbdsm_build_frontier has not built already.
         std::vector<Frontier> fr(nq);
-        for (int i = 0; i < nq; i++) fr[i] = BuildFrontier(qs[i]);
+        double before = 0, now = 0;  // of the deadline: frontiers built side by side before, and here
+        for (int i = 0; i < nq; i++) {
+            const bool had = qs[i]->fr_ready;
+            fr[i] = BuildFrontier(qs[i]);
+            if (had) before = std::max(before, fr[i].ms);
+            else now += fr[i].ms;
+            qs[i]->fr.ms = 0;
+        }
         // One final-DFS launch for all of them, on the first query's stream
         // and work queue, after every other query's frontier is complete on
         // its own stream (the tag grouping may still be running there).
         cgbdsm_query* lead = qs[0];
+        lead->spent_ms = before + now;
         for (int i = 1; i < nq; i++) CGD_HIP(hipStreamWaitEvent(lead->s, qs[i]->fr_ev, 0));
         lead->h_jobs.clear();
         lead->h_rowbase.assign(1, 0ull);
@@ -1674,6 +1726,7 @@ cgbdsm_status cgbdsm_match_tuples(cgbdsm_query* q, uint32_t* out, uint64_t cap, 
             SetCounter(q, &Counters::tuples, 0);
             SetCounter(q, &Counters::flags, 0);
             FillU64((uint64_t*)&q->d_cnt->per_edge[0], 0, kMaxQE, q->s);
+            q->spent_ms = 0;
             RunDfs(q, q->front[q->last_buf].p, q->last_rows, q->last_depth, d_out, cap);
             ReadCounters(q);
             if (q->h_cnt->flags & kFlagTuples) Throw(CGBDSM_ERR_OVERFLOW, "tuple capacity exceeded");

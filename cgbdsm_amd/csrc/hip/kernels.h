@@ -86,10 +86,19 @@ void LaunchGroupByTag(const uint32_t* in, uint64_t n, uint32_t words, uint32_t t
                       uint32_t* out, hipStream_t s);
 // Depth-1 rows [(ei << tag_shift) | v0] (one word each).
 void LaunchSeed1(const Tables& T, const EiList& L, uint32_t* rows, uint64_t cap_rows, Counters* cnt, hipStream_t s);
+// When a BFS level ends early: more rows found than `rows` (at least its
+// capacity, so that kFlagFrontier is set and the level dropped), or the host
+// flag `abort` raised (kFlagAborted); blocks look once per `ticks`.
+struct LevelStop {
+    uint64_t rows;
+    const uint32_t* abort;
+    long long ticks;
+};
 // One BFS level: rows of `depth` words in, depth + 1 words out.  sets: no list
 // holds a value twice.  Scratch: offs n_in + 1 words, sel n_in bytes, the scan's.
 void LaunchExtend(const Tables& T, const uint32_t* in, uint64_t n_in, uint32_t depth, bool sets, uint64_t* offs,
-                  uint8_t* sel, void* scan_scratch, uint32_t* out, uint64_t cap_rows, Counters* cnt, hipStream_t s);
+                  uint8_t* sel, void* scan_scratch, uint32_t* out, uint64_t cap_rows, const LevelStop& stop,
+                  Counters* cnt, hipStream_t s);
 // One query's share of a final-DFS launch: its index tables, its frontier
 // rows (depth D, word 0 = ei tag | v0), its counters (per-edge counts,
 // duplicate flag of its update lists) and its counting options.

@@ -162,14 +162,15 @@ __device__ __forceinline__ uint32_t At(const List& L, uint32_t i) { return i < L
 // Frontier rows a wavefront has found, kept in its LDS until kRowBuf words are
 // full: one atomic on the row counter and one contiguous store per flush.  (An
 // atomic for every 64 candidates, on one line, took most of the kernels' time.)
+// Flush returns the rows that all waves had found up to and with this one's.
 constexpr uint32_t kRowBuf = 1024;
 struct RowBuf {
     uint32_t* buf;
     uint32_t words, n;  // words per row, rows held
     __device__ __forceinline__ uint32_t Room() const { return kRowBuf / words - n; }
-    __device__ __forceinline__ void Flush(uint32_t* __restrict__ rows, uint64_t cap_rows,
-                                          Counters* __restrict__ cnt) {
-        if (!n) return;
+    __device__ __forceinline__ uint64_t Flush(uint32_t* __restrict__ rows, uint64_t cap_rows,
+                                              Counters* __restrict__ cnt) {
+        if (!n) return 0;
         const uint32_t lane = LaneId();
         WaveSync();
         unsigned long long base = 0;
@@ -181,7 +182,9 @@ struct RowBuf {
             for (uint32_t i = lane; i < n * words; i += kWave) rows[base * words + i] = buf[i];
         }
         WaveSync();
+        const uint64_t found = base + n;
         n = 0;
+        return found;
     }
 };
 
@@ -448,8 +451,8 @@ constexpr uint32_t kFull = 0xFFFFFFFFu;
 constexpr uint32_t kNoSel = 0xFFu;
 constexpr uint32_t kNoSkip = 0xFFu;
 
-__device__ __forceinline__ bool AbortRequested(const StealQueue& Q) {
-    return __hip_atomic_load(Q.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0u;
+__device__ __forceinline__ bool AbortRequested(const uint32_t* abort) {
+    return __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0u;
 }
 
 __device__ __forceinline__ unsigned long long LoadAgent(const unsigned long long* p) {
@@ -612,13 +615,21 @@ __global__ void __launch_bounds__(kThreads) KExtendLens(Tables T, const uint32_t
 // idle (lists of a few entries), the hubs' rows to one wave each, and took an
 // atomic per 64 candidates: dense 6-vertex query on scale 20, 376k rows to
 // 2.2M: 7.2 -> 0.43 ms.
+//
+// A level ends early once it is of no use: a wave stops when the rows found
+// pass stop.rows (seen at its flush), a block once per stop.ticks when they do
+// or when the host asks for it (long scans with few survivors hardly flush).
+constexpr uint32_t kHostLooks = 32;
 __global__ void __launch_bounds__(kThreads) KExtend(Tables T, const uint32_t* __restrict__ in, uint64_t n, uint32_t D,
                                                     const uint64_t* __restrict__ offs, const uint8_t* __restrict__ sel,
-                                                    uint32_t* __restrict__ out, uint64_t cap_rows,
+                                                    uint32_t* __restrict__ out, uint64_t cap_rows, LevelStop stop,
                                                     Counters* __restrict__ cnt) {
     __shared__ PlanLds s_plan;
     __shared__ uint32_t s_buf[kWpb][kRowBuf];
-    FillPlanLds(T, &s_plan);
+    __shared__ Hint s_hint;
+    if (threadIdx.x == 0) s_hint = Hint{0, (long long)wall_clock64(), 0, 0};
+    FillPlanLds(T, &s_plan);  // (ends with a block barrier)
+    volatile LdsHint* hint = (volatile LdsHint*)&s_hint;
     LdsPlan* L = (LdsPlan*)&s_plan;
     const uint32_t wv = threadIdx.x / kWave;
     const uint32_t tag_shift = T.P->tag_shift, v_mask = T.P->v_mask;
@@ -628,8 +639,30 @@ __global__ void __launch_bounds__(kThreads) KExtend(Tables T, const uint32_t* __
     const uint64_t per = ((total + nw - 1) / nw + kWave - 1) & ~(uint64_t)(kWave - 1);
     const uint64_t lo = ((uint64_t)blockIdx.x * kWpb + wv) * per, hi = lo + per < total ? lo + per : total;
     uint64_t p0 = lo < hi ? LbFirst(offs, n, lo) : 0;
-    uint32_t probes = 0;
+    uint32_t probes = 0, iter = 0;
     for (uint64_t it0 = lo; it0 < hi; it0 += kWave) {
+        if ((++iter & 63u) == 0) {
+            const long long now = (long long)Uniform64((unsigned long long)wall_clock64());
+            if (now - (long long)Uniform64((unsigned long long)hint->t_host) >= stop.ticks) {
+                if (LaneId() == 0) {
+                    hint->t_host = now;
+                    // Every block looks at the device's words, one in
+                    // kHostLooks (another one each time) at the host's, across
+                    // the bus (a 5 ms level that was to end at its first look:
+                    // 2.3 ms on after that with 2 048 blocks reading it, 0.8 ms so).
+                    bool end = (LoadAgent(&cnt->flags) & kFlagAborted) || LoadAgent(&cnt->rows_out) > stop.rows;
+                    const uint32_t looks = hint->idle;
+                    hint->idle = looks + 1;
+                    if (!end && (blockIdx.x + looks) % kHostLooks == 0 && AbortRequested(stop.abort)) {
+                        atomicOr(&cnt->flags, kFlagAborted);
+                        end = true;
+                    }
+                    if (end) hint->stop = 1;
+                }
+                WaveSync();
+            }
+            if (Uniform(hint->stop)) break;
+        }
         const LbItem it = LbLocateFrom(offs, n, p0, it0, hi);
         if (it0 + kWave <= hi) p0 = ReadLane64(it.p, kWave - 1);
         const uint32_t* row = in + it.p * D;
@@ -654,7 +687,7 @@ __global__ void __launch_bounds__(kThreads) KExtend(Tables T, const uint32_t* __
         const uint64_t m = __ballot(ok);
         const uint32_t k = (uint32_t)__popcll(m);
         if (!k) continue;
-        if (buf.Room() < k) buf.Flush(out, cap_rows, cnt);
+        if (buf.Room() < k && buf.Flush(out, cap_rows, cnt) > stop.rows) break;
         if (ok) {
             uint32_t* o = buf.buf + (buf.n + RankBelow(m)) * (D + 1);
             for (uint32_t i = 0; i < D; i++) o[i] = row[i];
@@ -1513,7 +1546,7 @@ __global__ void __launch_bounds__(kThreads)
                 unsigned long long fl = LoadAgent(&cnt->flags);
                 if (now - hint->t_host >= Q.host_ticks) {
                     hint->t_host = now;
-                    if (AbortRequested(Q)) {
+                    if (AbortRequested(Q.abort)) {
                         atomicOr(&cnt->flags, kFlagAborted);
                         fl |= kFlagAborted;
                     }
@@ -2031,11 +2064,12 @@ void LaunchSeed1(const Tables& T, const EiList& L, uint32_t* rows, uint64_t cap_
 }
 
 void LaunchExtend(const Tables& T, const uint32_t* in, uint64_t n_in, uint32_t depth, bool sets, uint64_t* offs,
-                  uint8_t* sel, void* scan_scratch, uint32_t* out, uint64_t cap_rows, Counters* cnt, hipStream_t s) {
+                  uint8_t* sel, void* scan_scratch, uint32_t* out, uint64_t cap_rows, const LevelStop& stop,
+                  Counters* cnt, hipStream_t s) {
     if (!n_in) return;
     KExtendLens<<<Grid1(n_in, kThreads, 2048), kThreads, 0, s>>>(T, in, n_in, depth, sets, offs, sel);
     ScanU64(offs, offs, n_in, offs + n_in, scan_scratch, s);
-    KExtend<<<Grid1(n_in, kWpb, 2048), kThreads, 0, s>>>(T, in, n_in, depth, offs, sel, out, cap_rows, cnt);
+    KExtend<<<Grid1(n_in, kWpb, 2048), kThreads, 0, s>>>(T, in, n_in, depth, offs, sel, out, cap_rows, stop, cnt);
 }
 
 // LDS per final-DFS block (static tables + survivor stacks + cache) at nb

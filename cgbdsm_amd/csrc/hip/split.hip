@@ -305,7 +305,7 @@ struct HostDfs {
     // Stop asked, or the deadline passed (then asks every worker to stop).
     bool Stopped(SplitState* St) const {
         if (St->stop.load(std::memory_order_relaxed)) return true;
-        if (q->deadline_ms > 0 && MsSince(St->t0) > q->deadline_ms) {
+        if (q->deadline_ms > 0 && MsSince(St->t0) + q->spent_ms > q->deadline_ms) {
             uint32_t z = 0;
             St->stop.compare_exchange_strong(z, 2);
             return true;

@@ -225,7 +225,8 @@ cgbdsm_status cgbdsm_build_frontier(cgbdsm_query* q);
  * (optional array, entries optional) receives its per-edge counts.  Counts
  * are identical to nq separate cgbdsm_matching calls.  Every query must be
  * in the state cgbdsm_matching expects; the deadline and the statistics of
- * the launch are the first query's (last_dfs_* are stored in each query).
+ * the launch are the first query's (last_dfs_* are stored in each query); each
+ * query's own deadline bounds its BFS levels.
  * No reference counterpart: the reference runs one query per process
  * (main_calig.cpp:29-35).  nq <= CGBDSM_MAX_BATCH_QUERIES. */
 cgbdsm_status cgbdsm_matching_batch(cgbdsm_query* const* qs, int nq, unsigned long long* num_matches,
@@ -288,8 +289,9 @@ cgbdsm_status cgbdsm_set_dfs_search(cgbdsm_query* q, int wave_search);
  * applies. */
 cgbdsm_status cgbdsm_set_dfs_steal(cgbdsm_query* q, uint32_t range_min, uint32_t cache_cap);
 
-/* Cooperative deadline for the final DFS of cgbdsm_matching (default 120 s,
- * 0 = none).
+/* Cooperative deadline for the final DFS of cgbdsm_matching and the BFS levels
+ * above the row limit that its frontier takes (default 120 s, 0 = none).  A
+ * level that runs past it is given up, and the DFS has what is left.
  * Past the deadline the host raises a flag the kernel polls; the call then
  * returns CGBDSM_ERR_OVERFLOW because the count is incomplete.  No reference
  * counterpart (the reference waits unboundedly, graph/graph_gpu.cu:1457-1464). */

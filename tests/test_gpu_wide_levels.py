@@ -1,6 +1,7 @@
 """BFS levels above the row limit (queries whose product suffix is counted in
 batches): a level that fits at once, one written again at its size, one that
-does not fit and one without memory.
+does not fit and is then not tried on the next batch, one without memory and
+one past the deadline.
 
 The graph has one layer of vertices per query vertex, so that the count is a
 product of layer degrees: triangle 0-1-2 with a tail 2-3-4.  The new edges are
@@ -10,7 +11,7 @@ import numpy as np
 import pytest
 
 from cgbdsm_amd import _native as N
-from cgbdsm_amd.engine import Engine
+from cgbdsm_amd.engine import CgbdsmError, Engine
 from cgbdsm_amd.host import KeyBatch, Planner
 
 pytestmark = pytest.mark.gpu
@@ -88,11 +89,11 @@ def test_wide_level(fan, want):
     cnt, per = q.matching()
     assert cnt == g.count and per[1] == g.count
     assert levels(q) == want
-    # The same batch again: the buffer has its size now.
+    # The same batch again: the buffer has its size now, a level that did not fit is not tried.
     q.batch_update_global_index()
     g.prepare(q, again=True)
     assert q.matching()[0] == g.count
-    assert levels(q) == (1,) + want[1:]
+    assert levels(q) == ((1 if want[1] == 3 else 0),) + want[1:]
     q.close()
     eng.close()
 
@@ -115,3 +116,36 @@ def test_wide_level_without_memory():
         need = eng.memory()[0]
         q.close()
         eng.close()
+
+
+def test_wide_level_past_the_deadline():
+    """90 000 rows of 8 001 candidates each, one of them a common neighbour:
+    several milliseconds, of which the kernel runs about two before it sees
+    that the host asks it to stop."""
+    print("case wide level deadline", flush=True)
+    eng, g = Engine(0), Layers(1, apart=8000)
+    q = g.query(eng)
+    g.prepare(q)
+    q.set_deadline(0.001)
+    with pytest.raises(CgbdsmError) as ex:
+        q.matching()
+    assert ex.value.code == 5, ex.value  # CGBDSM_ERR_OVERFLOW
+    asked = q.kernel_times()["extend"]["ms"]
+    q.set_deadline(0)
+    assert q.matching()[0] == g.count
+    assert levels(q) == (1, 2, ROWS)  # the level was given up, the DFS counts from the seeds
+    # Without a deadline a batch of the same size does not try it either; a new plan does.
+    q.batch_update_global_index()
+    g.prepare(q, again=True)
+    assert q.matching()[0] == g.count
+    assert levels(q) == (0, 2, ROWS)
+    q.batch_update_global_index()
+    q.set_plan(q.tables)
+    g.prepare(q, again=True)
+    assert q.matching()[0] == g.count
+    whole = q.kernel_times()["extend"]["ms"]
+    print(f"extend {asked} ms of {whole}", flush=True)
+    assert levels(q) == (1, 3, ROWS)
+    assert asked < whole
+    q.close()
+    eng.close()

@@ -1174,8 +1174,10 @@ __device__ __forceinline__ SfxLevel SuffixLevel(const Ctx& X, const Tables& T, u
 //
 // A step over hub lists can hold a million entries, milliseconds of one
 // wavefront's time that nobody can take over: it then ends at the sibling lane
-// `used` where kStepEntries entries are reached (kWave if all were counted),
-// and the caller goes on from there, where it can also hand out the rest.
+// `used` whose entries pass kStepEntries (kWave if all were counted), and the
+// caller goes on from there, where it can also hand out the rest.  The bound is
+// per position: kStepEntries, or the entries of the first sibling that has any
+// (they are never cut), whichever is more.
 // The 250 000-edge batch's dense 4-vertex query spent 46 % of its wavefront
 // time waiting for such steps (38.2 ms; 22.9 ms with them cut here, 27 ms at 16384).
 constexpr uint32_t kStepEntries = 2048;
